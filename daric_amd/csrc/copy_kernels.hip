@@ -8,14 +8,11 @@
 // stores are nontemporal: every byte is touched once.
 //
 // Block order (measured on MI355X at the Llama-3-8B shape): both directions
-// cut each tile into parts of ~8 KiB. The scatter direction runs job-minor --
-// consecutive workgroups take the same part of consecutive jobs -- which
-// sustained ~6.3 TB/s against ~6.0 TB/s for a tile-major order (256 jobs of
-// 64 pages) and 5.9 against 5.3-5.4 TB/s (32 jobs of 4096 pages); the gather
-// direction runs tile-major within a job, which sustained ~6.3 TB/s (256 x 64)
-// and 5.8-6.0 TB/s (32 x 4096), against 5.5-5.6 TB/s for whole-tile
-// workgroups and job-minor orders. The fused scatter + rotation runs job-minor
-// on whole tiles.
+// cut each tile into parts of ~8 KiB. The scatter direction and the fused
+// scatter + rotation deal runs of 128 KiB of each job to the XCDs (JobRuns);
+// the gather direction runs tile-major within a job, which sustained ~6.3 TB/s
+// (256 jobs of 64 pages) and 5.8-6.0 TB/s (32 of 4096), against 5.5-5.6 TB/s
+// for whole-tile workgroups and job-minor orders.
 //
 // Pages whose block id is 0 (vLLM's null block) are skipped, as the
 // reference's kernels skip them (csrc/cache_ops/kernels.cu:26,39,69,79,104,117);
@@ -89,28 +86,18 @@ __device__ __forceinline__ bool resolve_tile(const CopyJob& j, int t, int& p, in
     return true;
 }
 
-// Block -> (job, unit) mapping. Job-minor: block b takes job b % n_jobs and
-// unit b / n_jobs; tile-major: job blockIdx.y, unit blockIdx.x. A unit is part
-// (unit & (parts - 1)) of tile (unit >> log2 parts).
-template <bool JOB_MINOR>
-__device__ __forceinline__ void block_unit(const FastDiv& njobs, int& job, int& unit) {
-    if (JOB_MINOR) {
-        const uint32_t b = blockIdx.x;
-        const uint32_t q = njobs.div(b);
-        job = static_cast<int>(b - q * njobs.d);
-        unit = static_cast<int>(q);
-    } else {
-        job = static_cast<int>(blockIdx.y);
-        unit = static_cast<int>(blockIdx.x);
-    }
-}
-
-template <int VW, bool GATHER, bool JOB_MINOR>
-__global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job0, FastDiv njobs,
+// A unit is part (unit & (parts - 1)) of tile (unit >> log2 parts). Gather:
+// grid.y = job, grid.x = unit in the order of `xr`; scatter: the order of `jr`.
+template <int VW, bool GATHER>
+__global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job0, JobRuns jr,
                                                               int log2_parts, XcdRuns xr) {
     int jb, unit;
-    block_unit<JOB_MINOR>(njobs, jb, unit);
-    if (!JOB_MINOR) unit = xr.map(unit);
+    if (GATHER) {
+        jb = static_cast<int>(blockIdx.y);
+        unit = xr.map(static_cast<int>(blockIdx.x));
+    } else {
+        jr.at_block(blockIdx.x, jb, unit);
+    }
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
     int p, s;
     uint8_t *cache, *stage;
@@ -128,7 +115,7 @@ __global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job
         copy_units<VW>(stage + b0, cache + b0, cnt);
 }
 
-// Fused scatter + rotation, job-minor block order. A work item of a K row is
+// Fused scatter + rotation, blocks in the order of JobRuns. A work item of a K row is
 // either a rotated item (NeoX: the two 16-byte units holding pairs
 // (i, i + R/2) for i in [k*VE, k*VE + VE); GPT-J: one unit holding VE/2
 // adjacent pairs) or a pass-through unit of the row's unrotated tail. Rows
@@ -139,14 +126,14 @@ __global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job
 // cancels in a linear rotation.
 template <int KIND, bool NEOX>
 __global__ __launch_bounds__(kThreads) void scatter_rotate_kernel(
-    DescArg d, int job0, FastDiv njobs, RowGeomDiv gd, const float* __restrict__ inv_freq) {
+    DescArg d, int job0, JobRuns jr, RowGeomDiv gd, const float* __restrict__ inv_freq) {
     using E = Elem<KIND>;
     constexpr int VE = E::VE;
     __shared__ float s_cos[kMaxHalfRot];
     __shared__ float s_sin[kMaxHalfRot];
 
     int jb, unit;
-    block_unit<true>(njobs, jb, unit);
+    jr.at_block(blockIdx.x, jb, unit);
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
     int p, s;
     uint8_t *cache, *stage;
@@ -265,7 +252,7 @@ constexpr int kRotLaneUnroll = 4;
 
 template <int KIND, bool NEOX>
 __global__ __launch_bounds__(kThreads) void scatter_rotate_lane_kernel(
-    DescArg d, int job0, FastDiv njobs, RowGeomDiv gd, const float* __restrict__ inv_freq, int log2_parts) {
+    DescArg d, int job0, JobRuns jr, RowGeomDiv gd, const float* __restrict__ inv_freq, int log2_parts) {
     using E = Elem<KIND>;
     constexpr int VE = E::VE;
     constexpr int EPW = E::EPW;
@@ -283,7 +270,7 @@ __global__ __launch_bounds__(kThreads) void scatter_rotate_lane_kernel(
     __shared__ float4 s_cs[kMaxHalfRot / 2];   // CSL: (cos, sin) of pairs 2i and 2i+1
 
     int jb, unit;
-    block_unit<true>(njobs, jb, unit);
+    jr.at_block(blockIdx.x, jb, unit);
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
     int p, s;
     uint8_t *cache, *stage;
@@ -440,8 +427,6 @@ __global__ __launch_bounds__(kThreads) void upload_kernel(const u32x4* __restric
     if (i < n16) dst[i] = src[i];
 }
 
-// Largest grid.x: grid.x * 256 lanes must stay below 2^32.
-constexpr int64_t kMaxBlocksX = (1ll << 24) - 1;
 constexpr int kMaxY = 65535;
 
 void launch_copy_pages(const DescArg& d, int n_jobs, int max_tiles, int64_t max_span, int vw,
@@ -449,33 +434,26 @@ void launch_copy_pages(const DescArg& d, int n_jobs, int max_tiles, int64_t max_
     // tiles cut into parts of about 8 KiB
     int log2_parts = 0;
     while (log2_parts < 3 && (max_span >> (log2_parts + 1)) >= 8192 &&
-           (static_cast<int64_t>(max_tiles) << (log2_parts + 1)) <= kMaxBlocksX)
+           (static_cast<int64_t>(max_tiles) << (log2_parts + 1)) <= kMaxGridBlocks)
         ++log2_parts;
+    const int64_t units = static_cast<int64_t>(max_tiles) << log2_parts;
     if (!gather) {
-        // job-minor: slices of jobs so that the grid fits grid.x
-        const int64_t units = static_cast<int64_t>(max_tiles) << log2_parts;
-        const int slice = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(n_jobs, kMaxBlocksX / units)));
-        for (int j0 = 0; j0 < n_jobs; j0 += slice) {
-            const int nj = std::min(slice, n_jobs - j0);
-            const FastDiv fd(static_cast<uint32_t>(nj));
-            const dim3 grid(static_cast<unsigned>(units * nj));
-            if (vw == 16) DARIC_LAUNCH((copy_pages_kernel<16, false, true>), grid, kThreads, 0, stream, d, j0, fd, log2_parts, XcdRuns());
-            else if (vw == 4) DARIC_LAUNCH((copy_pages_kernel<4, false, true>), grid, kThreads, 0, stream, d, j0, fd, log2_parts, XcdRuns());
-            else DARIC_LAUNCH((copy_pages_kernel<1, false, true>), grid, kThreads, 0, stream, d, j0, fd, log2_parts, XcdRuns());
+        for_job_runs(n_jobs, units, max_span >> log2_parts, [&](int j0, const JobRuns& jr, unsigned blocks) {
+            if (vw == 16) DARIC_LAUNCH((copy_pages_kernel<16, false>), blocks, kThreads, 0, stream, d, j0, jr, log2_parts, XcdRuns());
+            else if (vw == 4) DARIC_LAUNCH((copy_pages_kernel<4, false>), blocks, kThreads, 0, stream, d, j0, jr, log2_parts, XcdRuns());
+            else DARIC_LAUNCH((copy_pages_kernel<1, false>), blocks, kThreads, 0, stream, d, j0, jr, log2_parts, XcdRuns());
             check_launch("scatter_pages");
-        }
+        });
         return;
     }
     // gather: tile-major within a job
-    const FastDiv fd(1);
-    const int64_t gx = static_cast<int64_t>(max_tiles) << log2_parts;
-    const XcdRuns xr(gx, max_span >> log2_parts);
+    const XcdRuns xr(units, max_span >> log2_parts);
     for (int j0 = 0; j0 < n_jobs; j0 += kMaxY) {
         const int nj = std::min(kMaxY, n_jobs - j0);
-        const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(nj));
-        if (vw == 16) DARIC_LAUNCH((copy_pages_kernel<16, true, false>), grid, kThreads, 0, stream, d, j0, fd, log2_parts, xr);
-        else if (vw == 4) DARIC_LAUNCH((copy_pages_kernel<4, true, false>), grid, kThreads, 0, stream, d, j0, fd, log2_parts, xr);
-        else DARIC_LAUNCH((copy_pages_kernel<1, true, false>), grid, kThreads, 0, stream, d, j0, fd, log2_parts, xr);
+        const dim3 grid(static_cast<unsigned>(units), static_cast<unsigned>(nj));
+        if (vw == 16) DARIC_LAUNCH((copy_pages_kernel<16, true>), grid, kThreads, 0, stream, d, j0, JobRuns(), log2_parts, xr);
+        else if (vw == 4) DARIC_LAUNCH((copy_pages_kernel<4, true>), grid, kThreads, 0, stream, d, j0, JobRuns(), log2_parts, xr);
+        else DARIC_LAUNCH((copy_pages_kernel<1, true>), grid, kThreads, 0, stream, d, j0, JobRuns(), log2_parts, xr);
         check_launch("gather_pages");
     }
 }
@@ -506,28 +484,24 @@ void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles,
         while ((units >> (lp + 1)) * 16 >= 16384 && units % (2ll << lp) == 0 && (units >> (lp + 1)) % upr == 0)
             ++lp;
     }
-    const int64_t units_per_job = static_cast<int64_t>(max_tiles) << lp;
-    const int slice = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(n_jobs, kMaxBlocksX / units_per_job)));
-    for (int j0 = 0; j0 < n_jobs; j0 += slice) {
-        const int nj = std::min(slice, n_jobs - j0);
-        const FastDiv fd(static_cast<uint32_t>(nj));
-        const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(max_tiles) * nj));
+    const int64_t span = static_cast<int64_t>(geom.g.n_rows) * upr * 16;
+    for_job_runs(n_jobs, static_cast<int64_t>(max_tiles) << lp, span >> lp,
+                 [&](int j0, const JobRuns& jr, unsigned blocks) {
         if (lane) {
-            const dim3 grid2(static_cast<unsigned>(units_per_job * nj));
-#define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_lane_kernel<K, N>), grid2, kThreads, 0, stream, d, j0, fd, geom, inv_freq, lp)
+#define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_lane_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, geom, inv_freq, lp)
             if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
             else if (kind == kF16) { if (neox) DARIC_SR(kF16, true); else DARIC_SR(kF16, false); }
             else { if (neox) DARIC_SR(kE4M3, true); else DARIC_SR(kE4M3, false); }
 #undef DARIC_SR
         } else {
-#define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_kernel<K, N>), grid, kThreads, 0, stream, d, j0, fd, geom, inv_freq)
+#define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, geom, inv_freq)
             if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
             else if (kind == kF16) { if (neox) DARIC_SR(kF16, true); else DARIC_SR(kF16, false); }
             else { if (neox) DARIC_SR(kE4M3, true); else DARIC_SR(kE4M3, false); }
 #undef DARIC_SR
         }
         check_launch("scatter_pages_rerotate");
-    }
+    });
 }
 
 }  // namespace daric

@@ -69,4 +69,33 @@ int64_t daric_hosttest_layer_minor(int n_layers, int64_t n_items) {
     return bad ? -1 : launches;
 }
 
+// Walks the launches for_job_runs makes for n_jobs x units and decodes every
+// block with JobRuns::at_block. Returns the number of launches when every
+// (job, unit) pair is covered exactly once, every job lies in the launch and
+// no launch exceeds kMaxGridBlocks, else -1 or -2 (an oversized launch).
+// *log2_run gets the last launch's run length.
+int64_t daric_hosttest_job_runs(int n_jobs, int64_t units, int64_t unit_bytes, int32_t* log2_run) {
+    std::vector<uint8_t> seen(static_cast<size_t>(n_jobs) * static_cast<size_t>(units), 0);
+    int64_t launches = 0;
+    bool bad = false, big = false;
+    daric::for_job_runs(n_jobs, units, unit_bytes, [&](int j0, const daric::JobRuns& jr, unsigned blocks) {
+        ++launches;
+        *log2_run = static_cast<int32_t>(jr.log2_run);
+        if (static_cast<int64_t>(blocks) > daric::kMaxGridBlocks || blocks == 0) big = true;
+        for (uint32_t b = 0; b < blocks; ++b) {
+            int job, unit;
+            jr.at_block(b, job, unit);
+            if (job < 0 || job >= static_cast<int>(jr.jobs.d) || j0 + job >= n_jobs || unit < 0) { bad = true; continue; }
+            if (unit >= units) continue;   // past the job's end: the kernels' tile check drops it
+            uint8_t& s = seen[static_cast<size_t>(j0 + job) * static_cast<size_t>(units) + static_cast<size_t>(unit)];
+            if (s) bad = true;
+            s = 1;
+        }
+    });
+    for (uint8_t s : seen)
+        if (!s) bad = true;
+    if (big) return -2;
+    return bad ? -1 : launches;
+}
+
 }

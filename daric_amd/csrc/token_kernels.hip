@@ -28,7 +28,8 @@
 //    faster, so the host picks it there); 8 KiB parts beat whole 32 KiB
 //    pages (5.9 TB/s), 16 KiB parts were no faster; part-major order within
 //    a job beat a job-minor order (5.3 TB/s);
-//  - scatter: job-minor order 6.4-6.6 TB/s against 5.5-5.9 TB/s part-major.
+//  - scatter: job-minor order 6.4-6.6 TB/s against 5.5-5.9 TB/s part-major;
+//    it now takes the jobs' 128 KiB runs per XCD of JobRuns (kernels.h).
 // The physical-span gather_pages of the same pages ran 6.2-6.4 TB/s, so the
 // transpose costs about 1%.
 //
@@ -51,8 +52,6 @@ constexpr int kThreads = 256;
 constexpr int kRowUnroll = 8;
 constexpr int kLdsUnits = 512;   // 16-byte units of LDS per workgroup (8 KiB)
 constexpr int kMaxY = 65535;
-constexpr int64_t kMaxBlocksX = (1ll << 24) - 1;
-constexpr bool kTokenJobMinor = true;    // scatter direction: job-minor block order
 
 template <typename T>
 __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_load(p); }
@@ -84,27 +83,23 @@ __device__ __forceinline__ bool resolve_part(const TokenJob& j, int q, uint8_t*&
     return true;
 }
 
-// Workgroup -> (job, part): part-major within a job (grid.y = job), or
-// job-minor (consecutive workgroups take the same part of consecutive jobs).
-template <bool JOB_MINOR>
-__device__ __forceinline__ void block_part(FastDiv njobs, int& job, int& q) {
-    if (JOB_MINOR) {
-        const uint32_t x = blockIdx.x;
-        const uint32_t p = njobs.div(x);
-        q = static_cast<int>(p);
-        job = static_cast<int>(x - p * njobs.d);
-    } else {
+// Workgroup -> (job, part). Gather: part-major within a job (grid.y = job), in
+// the order of `xr`; scatter: the order of `jr`.
+template <bool GATHER>
+__device__ __forceinline__ void block_part(const JobRuns& jr, const XcdRuns& xr, int& job, int& q) {
+    if (GATHER) {
         job = static_cast<int>(blockIdx.y);
-        q = static_cast<int>(blockIdx.x);
+        q = xr.map(static_cast<int>(blockIdx.x));
+    } else {
+        jr.at_block(blockIdx.x, job, q);
     }
 }
 
-template <int VW, bool GATHER, bool JOB_MINOR>
-__global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job0, FastDiv njobs, XcdRuns xr) {
+template <int VW, bool GATHER>
+__global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job0, JobRuns jr, XcdRuns xr) {
     using T = typename Unit<VW>::T;
     int jb, q;
-    block_part<JOB_MINOR>(njobs, jb, q);
-    if (!JOB_MINOR) q = xr.map(q);
+    block_part<GATHER>(jr, xr, jb, q);
     const TokenJob j = desc_load(desc_at<TokenJob>(d, 0) + job0 + jb);
     uint8_t *cache, *stage;
     int n_tok;
@@ -139,12 +134,11 @@ __global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job
 
 // Head-major pages: the cache side of a part is H runs of n_tok rows, each
 // run contiguous (token stride == row bytes, head stride == PS * row bytes).
-template <bool GATHER, bool JOB_MINOR>
-__global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0, FastDiv njobs, XcdRuns xr) {
+template <bool GATHER>
+__global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0, JobRuns jr, XcdRuns xr) {
     __shared__ u32x4 sm[kLdsUnits];
     int jb, q;
-    block_part<JOB_MINOR>(njobs, jb, q);
-    if (!JOB_MINOR) q = xr.map(q);
+    block_part<GATHER>(jr, xr, jb, q);
     const TokenJob j = desc_load(desc_at<TokenJob>(d, 0) + job0 + jb);
     uint8_t *cache, *stage;
     int n_tok;
@@ -218,37 +212,24 @@ __global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0
 
 void launch_token_copy(const DescArg& d, int n_jobs, int max_parts, int64_t part_bytes, int vw,
                        bool lds, bool gather, hipStream_t stream) {
-#define DARIC_TOK(JM, FD, XR)                                                                            \
+#define DARIC_TOK(G, GRID, JR, XR)                                                                     \
     do {                                                                                               \
-        if (lds) {                                                                                     \
-            if (gather) DARIC_LAUNCH((token_lds_kernel<true, JM>), grid, kThreads, 0, stream, d, j0, FD, XR);  \
-            else DARIC_LAUNCH((token_lds_kernel<false, JM>), grid, kThreads, 0, stream, d, j0, FD, XR);        \
-        } else if (vw == 16) {                                                                         \
-            if (gather) DARIC_LAUNCH((token_rows_kernel<16, true, JM>), grid, kThreads, 0, stream, d, j0, FD, XR); \
-            else DARIC_LAUNCH((token_rows_kernel<16, false, JM>), grid, kThreads, 0, stream, d, j0, FD, XR);   \
-        } else {                                                                                       \
-            if (gather) DARIC_LAUNCH((token_rows_kernel<1, true, JM>), grid, kThreads, 0, stream, d, j0, FD, XR); \
-            else DARIC_LAUNCH((token_rows_kernel<1, false, JM>), grid, kThreads, 0, stream, d, j0, FD, XR);    \
-        }                                                                                              \
-        check_launch(gather ? "gather_tokens" : "scatter_tokens");                                    \
+        if (lds) DARIC_LAUNCH((token_lds_kernel<G>), GRID, kThreads, 0, stream, d, j0, JR, XR);          \
+        else if (vw == 16) DARIC_LAUNCH((token_rows_kernel<16, G>), GRID, kThreads, 0, stream, d, j0, JR, XR); \
+        else DARIC_LAUNCH((token_rows_kernel<1, G>), GRID, kThreads, 0, stream, d, j0, JR, XR);          \
+        check_launch(G ? "gather_tokens" : "scatter_tokens");                                         \
     } while (0)
-    if (kTokenJobMinor && !gather) {
-        // job-minor: slices of jobs so that the grid fits grid.x
-        const int slice = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(n_jobs, kMaxBlocksX / max_parts)));
-        for (int j0 = 0; j0 < n_jobs; j0 += slice) {
-            const int nj = std::min(slice, n_jobs - j0);
-            const FastDiv fd(static_cast<uint32_t>(nj));
-            const dim3 grid(static_cast<unsigned>(static_cast<int64_t>(max_parts) * nj));
-            DARIC_TOK(true, fd, XcdRuns());
-        }
+    if (!gather) {
+        for_job_runs(n_jobs, max_parts, part_bytes, [&](int j0, const JobRuns& jr, unsigned blocks) {
+            DARIC_TOK(false, blocks, jr, XcdRuns());
+        });
         return;
     }
     const XcdRuns xr(max_parts, part_bytes);
     for (int j0 = 0; j0 < n_jobs; j0 += kMaxY) {
         const int nj = std::min(kMaxY, n_jobs - j0);
         const dim3 grid(static_cast<unsigned>(max_parts), static_cast<unsigned>(nj));
-        const FastDiv fd(1);
-        DARIC_TOK(false, fd, xr);
+        DARIC_TOK(true, grid, JobRuns(), xr);
     }
 #undef DARIC_TOK
 }

@@ -511,3 +511,21 @@ def test_layer_minor_grid_covers_every_pair_once(hosttest, n_layers, n_items, la
     (grid.x x 256 lanes < 2^32), and the grid is cut only when it must be."""
     assert hosttest.daric_hosttest_layer_minor(n_layers, n_items) == launches
 
+
+# (jobs, units, unit bytes, launches, log2 run): 256 and 1280 jobs of 16 KiB
+# parts, 8 KiB parts, jobs and units that divide nothing, calls too small for
+# whole runs, units past 128 KiB, and grids past 2^24 - 1 blocks.
+@pytest.mark.parametrize("n_jobs,units,unit_bytes,launches,log2_run", [
+    (256, 256, 16384, 1, 3), (1280, 256, 16384, 1, 3), (32, 2049, 8192, 1, 4), (7, 333, 8192, 1, 4),
+    (61, 97, 9216, 1, 3), (1, 1, 16384, 1, 0), (3, 5, 16384, 1, 0), (9, 100, 16384, 1, 2),
+    (2, 70, 512, 1, 0), (13, 40, 1 << 18, 1, 0), (2, (1 << 24) - 1, 16384, 2, 0), (70_001, 300, 16384, 2, 3),
+    (1, (1 << 24) - 9, 16384, 1, 0),
+])
+def test_job_runs_grid_covers_every_unit_once(hosttest, n_jobs, units, unit_bytes, launches, log2_run):
+    """The scatters' block order: every (job, unit) pair is taken by exactly
+    one block of exactly one launch, no launch passes 2^24 - 1 blocks, and
+    runs are shortened where a call has fewer than 16 per XCD."""
+    got = ctypes.c_int32(-1)
+    assert hosttest.daric_hosttest_job_runs(n_jobs, ctypes.c_int64(units), ctypes.c_int64(unit_bytes),
+                                            ctypes.byref(got)) == launches
+    assert got.value == log2_run
