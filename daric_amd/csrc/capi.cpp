@@ -525,7 +525,6 @@ bool row_geometry(const daric_tensor& t, bool page_first, const RopeLayout& L, i
     if (n_rows * W * e != span_bytes) { *why = "page span is not the K/V head rows"; return false; }
     if ((W * e) % 16 != 0) { *why = "row bytes are not a multiple of 16"; return false; }
     const int64_t rot_units_elems = neox ? rotary_dim / 2 : rotary_dim;
-    if (rot_units_elems % VE != 0) { *why = "rotary pairs are not 16-byte aligned"; return false; }
     RowGeom g{};
     g.W = static_cast<int32_t>(W);
     g.n_rows = static_cast<int32_t>(n_rows);
@@ -534,8 +533,8 @@ bool row_geometry(const daric_tensor& t, bool page_first, const RopeLayout& L, i
     g.PS = static_cast<int32_t>(L.PS);
     g.H = static_cast<int32_t>(L.H);
     g.R = rotary_dim;
+    g.aligned = rot_units_elems % VE == 0 ? 1 : 0;
     g.n_rot = static_cast<int32_t>(rot_units_elems / VE);
-    g.ipr = static_cast<int32_t>(g.n_rot + (W - rotary_dim) / VE);
     *out = g;
     return true;
 }
@@ -873,10 +872,11 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
         if (r.jobs.empty() || r.max_elements == 0) return;
         check_rope(rope);
         DARIC_CHECK(deltas != nullptr && num_tokens != nullptr, "deltas and num_tokens must not be null");
-        // The fused kernel needs 16-byte aligned pages and dense K head rows
-        // whose rotated halves are 16-byte multiples; otherwise the call
-        // scatters with the copy kernel and then rotates in place.
-        bool fused = r.vw == 16;
+        // The fused kernels need 16-byte aligned pages and dense K head rows of
+        // a 16-byte multiple; otherwise the call scatters with the copy kernel
+        // and then rotates in place. aligned: rotated halves of whole 16-byte
+        // units, which the allocation-free entry point asks for.
+        bool fused = r.vw == 16, aligned = true;
         // Group jobs by row geometry and element type; one launch per group
         // (normally one: every layer of a model shares its geometry).
         struct Group {
@@ -914,6 +914,7 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
                         "k_scale of job ", i, " has ", L->k_scale_numel, " entries, the layer has ",
                         L->lay.H, " heads");
             fused = fused && L->geom_ok;
+            aligned = aligned && L->geom.aligned != 0;
             CopyJob& j = r.jobs[i];
             j.delta = static_cast<float>(deltas[i]);
             j.n_tokens = static_cast<int32_t>(std::min<int64_t>(num_tokens[i], kIntMax));
@@ -928,9 +929,10 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
             grp->jobs.push_back(j);
             grp->max_tiles = std::max<int64_t>(grp->max_tiles, int64_t(j.prefix) * j.n_sel);
         }
+        if (noalloc)
+            DARIC_CHECK(fused && aligned, "scatter_pages_rerotate_noalloc needs a layout the fused kernel takes "
+                                          "(16-byte aligned pages, dense K head rows, 16-byte rotated halves)");
         if (!fused) {
-            DARIC_CHECK(!noalloc, "scatter_pages_rerotate_noalloc needs a layout the fused kernel takes "
-                                  "(16-byte aligned pages, dense K head rows, 16-byte rotated halves)");
             scatter_then_rotate(r, indices, indices_offsets, deltas, num_tokens, rope, stream);
             return;
         }
@@ -955,11 +957,6 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
         size_t scratch_off = 0;
         for (const Group& gr : groups) {
             if (gr.max_tiles == 0) continue;
-            RowGeomDiv gd;
-            gd.g = gr.g;
-            gd.ipr = FastDiv(gd.g.ipr);
-            gd.tok_div = FastDiv(gd.g.tok_div);
-            gd.ps = FastDiv(gd.g.PS);
             const size_t bytes = gr.jobs.size() * sizeof(CopyJob);
             if (noalloc) {
                 DescArg arg;
@@ -973,7 +970,7 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
                     scratch_off += (bytes + 255) / 256 * 256;
                 }
                 launch_scatter_rotate(arg, static_cast<int>(gr.jobs.size()), static_cast<int>(gr.max_tiles),
-                                      gd, gr.kind, rope->is_neox != 0, rope->inv_freq, st);
+                                      gr.g, gr.kind, rope->is_neox != 0, rope->inv_freq, st);
                 continue;
             }
             // Job sets too large to travel inline are read by the fused
@@ -984,7 +981,7 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
             // and reading over the host link cost the gather ~5 us.
             DescHandOver ho(r.device, gr.jobs.data(), bytes, st, true);
             launch_scatter_rotate(ho.arg(), static_cast<int>(gr.jobs.size()), static_cast<int>(gr.max_tiles),
-                                  gd, gr.kind, rope->is_neox != 0, rope->inv_freq, st);
+                                  gr.g, gr.kind, rope->is_neox != 0, rope->inv_freq, st);
         }
         if (use) use->finish();
     });

@@ -25,12 +25,12 @@
 #include "jobs.h"
 #include "kernels.h"
 #include "launch.h"
+#include "rotate_rows.h"
 
 namespace daric {
 
 constexpr int kThreads = 256;
 constexpr int kUnroll = 8;
-constexpr int kRotUnroll = 4;
 constexpr int kMaxHalfRot = 256;  // rotary_dim / 2 limit of the LDS cos/sin table
 
 template <int VW> struct VecOf;
@@ -63,12 +63,6 @@ __device__ __forceinline__ void copy_units(const uint8_t* __restrict__ src,
             if (i < n_units) st_nt(d + i, v[u]);
         }
     }
-}
-
-template <int VW>
-__device__ __forceinline__ void copy_span(const uint8_t* __restrict__ src,
-                                          uint8_t* __restrict__ dst, int64_t span) {
-    copy_units<VW>(src, dst, static_cast<int>(span / VW));
 }
 
 // Resolves tile t of job j. Returns false when the tile is beyond the job or
@@ -115,117 +109,76 @@ __global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job
         copy_units<VW>(stage + b0, cache + b0, cnt);
 }
 
-// Fused scatter + rotation, blocks in the order of JobRuns. A work item of a K row is
-// either a rotated item (NeoX: the two 16-byte units holding pairs
-// (i, i + R/2) for i in [k*VE, k*VE + VE); GPT-J: one unit holding VE/2
-// adjacent pairs) or a pass-through unit of the row's unrotated tail. Rows
-// that are not rotated (V rows, tokens past the job's n_tokens) are copied
-// bit-exactly. The first round's loads are issued before the workgroup
-// computes the tile's cos/sin values into LDS, so the sincos latency overlaps
-// the memory latency. fp8 codes are rotated as stored: a per-head scale
-// cancels in a linear rotation.
-template <int KIND, bool NEOX>
-__global__ __launch_bounds__(kThreads) void scatter_rotate_kernel(
+// Fused scatter + rotation for any row width (rotate_rows.h). A workgroup takes
+// a part of a page span: whole rows, up to 16 KiB, in the order of JobRuns. The
+// loads are issued before the workgroup computes the tile's cos/sin values into
+// LDS, so the sincos latency overlaps the memory latency. Rows that are not
+// rotated (V rows, tokens past the job's n_tokens) are copied bit-exactly. fp8
+// codes are rotated as stored: a per-head scale cancels in a linear rotation.
+// Bound by HBM. Against one workgroup per page span with a lane per pair of
+// units, on MI355X: 48 layers x 78 pages of 64 x 576 bf16 122 -> 109 us (5.1
+// TB/s), 60 layers x 855 pages of 16 x 576 e4m3 365 -> 216 us, 6 layers x 76
+// K+V pages of 64 x 8 x 192 bf16 99 -> 69 us. Rotary halves inside a unit took a
+// scatter and a pass per layer before: 18 layers, 8 heads of 80 with 40 rotated,
+// 22000 tokens 686 -> 362 us in one launch instead of 19.
+template <int KIND, bool NEOX, bool ALIGNED>
+__global__ __launch_bounds__(kThreads) void scatter_rotate_rows_kernel(
     DescArg d, int job0, JobRuns jr, RowGeomDiv gd, const float* __restrict__ inv_freq) {
-    using E = Elem<KIND>;
-    constexpr int VE = E::VE;
-    __shared__ float s_cos[kMaxHalfRot];
-    __shared__ float s_sin[kMaxHalfRot];
+    static_assert(kThreads == kRowThreads && kRowPartUnits == kRowUnits, "one part per workgroup");
+    using RR = RowRotation<KIND, NEOX, ALIGNED>;
+    __shared__ u32x4 s_row[NEOX ? kRowUnits : 1];
+    __shared__ float4 s_cs[kRowMaxHalf / 2];
 
     int jb, unit;
     jr.at_block(blockIdx.x, jb, unit);
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
+    const int tile = static_cast<int>(gd.parts.div(static_cast<uint32_t>(unit)));
     int p, s;
     uint8_t *cache, *stage;
-    if (!resolve_tile(j, unit, p, s, cache, stage)) return;
+    if (!resolve_tile(j, tile, p, s, cache, stage)) return;
 
     const RowGeom& g = gd.g;
+    const int upr = static_cast<int>(gd.upr.d);
+    const int r0 = (unit - tile * static_cast<int>(gd.parts.d)) * gd.part_rows;
+    const int n = min(gd.part_rows, g.n_rows - r0) * upr;
+    const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(stage) + static_cast<int64_t>(r0) * upr;
+    u32x4* __restrict__ dst = reinterpret_cast<u32x4*>(cache) + static_cast<int64_t>(r0) * upr;
     const int n_valid = min(max(j.n_tokens - s * g.PS, 0), g.PS);
-    if (p != 0 || n_valid == 0 || j.delta == 0.0f || g.krows == 0) {
-        copy_span<16>(stage, cache, j.span);
+    if (p != 0 || n_valid == 0 || j.delta == 0.0f || r0 >= g.krows) {
+        copy_units<16>(reinterpret_cast<const uint8_t*>(src), reinterpret_cast<uint8_t*>(dst), n);
         return;
     }
 
-    const int half = g.R / 2;
-    const u32x4* __restrict__ src = reinterpret_cast<const u32x4*>(stage);
-    u32x4* __restrict__ dst = reinterpret_cast<u32x4*>(cache);
-    const int upr = g.W / VE;                      // 16-byte units per row
-    const int partner = NEOX ? half / VE : 0;      // unit distance of pair halves
-    const int pass0 = NEOX ? 2 * g.n_rot : g.n_rot;  // first pass-through unit
-    const int items = g.n_rows * g.ipr;
-
-    for (int base = 0; base < items; base += kThreads * kRotUnroll) {
-        u32x4 a[kRotUnroll], b[kRotUnroll];
-        int ua[kRotUnroll], kk[kRotUnroll];
-        bool rot[kRotUnroll], pair[kRotUnroll], ok[kRotUnroll];
+    // A row wider than the part: its rotated dims (at most 512) lie in the first
+    // kRowUnits units.
+    if (n > kRowUnits)
+        copy_units<16>(reinterpret_cast<const uint8_t*>(src + kRowUnits), reinterpret_cast<uint8_t*>(dst + kRowUnits),
+                       n - kRowUnits);
+    const int tid = static_cast<int>(threadIdx.x);
+    u32x4 v[kRowUnroll];
 #pragma unroll
-        for (int u = 0; u < kRotUnroll; ++u) {
-            const int it = base + u * kThreads + static_cast<int>(threadIdx.x);
-            ok[u] = it < items;
-            const int r = static_cast<int>(gd.ipr.div(static_cast<uint32_t>(it)));
-            const int k = it - r * g.ipr;
-            const int row0 = r * upr;
-            kk[u] = k;
-            if (k < g.n_rot) {
-                ua[u] = row0 + k;
-                pair[u] = NEOX;
-                const uint32_t q = gd.tok_div.div(static_cast<uint32_t>(r));
-                const int token = static_cast<int>(q - gd.ps.div(q) * g.PS);
-                rot[u] = (r < g.krows) && (token < n_valid);
-            } else {
-                ua[u] = row0 + pass0 + (k - g.n_rot);
-                pair[u] = false;
-                rot[u] = false;
-            }
-            if (ok[u]) {
-                a[u] = ld_nt(src + ua[u]);
-                if (pair[u]) b[u] = ld_nt(src + ua[u] + partner);
-            }
-        }
-        if (base == 0) {
-            for (int i = threadIdx.x; i < half; i += kThreads) {
-                float sn, cs;
-                sincosf(j.delta * inv_freq[i], &sn, &cs);
-                s_cos[i] = cs;
-                s_sin[i] = sn;
-            }
-            __syncthreads();
-        }
+    for (int u = 0; u < kRowUnroll; ++u) {
+        const int i = u * kThreads + tid;
+        v[u] = u32x4{0u, 0u, 0u, 0u};
+        if (i < n) v[u] = ld_nt(src + i);
+    }
+    RR::fill(s_cs, g.R / 2, j.delta, inv_freq);
+    if constexpr (NEOX) {
 #pragma unroll
-        for (int u = 0; u < kRotUnroll; ++u) {
-            if (!ok[u]) continue;
-            if (!rot[u]) {
-                st_nt(dst + ua[u], a[u]);
-                if (pair[u]) st_nt(dst + ua[u] + partner, b[u]);
-                continue;
-            }
-            float x[VE];
-            E::unpack(a[u], x, 1.0f);
-            if (NEOX) {
-                float y[VE];
-                E::unpack(b[u], y, 1.0f);
-                const int i0 = kk[u] * VE;
+        for (int u = 0; u < kRowUnroll; ++u) s_row[u * kThreads + tid] = v[u];
+    }
+    __syncthreads();
+    const int rot_units = RR::rotated_units(g.R);
 #pragma unroll
-                for (int e = 0; e < VE; ++e) {
-                    const float c = s_cos[i0 + e], sn = s_sin[i0 + e];
-                    const float x1 = x[e], x2 = y[e];
-                    x[e] = x1 * c - x2 * sn;
-                    y[e] = x2 * c + x1 * sn;
-                }
-                st_nt(dst + ua[u], E::pack(x, 1.0f));
-                st_nt(dst + ua[u] + partner, E::pack(y, 1.0f));
-            } else {
-                const int i0 = kk[u] * (VE / 2);
-#pragma unroll
-                for (int m = 0; m < VE / 2; ++m) {
-                    const float c = s_cos[i0 + m], sn = s_sin[i0 + m];
-                    const float x1 = x[2 * m], x2 = x[2 * m + 1];
-                    x[2 * m] = x1 * c - x2 * sn;
-                    x[2 * m + 1] = x2 * c + x1 * sn;
-                }
-                st_nt(dst + ua[u], E::pack(x, 1.0f));
-            }
-        }
+    for (int u = 0; u < kRowUnroll; ++u) {
+        const int i = u * kThreads + tid;
+        if (i >= n) continue;
+        const int row = static_cast<int>(gd.upr.div(static_cast<uint32_t>(i)));
+        const int k = i - row * upr;
+        const uint32_t q = gd.tok_div.div(static_cast<uint32_t>(r0 + row));
+        const int token = static_cast<int>(q - gd.ps.div(q) * static_cast<uint32_t>(g.PS));
+        const bool rot = k < rot_units && r0 + row < g.krows && token < n_valid;
+        st_nt(dst + i, rot ? RR::turn(v[u], s_row + (NEOX ? i - k : 0), k, s_cs, g.R / 2) : v[u]);
     }
 }
 
@@ -428,6 +381,7 @@ __global__ __launch_bounds__(kThreads) void upload_kernel(const u32x4* __restric
 }
 
 constexpr int kMaxY = 65535;
+constexpr int64_t kScatterRunsFrom = (128ll << 20) + 1, kFusedRunsFrom = 64ll << 20;   // JobRuns
 
 void launch_copy_pages(const DescArg& d, int n_jobs, int max_tiles, int64_t max_span, int vw,
                        bool gather, hipStream_t stream) {
@@ -438,7 +392,7 @@ void launch_copy_pages(const DescArg& d, int n_jobs, int max_tiles, int64_t max_
         ++log2_parts;
     const int64_t units = static_cast<int64_t>(max_tiles) << log2_parts;
     if (!gather) {
-        for_job_runs(n_jobs, units, max_span >> log2_parts, [&](int j0, const JobRuns& jr, unsigned blocks) {
+        for_job_runs(n_jobs, units, max_span >> log2_parts, kScatterRunsFrom, [&](int j0, const JobRuns& jr, unsigned blocks) {
             if (vw == 16) DARIC_LAUNCH((copy_pages_kernel<16, false>), blocks, kThreads, 0, stream, d, j0, jr, log2_parts, XcdRuns());
             else if (vw == 4) DARIC_LAUNCH((copy_pages_kernel<4, false>), blocks, kThreads, 0, stream, d, j0, jr, log2_parts, XcdRuns());
             else DARIC_LAUNCH((copy_pages_kernel<1, false>), blocks, kThreads, 0, stream, d, j0, jr, log2_parts, XcdRuns());
@@ -466,40 +420,49 @@ void launch_upload(const void* src, void* dst, size_t n16, hipStream_t stream) {
     check_launch("descriptor upload");
 }
 
-void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles,
-                           const RowGeomDiv& geom, int kind, bool neox, const float* inv_freq,
-                           hipStream_t stream) {
-    // the lane-exchange kernel needs whole rows inside a wavefront
-    const int ve = kind == kE4M3 ? 16 : 8;
-    const int upr = geom.g.W / ve;
-    const bool lane = upr > 0 && 64 % upr == 0;
-    // Lane kernel: pages cut into parts of at least 16 KiB, whole rows each.
-    // Two 16 KiB halves of the 32 KiB bf16 pages measured ~1% faster than
-    // whole pages at config 2, kernel and whole call alike (347.2 against
-    // 350.2 us per kernel, 347.5 against 350.7 us per call; bit-identical
-    // output); 8 KiB parts were 4% slower.
-    int lp = 0;
-    if (lane) {
-        const int64_t units = static_cast<int64_t>(geom.g.n_rows) * upr;   // 16-byte units per page
+void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles, const RowGeom& g, int kind, bool neox,
+                           const float* inv_freq, hipStream_t stream) {
+    RowGeomDiv gd;
+    gd.g = g;
+    gd.tok_div = FastDiv(static_cast<uint32_t>(g.tok_div));
+    gd.ps = FastDiv(static_cast<uint32_t>(g.PS));
+    const int upr = g.W / (kind == kE4M3 ? 16 : 8);
+    gd.upr = FastDiv(static_cast<uint32_t>(upr));
+    const int64_t units = static_cast<int64_t>(g.n_rows) * upr;   // 16-byte units per page span
+    // The lane-exchange kernel needs whole rows inside a wavefront and pair
+    // halves of whole units; the rows kernel takes the other rows.
+    if (g.aligned && 64 % upr == 0) {
+        // Pages cut into parts of at least 16 KiB, whole rows each. Two 16 KiB
+        // halves of the 32 KiB bf16 pages measured ~1% faster than whole pages
+        // at config 2, kernel and whole call alike (347.2 against 350.2 us per
+        // kernel, 347.5 against 350.7 us per call; bit-identical output);
+        // 8 KiB parts were 4% slower.
+        int lp = 0;
         while ((units >> (lp + 1)) * 16 >= 16384 && units % (2ll << lp) == 0 && (units >> (lp + 1)) % upr == 0)
             ++lp;
+        for_job_runs(n_jobs, static_cast<int64_t>(max_tiles) << lp, (units * 16) >> lp, kFusedRunsFrom,
+                     [&](int j0, const JobRuns& jr, unsigned blocks) {
+#define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_lane_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq, lp)
+            if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
+            else if (kind == kF16) { if (neox) DARIC_SR(kF16, true); else DARIC_SR(kF16, false); }
+            else { if (neox) DARIC_SR(kE4M3, true); else DARIC_SR(kE4M3, false); }
+#undef DARIC_SR
+            check_launch("scatter_pages_rerotate");
+        });
+        return;
     }
-    const int64_t span = static_cast<int64_t>(geom.g.n_rows) * upr * 16;
-    for_job_runs(n_jobs, static_cast<int64_t>(max_tiles) << lp, span >> lp,
-                 [&](int j0, const JobRuns& jr, unsigned blocks) {
-        if (lane) {
-#define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_lane_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, geom, inv_freq, lp)
-            if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
-            else if (kind == kF16) { if (neox) DARIC_SR(kF16, true); else DARIC_SR(kF16, false); }
-            else { if (neox) DARIC_SR(kE4M3, true); else DARIC_SR(kE4M3, false); }
+    const RowParts rp(g.n_rows, upr);
+    gd.parts = FastDiv(static_cast<uint32_t>(rp.parts));
+    gd.part_rows = rp.part_rows;
+    for_job_runs(n_jobs, static_cast<int64_t>(max_tiles) * rp.parts, static_cast<int64_t>(rp.part_rows) * upr * 16,
+                 kFusedRunsFrom, [&](int j0, const JobRuns& jr, unsigned blocks) {
+#define DARIC_SR(K, N, A) DARIC_LAUNCH((scatter_rotate_rows_kernel<K, N, A>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq)
+#define DARIC_SRA(K, N) do { if (g.aligned) DARIC_SR(K, N, true); else DARIC_SR(K, N, false); } while (0)
+        if (kind == kBF16) { if (neox) DARIC_SRA(kBF16, true); else DARIC_SRA(kBF16, false); }
+        else if (kind == kF16) { if (neox) DARIC_SRA(kF16, true); else DARIC_SRA(kF16, false); }
+        else { if (neox) DARIC_SRA(kE4M3, true); else DARIC_SRA(kE4M3, false); }
+#undef DARIC_SRA
 #undef DARIC_SR
-        } else {
-#define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, geom, inv_freq)
-            if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
-            else if (kind == kF16) { if (neox) DARIC_SR(kF16, true); else DARIC_SR(kF16, false); }
-            else { if (neox) DARIC_SR(kE4M3, true); else DARIC_SR(kE4M3, false); }
-#undef DARIC_SR
-        }
         check_launch("scatter_pages_rerotate");
     });
 }

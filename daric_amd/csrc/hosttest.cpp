@@ -74,11 +74,11 @@ int64_t daric_hosttest_layer_minor(int n_layers, int64_t n_items) {
 // (job, unit) pair is covered exactly once, every job lies in the launch and
 // no launch exceeds kMaxGridBlocks, else -1 or -2 (an oversized launch).
 // *log2_run gets the last launch's run length.
-int64_t daric_hosttest_job_runs(int n_jobs, int64_t units, int64_t unit_bytes, int32_t* log2_run) {
+int64_t daric_hosttest_job_runs(int n_jobs, int64_t units, int64_t unit_bytes, int64_t runs_from, int32_t* log2_run) {
     std::vector<uint8_t> seen(static_cast<size_t>(n_jobs) * static_cast<size_t>(units), 0);
     int64_t launches = 0;
     bool bad = false, big = false;
-    daric::for_job_runs(n_jobs, units, unit_bytes, [&](int j0, const daric::JobRuns& jr, unsigned blocks) {
+    daric::for_job_runs(n_jobs, units, unit_bytes, runs_from, [&](int j0, const daric::JobRuns& jr, unsigned blocks) {
         ++launches;
         *log2_run = static_cast<int32_t>(jr.log2_run);
         if (static_cast<int64_t>(blocks) > daric::kMaxGridBlocks || blocks == 0) big = true;

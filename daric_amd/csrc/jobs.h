@@ -82,9 +82,8 @@ struct RowGeom {
     int32_t PS;        // tokens per page
     int32_t H;         // heads
     int32_t R;         // rotary dim
-    int32_t ipr;       // work items per row
-    int32_t n_rot;     // rotated items per row
-    int32_t pad0;
+    int32_t n_rot;     // aligned: 16-byte units of a pair half (NeoX) or of the rotary dims (GPT-J)
+    int32_t aligned;   // 1 when those are whole units
 };
 
 // In-place rotation geometry (elements): K element (b, s, h, d) of a layer is

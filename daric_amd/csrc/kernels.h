@@ -37,7 +37,24 @@ struct FastDiv {
 
 struct RowGeomDiv {
     RowGeom g;
-    FastDiv ipr, tok_div, ps;
+    FastDiv tok_div, ps;
+    FastDiv upr;     // 16-byte units per row
+    FastDiv parts;   // parts a page span is cut into, each but the last of part_rows rows (rows kernel)
+    int32_t part_rows = 0;
+};
+
+// Page spans of rows of `upr` 16-byte units, cut into parts of whole rows for
+// a kernel whose workgroups hold up to kRowPartUnits units: the fewest parts,
+// of nearly equal size.
+constexpr int64_t kRowPartUnits = 1024;
+struct RowParts {
+    int32_t parts = 1, part_rows = 1;
+    RowParts(int64_t n_rows, int64_t upr) {
+        const int64_t most = std::max<int64_t>(1, kRowPartUnits / std::max<int64_t>(upr, 1));
+        const int64_t n = (n_rows + most - 1) / most;
+        part_rows = static_cast<int32_t>((n_rows + n - 1) / n);
+        parts = static_cast<int32_t>((n_rows + part_rows - 1) / part_rows);
+    }
 };
 
 // Layer-minor block order for kernels over (layer, work item) pairs: block b
@@ -102,9 +119,14 @@ void for_layer_minor(int n_layers, int64_t n_items, F&& launch) {
 // 404 -> 381 and 345 -> 332 us; fused fp8 scatter of 1280 jobs 2135 -> 2016 us;
 // two layers of 8 chunks of 1800 to 11800 tokens 214 -> 192 us, most of it the
 // shift. Runs of 64 KiB gained half as much and runs of 512 KiB nothing on the
-// fused scatter. Fewer than 16 runs per XCD leave some XCDs idle at the end, so
-// small calls take shorter runs. Runs of one unit are not shifted: units of
-// 72 KiB ran 2.5% slower so (48 layers x 78 pages of 64 rows of 576 bf16).
+// fused scatter. Below `runs_from` bytes, where a call's traffic stays mostly in
+// the 256 MB Infinity Cache, runs gained nothing and cost up to 5%: fused scatter
+// 1.00-1.08x from 64 MiB and 0.96-1.02x below, plain scatter 1.00-1.05x above
+// 128 MiB and 0.96-1.00x up to it, token-major scatter 1.01-1.04x from 512 MiB
+// and 0.95-1.02x below 256 MiB (same process, 1 to 80 layers, even and uneven
+// chunks). Fewer than 16 runs per XCD leave some XCDs idle at the end, so such
+// calls take shorter runs. Runs of one unit are not shifted: units of 72 KiB ran
+// 2.5% slower so.
 struct JobRuns {
     static constexpr uint32_t kXcds = 8;
     static constexpr int64_t kRunBytes = 128 * 1024;
@@ -133,16 +155,18 @@ struct JobRuns {
 };
 
 // Calls launch(first job, JobRuns, blocks) for launches that together cover
-// the units of every job, each of at most kMaxGridBlocks blocks.
+// the units of every job, each of at most kMaxGridBlocks blocks. Runs longer
+// than one unit are used where the jobs' units make at least runs_from bytes.
 template <class F>
-void for_job_runs(int n_jobs, int64_t units, int64_t unit_bytes, F&& launch) {
+void for_job_runs(int n_jobs, int64_t units, int64_t unit_bytes, int64_t runs_from, F&& launch) {
     if (n_jobs <= 0 || units <= 0) return;
     const int slice = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(n_jobs, kMaxGridBlocks / units)));
     for (int j0 = 0; j0 < n_jobs; j0 += slice) {
         const int nj = std::min(slice, n_jobs - j0);
         JobRuns jr;
         jr.jobs = FastDiv(static_cast<uint32_t>(nj));
-        while (jr.log2_run < 10 && (unit_bytes << (jr.log2_run + 1)) <= JobRuns::kRunBytes) ++jr.log2_run;
+        if (static_cast<int64_t>(n_jobs) * units * unit_bytes >= runs_from)
+            while (jr.log2_run < 10 && (unit_bytes << (jr.log2_run + 1)) <= JobRuns::kRunBytes) ++jr.log2_run;
         while (jr.log2_run > 0 && (nj * JobRuns::per_job(units, jr.log2_run) < JobRuns::kMinRuns ||
                                    JobRuns::blocks(nj, units, jr.log2_run) > kMaxGridBlocks))
             --jr.log2_run;
@@ -215,9 +239,8 @@ void launch_copy_pages(const DescArg& d, int n_jobs, int max_tiles, int64_t max_
 
 // Fused scatter + K re-rotation of the n_jobs CopyJobs in `d`; kind is an
 // ElemKind. All jobs share `geom`.
-void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles,
-                           const RowGeomDiv& geom, int kind, bool neox, const float* inv_freq,
-                           hipStream_t stream);
+void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles, const RowGeom& geom, int kind, bool neox,
+                           const float* inv_freq, hipStream_t stream);
 
 // In-place K re-rotation over segments of tokens. `d` holds the n_segs
 // RopeSegs, then (at byte layer_off) the n_layers K base pointers. `path`:

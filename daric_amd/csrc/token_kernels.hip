@@ -52,6 +52,7 @@ constexpr int kThreads = 256;
 constexpr int kRowUnroll = 8;
 constexpr int kLdsUnits = 512;   // 16-byte units of LDS per workgroup (8 KiB)
 constexpr int kMaxY = 65535;
+constexpr int64_t kRunsFrom = 512ll << 20;   // JobRuns
 
 template <typename T>
 __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_load(p); }
@@ -220,7 +221,7 @@ void launch_token_copy(const DescArg& d, int n_jobs, int max_parts, int64_t part
         check_launch(G ? "gather_tokens" : "scatter_tokens");                                         \
     } while (0)
     if (!gather) {
-        for_job_runs(n_jobs, max_parts, part_bytes, [&](int j0, const JobRuns& jr, unsigned blocks) {
+        for_job_runs(n_jobs, max_parts, part_bytes, kRunsFrom, [&](int j0, const JobRuns& jr, unsigned blocks) {
             DARIC_TOK(false, blocks, jr, XcdRuns());
         });
         return;

@@ -171,9 +171,9 @@ int daric_copier_scatter_pages(daric_copier* copier, const char* const* layer_na
  * tails and tokens >= num_tokens[i] are copied unchanged. For an fp8 layer
  * the e4m3 codes are decoded, rotated in fp32 and re-encoded (saturating
  * round-to-nearest-even); a per-head scale would cancel, see
- * daric_copier_register_k_scale. The one-pass kernel needs 16-byte aligned
- * pages, strides and store offsets, K head rows dense in the page span and
- * rotated halves that are 16-byte multiples; for any other layout accepted
+ * daric_copier_register_k_scale. The one-pass kernels need 16-byte aligned
+ * pages, strides and store offsets, and K head rows of 16-byte multiples dense
+ * in the page span; for any other layout accepted
  * by the copy and rotation checks, the call scatters with the copy kernel and
  * then rotates the moved tokens in place (pages with id 0 skipped by both),
  * to the same results up to the rotation's rounding. (A page listed by two
@@ -203,8 +203,9 @@ int daric_copier_scatter_pages_rerotate(daric_copier* copier,
  * or hipHostMalloc and enqueues only kernels (plus, for staged job lists,
  * one event record, and a stream wait when the stream changes; the event is
  * created once per GPU, with the array's address, at the first staging call).
- * A call whose jobs need more than the array holds, or whose layout needs the
- * scatter-then-rotate form, returns DARIC_ERR_INVALID before any device work.
+ * A call whose jobs need more than the array holds, whose layout needs the
+ * scatter-then-rotate form, or whose rotated halves are not 16-byte multiples,
+ * returns DARIC_ERR_INVALID before any device work.
  * Every call on one GPU uses that GPU's array, which keeps the last call's
  * descriptors. Eager calls are ordered on it by the library: a call on
  * another stream than the previous staging call waits for that call's

@@ -523,9 +523,12 @@ def test_layer_minor_grid_covers_every_pair_once(hosttest, n_layers, n_items, la
 ])
 def test_job_runs_grid_covers_every_unit_once(hosttest, n_jobs, units, unit_bytes, launches, log2_run):
     """The scatters' block order: every (job, unit) pair is taken by exactly
-    one block of exactly one launch, no launch passes 2^24 - 1 blocks, and
-    runs are shortened where a call has fewer than 16 per XCD."""
-    got = ctypes.c_int32(-1)
-    assert hosttest.daric_hosttest_job_runs(n_jobs, ctypes.c_int64(units), ctypes.c_int64(unit_bytes),
-                                            ctypes.byref(got)) == launches
-    assert got.value == log2_run
+    one block of exactly one launch, no launch passes 2^24 - 1 blocks, runs are
+    shortened where a call has fewer than 16 per XCD, and are one unit below
+    runs_from bytes."""
+    total = n_jobs * units * unit_bytes
+    for runs_from, want in ((total, log2_run), (total + 1, 0)):
+        got = ctypes.c_int32(-1)
+        assert hosttest.daric_hosttest_job_runs(n_jobs, ctypes.c_int64(units), ctypes.c_int64(unit_bytes),
+                                                ctypes.c_int64(runs_from), ctypes.byref(got)) == launches
+        assert got.value == want

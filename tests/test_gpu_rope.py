@@ -143,6 +143,31 @@ def test_fused_call_on_unaligned_rotary_scatters_then_rotates(dev, layout, dtype
     fused_case(dev, layout, dtype, neox, rotary_dim, seed=21)
 
 
+# (layout, page, heads, head dim, dtype, NeoX, rotary dim): rows of 10, 12, 24,
+# 36, 5 and 72 units; one part per page, several (the last one shorter), and
+# parts that hold K rows only, V rows only and both; rotary halves that end
+# inside a unit; a row wider than one part.
+ROWS_CASES = [
+    ("nhd", 16, 8, 96, torch.bfloat16, True, 96),
+    ("hnd", 16, 8, 96, torch.float16, False, 48),
+    ("pf", 16, 5, 96, torch.bfloat16, True, 96),
+    ("pf_hnd", 8, 3, 80, torch.float16, True, 40),
+    ("packed", 32, 8, 80, torch.bfloat16, True, 80),
+    ("packed", 16, 4, 80, torch.uint8, True, 80),
+    ("nhd", 64, 8, 192, torch.bfloat16, True, 96),
+    ("nhd", 1, 1, 40, torch.bfloat16, True, 20),
+    ("nhd", 3, 8, 80, torch.uint8, False, 36),
+    ("mla", 64, 1, 576, torch.bfloat16, False, 64),
+    ("mla", 16, 1, 576, torch.uint8, True, 64),
+    ("mla", 4, 1, 8704, torch.bfloat16, True, 512),
+]
+
+
+@pytest.mark.parametrize("layout,ps,h,d,dtype,neox,rotary_dim", ROWS_CASES)
+def test_fused_rows_kernel(dev, layout, ps, h, d, dtype, neox, rotary_dim):
+    fused_case(dev, layout, dtype, neox, rotary_dim, nb=200 if ps < 8 else 48, ps=ps, h=h, d=d, seed=41)
+
+
 def inplace_case(dev, layout, dtype, neox, rotary_dim, nb=40, ps=16, h=4, d=64, L=3, seed=0, plan=None):
     """plan(perm) -> (block table, segments), given a permutation of the
     block ids; by default two requests' block lists with segments as
