@@ -1,6 +1,10 @@
 // Device-side descriptors shared by the host launchers and the kernels.
 #pragma once
 
+#ifdef __HIPCC__
+#include <hip/hip_runtime.h>
+#endif
+
 #include <cstdint>
 
 namespace daric {
@@ -33,17 +37,49 @@ template <typename T>
 __device__ __forceinline__ DescPtr<T> desc_at(const DescArg& d, int byte_off) {
     return (DescPtr<T>)(d.base() + byte_off);
 }
-// Copies one descriptor out of the constant address space, word by word.
+typedef unsigned int DescWords __attribute__((ext_vector_type(4)));
+// Copies one descriptor out of the constant address space. Its loads are all
+// issued before the wait for any of them: left alone, the compiler sinks each
+// load to its first use, and a workgroup's start becomes a chain of waits, each
+// a round trip to the kernel arguments or to pinned memory (half a microsecond
+// and more on MI355X).
 template <typename T>
 __device__ __forceinline__ T desc_load(DescPtr<T> p) {
-    static_assert(sizeof(T) % 4 == 0, "descriptors are whole 32-bit words");
-    T v;
-    uint32_t* dst = reinterpret_cast<uint32_t*>(&v);
-    const __attribute__((address_space(4))) uint32_t* src =
-        reinterpret_cast<const __attribute__((address_space(4))) uint32_t*>(p);
+    constexpr int N = sizeof(T) / 16;
+    static_assert(sizeof(T) % 16 == 0 && (N == 2 || N == 5 || N == 7), "descriptors are whole 16-byte words");
+    const __attribute__((address_space(4))) DescWords* src =
+        reinterpret_cast<const __attribute__((address_space(4))) DescWords*>(p);
+    DescWords w[N];
 #pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 4; ++i) dst[i] = src[i];
+    for (int i = 0; i < N; ++i) w[i] = src[i];
+    if constexpr (N == 2) asm volatile("" : "+s"(w[0]), "+s"(w[1]));
+    else if constexpr (N == 5) asm volatile("" : "+s"(w[0]), "+s"(w[1]), "+s"(w[2]), "+s"(w[3]), "+s"(w[4]));
+    else asm volatile("" : "+s"(w[0]), "+s"(w[1]), "+s"(w[2]), "+s"(w[3]), "+s"(w[4]), "+s"(w[5]), "+s"(w[6]));
+    T v;
+    __builtin_memcpy(&v, w, sizeof(T));
     return v;
+}
+// Has the listed kernel arguments (up to 8 words or pointers) in registers before
+// what follows, so that their loads share one round trip.
+#define DARIC_ARGS_TOGETHER2(a, b) asm volatile("" ::"s"(a), "s"(b))
+#define DARIC_ARGS_TOGETHER4(a, b, c, d) asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d))
+#define DARIC_ARGS_TOGETHER6(a, b, c, d, e, f) asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d), "s"(e), "s"(f))
+// Reads one value of a list that every lane of the workgroup reads at the same
+// place (a page id, a layer's address) through the scalar unit.
+template <typename T>
+__device__ __forceinline__ T uniform_load(const T* p) {
+    return *(const __attribute__((address_space(4))) T*)p;
+}
+// The last descriptor whose tile_begin is at most `tile`, of n in ascending
+// order that start at tile 0.
+template <typename T>
+__device__ __forceinline__ int find_by_tile(DescPtr<T> p, int n, int tile) {
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (p[mid].tile_begin <= tile) lo = mid; else hi = mid - 1;
+    }
+    return lo;
 }
 #endif
 

@@ -34,7 +34,7 @@ using u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
 // Lane i writes 16-byte unit i of the blob (vector stores) to dst.
 __global__ __launch_bounds__(256) void stash_kernel(DescArg blob, u32x4* __restrict__ dst, uint32_t n16) {
     const uint32_t i = threadIdx.x;
-    if (i < n16) dst[i] = desc_load(desc_at<u32x4>(blob, static_cast<int>(i * 16)));
+    if (i < n16) dst[i] = *desc_at<u32x4>(blob, static_cast<int>(i * 16));
 }
 
 static_assert(kInlineDescBytes % 16 == 0 && kInlineDescBytes / 16 <= 256, "one stash workgroup per blob");

@@ -26,15 +26,6 @@ constexpr int kThreads = 256;
 constexpr int kVecUnroll = 2;
 constexpr int kMaxHalfRot = 256;
 
-__device__ __forceinline__ int find_segment(DescPtr<RopeSeg> segs, int n, int tile) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (segs[mid].tile_begin <= tile) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
 __device__ __forceinline__ void fill_cos_sin(float* s_cos, float* s_sin, int half, float delta,
                                              const float* __restrict__ inv_freq) {
     for (int i = threadIdx.x; i < half; i += kThreads) {
@@ -67,7 +58,7 @@ __global__ __launch_bounds__(kThreads) void rerotate_vec_kernel(
     const DescPtr<RopeSeg> segs = desc_at<RopeSeg>(d, 0);
     const DescPtr<uint8_t*> layers = desc_at<uint8_t*>(d, layer_off) + layer0;
     const int tile = static_cast<int>(blockIdx.x);
-    const RopeSeg sg = desc_load(segs + find_segment(segs, n_segs, tile));
+    const RopeSeg sg = desc_load(segs + find_by_tile(segs, n_segs, tile));
     const int tok0 = (tile - sg.tile_begin) * g.tile_tokens;
     const int n_tok = min(g.tile_tokens, sg.n_tokens - tok0);
     if (n_tok <= 0 || sg.delta == 0.0f) return;
@@ -185,11 +176,13 @@ __global__ __launch_bounds__(kThreads) void rerotate_lane_kernel(
 
     const DescPtr<RopeSeg> segs = desc_at<RopeSeg>(d, 0);
     const DescPtr<uint8_t*> layers = desc_at<uint8_t*>(d, layer_off);
+    DARIC_ARGS_TOGETHER6(d.ptr, layer_off, lm.nl, n_segs, g.PS, bt);
     int lyr;
     int64_t item;
     lm.at(lyr, item);
     const int tile = static_cast<int>(item);
-    const RopeSeg sg = desc_load(segs + find_segment(segs, n_segs, tile));
+    uint8_t* const base = layers[lyr];
+    const RopeSeg sg = desc_load(segs + find_by_tile(segs, n_segs, tile));
     if (sg.delta == 0.0f) return;
     const int page = sg.tok_start / g.PS + ((tile - sg.tile_begin) >> log2_parts);
     const int part = (tile - sg.tile_begin) & ((1 << log2_parts) - 1);
@@ -197,9 +190,9 @@ __global__ __launch_bounds__(kThreads) void rerotate_lane_kernel(
     const int lo = max(sg.tok_start - page_tok0, 0);
     const int hi = min(sg.tok_start + sg.n_tokens - page_tok0, g.PS);
     if (hi <= lo) return;
-    const int blk = bt[sg.bt_offset + page];
+    const int blk = uniform_load(bt + sg.bt_offset + page);
     if (blk < g.min_block || blk >= g.num_blocks) return;
-    u32x4* __restrict__ pg = reinterpret_cast<u32x4*>(layers[lyr] + static_cast<int64_t>(blk) * g.sb * ES);
+    u32x4* __restrict__ pg = reinterpret_cast<u32x4*>(base + static_cast<int64_t>(blk) * g.sb * ES);
 
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = tid & 63;
@@ -355,7 +348,7 @@ __global__ __launch_bounds__(kThreads) void rerotate_elem_kernel(
     const DescPtr<RopeSeg> segs = desc_at<RopeSeg>(d, 0);
     const DescPtr<uint8_t*> layers = desc_at<uint8_t*>(d, layer_off) + layer0;
     const int tile = static_cast<int>(blockIdx.x);
-    const RopeSeg sg = desc_load(segs + find_segment(segs, n_segs, tile));
+    const RopeSeg sg = desc_load(segs + find_by_tile(segs, n_segs, tile));
     const int tok0 = (tile - sg.tile_begin) * g.tile_tokens;
     const int n_tok = min(g.tile_tokens, sg.n_tokens - tok0);
     if (n_tok <= 0 || sg.delta == 0.0f) return;

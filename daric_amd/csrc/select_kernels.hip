@@ -34,15 +34,6 @@ constexpr int kMergeTok = 8;                       // selected tokens per merge 
 constexpr int kMaxGridYZ = 65535;                  // grid.y / grid.z limit; larger counts are sliced
 constexpr int kTopkLdsTokens = 8192;               // top-k keys staged in LDS up to this chunk length
 
-__device__ __forceinline__ int find_chunk(DescPtr<SelChunk> ch, int n, int tile) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (ch[mid].tile_begin <= tile) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
 // 8 elements: 16 bytes for 2-byte types, 8 bytes for fp8. Loaded raw (so a
 // lane keeps few registers per load in flight) and converted when summed.
 template <int KIND> struct Raw8 { u32x4 w; };
@@ -167,7 +158,7 @@ __global__ __launch_bounds__(kThreads) void deviation_kernel(
     const DescPtr<uint8_t*> layers = desc_at<uint8_t*>(d, layer_off);
     const int l = static_cast<int>(blockIdx.y) + l0;
     const int tile = static_cast<int>(blockIdx.x);
-    const SelChunk c = desc_load(chunks + find_chunk(chunks, n_chunks, tile));
+    const SelChunk c = desc_load(chunks + find_by_tile(chunks, n_chunks, tile));
     const int lane = static_cast<int>(threadIdx.x) & 63;
     const int wave = static_cast<int>(threadIdx.x) >> 6;
     constexpr int kTokPerWave = dev_tok_per_wave<CK>();

@@ -70,11 +70,11 @@ __device__ __forceinline__ bool resolve_part(const TokenJob& j, int q, uint8_t*&
                                              uint8_t*& stage, int& n_tok) {
     const int per_kv = j.n_sel * j.parts_per_page;
     if (q >= j.n_kv * per_kv) return false;
-    const int kv = q / per_kv;
+    const int kv = q >= per_kv ? 1 : 0;   // n_kv <= 2
     const int r = q - kv * per_kv;
-    const int s = r / j.parts_per_page;
+    const int s = static_cast<int>(static_cast<uint32_t>(r) / static_cast<uint32_t>(j.parts_per_page));
     const int pp = r - s * j.parts_per_page;
-    const int blk = j.idx[s];
+    const int blk = uniform_load(j.idx + s);
     if (blk <= 0 || blk >= j.num_blocks) return false;
     const int tok0 = pp * j.part_tokens;
     n_tok = min(j.part_tokens, j.PS - tok0);
@@ -99,6 +99,7 @@ __device__ __forceinline__ void block_part(const JobRuns& jr, const XcdRuns& xr,
 template <int VW, bool GATHER>
 __global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job0, JobRuns jr, XcdRuns xr) {
     using T = typename Unit<VW>::T;
+    DARIC_ARGS_TOGETHER4(d.ptr, job0, jr.jobs.d, xr.full);
     int jb, q;
     block_part<GATHER>(jr, xr, jb, q);
     const TokenJob j = desc_load(desc_at<TokenJob>(d, 0) + job0 + jb);
@@ -138,6 +139,7 @@ __global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job
 template <bool GATHER>
 __global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0, JobRuns jr, XcdRuns xr) {
     __shared__ u32x4 sm[kLdsUnits];
+    DARIC_ARGS_TOGETHER4(d.ptr, job0, jr.jobs.d, xr.full);
     int jb, q;
     block_part<GATHER>(jr, xr, jb, q);
     const TokenJob j = desc_load(desc_at<TokenJob>(d, 0) + job0 + jb);
