@@ -10,9 +10,9 @@
 // Block order (measured on MI355X at the Llama-3-8B shape): both directions
 // cut each tile into parts of 8 KiB. The scatter direction and the fused
 // scatter + rotation deal runs of 128 KiB of each job to the XCDs (JobRuns);
-// the gather direction runs tile-major within a job, which sustained ~6.3 TB/s
-// (256 jobs of 64 pages) and 5.8-6.0 TB/s (32 of 4096), against 5.5-5.6 TB/s
-// for whole-tile workgroups and job-minor orders.
+// the gather direction runs job by job, tile by tile (JobRows), which sustained
+// ~6.3 TB/s (256 jobs of 64 pages) and 5.8-6.0 TB/s (32 of 4096), against
+// 5.5-5.6 TB/s for whole-tile workgroups and job-minor orders.
 //
 // Pages whose block id is 0 (vLLM's null block) are skipped, as the
 // reference's kernels skip them (csrc/cache_ops/kernels.cu:26,39,69,79,104,117);
@@ -66,11 +66,7 @@ __device__ __forceinline__ void copy_units(const uint8_t* __restrict__ src,
 }
 
 // Resolves tile t of job j. Returns false when the tile is beyond the job or
-// its page is skipped. SCALAR: the page id comes through the scalar unit, so
-// that the tile's addresses stay in scalar registers. The gather of 32 KiB pages
-// in 8 KiB parts ran 354 us so against 336 us with a vector load (32 layers x
-// 8192 tokens), the scatters 1-4% faster (MI355X).
-template <bool SCALAR>
+// its page is skipped.
 __device__ __forceinline__ bool resolve_tile(const CopyJob& j, int t, int& p, int& s,
                                              uint8_t*& cache, uint8_t*& stage) {
     const int n_sel = j.n_sel;
@@ -79,7 +75,7 @@ __device__ __forceinline__ bool resolve_tile(const CopyJob& j, int t, int& p, in
     else if (t < 2 * n_sel) p = 1;      // the K/V pair of vLLM's caches: no division
     else p = t / n_sel;
     s = t - p * n_sel;
-    const int page = SCALAR ? uniform_load(j.idx + s) : j.idx[s];
+    const int page = uniform_load(j.idx + s);
     if (page <= 0 || page >= j.num_pages) return false;
     cache = j.layer + p * j.prefix_stride + static_cast<int64_t>(page) * j.page_stride;
     stage = j.stage + static_cast<int64_t>(t) * j.span;
@@ -87,24 +83,18 @@ __device__ __forceinline__ bool resolve_tile(const CopyJob& j, int t, int& p, in
 }
 
 // A unit is a part of a tile: part_units accesses of VW bytes, the last part of a
-// tile what is left. Gather: grid.y = job, grid.x = unit in the order of `xr`;
-// scatter: the order of `jr`.
-template <int VW, bool GATHER>
-__global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job0, JobRuns jr, FastDiv parts,
-                                                              int part_units, XcdRuns xr) {
-    DARIC_ARGS_TOGETHER6(d.ptr, job0, jr.jobs.d, parts.d, part_units, xr.full);
+// tile what is left.
+template <int VW, bool GATHER, class Grid>
+__global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job0, Grid grid, FastDiv parts,
+                                                              int part_units) {
+    DARIC_ARGS_TOGETHER6(d.ptr, job0, grid.begin[1], grid.cls[0].div.d, parts.d, part_units);
     int jb, unit;
-    if (GATHER) {
-        jb = static_cast<int>(blockIdx.y);
-        unit = xr.map(static_cast<int>(blockIdx.x));
-    } else {
-        jr.at_block(blockIdx.x, jb, unit);
-    }
+    grid.at_block(blockIdx.x, jb, unit);
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
     const int tile = static_cast<int>(parts.div(static_cast<uint32_t>(unit)));
     int p, s;
     uint8_t *cache, *stage;
-    if (!resolve_tile<!GATHER>(j, tile, p, s, cache, stage)) return;
+    if (!resolve_tile(j, tile, p, s, cache, stage)) return;
     const int u0 = (unit - tile * static_cast<int>(parts.d)) * part_units;
     const int cnt = min(part_units, static_cast<int>(j.span / VW) - u0);
     if (cnt <= 0) return;
@@ -135,14 +125,14 @@ __global__ __launch_bounds__(kThreads) void scatter_rotate_rows_kernel(
     __shared__ u32x4 s_row[NEOX ? kRowUnits : 1];
     __shared__ float4 s_cs[kRowMaxHalf / 2];
 
-    DARIC_ARGS_TOGETHER6(d.ptr, job0, jr.jobs.d, gd.parts.d, gd.part_rows, gd.ps.d);
+    DARIC_ARGS_TOGETHER6(d.ptr, job0, jr.begin[1], jr.cls[0].div.d, gd.parts.d, gd.ps.d);
     int jb, unit;
     jr.at_block(blockIdx.x, jb, unit);
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
     const int tile = static_cast<int>(gd.parts.div(static_cast<uint32_t>(unit)));
     int p, s;
     uint8_t *cache, *stage;
-    if (!resolve_tile<true>(j, tile, p, s, cache, stage)) return;
+    if (!resolve_tile(j, tile, p, s, cache, stage)) return;
 
     const RowGeom& g = gd.g;
     const int upr = static_cast<int>(gd.upr.d);
@@ -229,13 +219,13 @@ __global__ __launch_bounds__(kThreads) void scatter_rotate_lane_kernel(
     __shared__ float s_sin[kMaxHalfRot];
     __shared__ float4 s_cs[kMaxHalfRot / 2];   // CSL: (cos, sin) of pairs 2i and 2i+1
 
-    DARIC_ARGS_TOGETHER6(d.ptr, job0, jr.jobs.d, gd.g.W, gd.ps.d, log2_parts);
+    DARIC_ARGS_TOGETHER6(d.ptr, job0, jr.begin[1], jr.cls[0].div.d, gd.ps.d, log2_parts);
     int jb, unit;
     jr.at_block(blockIdx.x, jb, unit);
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
     int p, s;
     uint8_t *cache, *stage;
-    if (!resolve_tile<true>(j, unit >> log2_parts, p, s, cache, stage)) return;
+    if (!resolve_tile(j, unit >> log2_parts, p, s, cache, stage)) return;
     const int n_units = static_cast<int>(j.span / 16);
     const int per = n_units >> log2_parts;
     const int u0 = (unit & ((1 << log2_parts) - 1)) * per;
@@ -388,39 +378,35 @@ __global__ __launch_bounds__(kThreads) void upload_kernel(const u32x4* __restric
     if (i < n16) dst[i] = src[i];
 }
 
-constexpr int kMaxY = 65535;
 constexpr int64_t kScatterRunsFrom = (128ll << 20) + 1, kFusedRunsFrom = 64ll << 20;   // JobRuns
 
-void launch_copy_pages(const DescArg& d, int n_jobs, int max_tiles, int64_t max_span, int vw,
+void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t max_span, int vw,
                        bool gather, hipStream_t stream) {
+    if (classes.empty()) return;
     // Tiles cut into parts of 8 KiB (two accesses of 16 bytes per lane), the last
     // part of a tile what is left, so that every part but that one fills its
     // lanes. Tiles above 64 KiB ran 1.1-1.25x faster than in eight parts each, and
-    // 72 KiB ones 1.1x faster than in eight parts of 9 KiB (MI355X).
+    // 72 KiB ones 1.1x faster than in eight parts of 9 KiB; parts of 4 KiB ran
+    // 0.88-1.05x of these rates (MI355X, tiles of 4 to 256 KiB).
     int64_t part = 8192;
-    while ((max_span + part - 1) / part * max_tiles > kMaxGridBlocks) part *= 2;
+    while ((max_span + part - 1) / part * classes[0].tiles > kMaxGridBlocks - 8) part *= 2;
     const FastDiv parts(static_cast<uint32_t>((max_span + part - 1) / part));
     const int part_units = static_cast<int>(part / vw);
-    const int64_t units = static_cast<int64_t>(max_tiles) * parts.d;
-    if (!gather) {
-        for_job_runs(n_jobs, units, part, kScatterRunsFrom, [&](int j0, const JobRuns& jr, unsigned blocks) {
-            if (vw == 16) DARIC_LAUNCH((copy_pages_kernel<16, false>), blocks, kThreads, 0, stream, d, j0, jr, parts, part_units, XcdRuns());
-            else if (vw == 4) DARIC_LAUNCH((copy_pages_kernel<4, false>), blocks, kThreads, 0, stream, d, j0, jr, parts, part_units, XcdRuns());
-            else DARIC_LAUNCH((copy_pages_kernel<1, false>), blocks, kThreads, 0, stream, d, j0, jr, parts, part_units, XcdRuns());
-            check_launch("scatter_pages");
+    if (gather) {
+        for_job_rows(classes, parts.d, part, [&](int j0, const JobRows& g, unsigned blocks) {
+#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, true, JobRows>), blocks, kThreads, 0, stream, d, j0, g, parts, part_units)
+            if (vw == 16) DARIC_CP(16); else if (vw == 4) DARIC_CP(4); else DARIC_CP(1);
+#undef DARIC_CP
+            check_launch("gather_pages");
         });
         return;
     }
-    // gather: tile-major within a job
-    const XcdRuns xr(units, part);
-    for (int j0 = 0; j0 < n_jobs; j0 += kMaxY) {
-        const int nj = std::min(kMaxY, n_jobs - j0);
-        const dim3 grid(static_cast<unsigned>(units), static_cast<unsigned>(nj));
-        if (vw == 16) DARIC_LAUNCH((copy_pages_kernel<16, true>), grid, kThreads, 0, stream, d, j0, JobRuns(), parts, part_units, xr);
-        else if (vw == 4) DARIC_LAUNCH((copy_pages_kernel<4, true>), grid, kThreads, 0, stream, d, j0, JobRuns(), parts, part_units, xr);
-        else DARIC_LAUNCH((copy_pages_kernel<1, true>), grid, kThreads, 0, stream, d, j0, JobRuns(), parts, part_units, xr);
-        check_launch("gather_pages");
-    }
+    for_job_runs(classes, parts.d, part, kScatterRunsFrom, [&](int j0, const JobRuns& g, unsigned blocks) {
+#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, false, JobRuns>), blocks, kThreads, 0, stream, d, j0, g, parts, part_units)
+        if (vw == 16) DARIC_CP(16); else if (vw == 4) DARIC_CP(4); else DARIC_CP(1);
+#undef DARIC_CP
+        check_launch("scatter_pages");
+    });
 }
 
 void launch_upload(const void* src, void* dst, size_t n16, hipStream_t stream) {
@@ -431,8 +417,8 @@ void launch_upload(const void* src, void* dst, size_t n16, hipStream_t stream) {
     check_launch("descriptor upload");
 }
 
-void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles, const RowGeom& g, int kind, bool neox,
-                           const float* inv_freq, hipStream_t stream) {
+void launch_scatter_rotate(const DescArg& d, const JobClasses& classes, const RowGeom& g, int kind,
+                           bool neox, const float* inv_freq, hipStream_t stream) {
     RowGeomDiv gd;
     gd.g = g;
     gd.tok_div = FastDiv(static_cast<uint32_t>(g.tok_div));
@@ -451,7 +437,7 @@ void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles, const Ro
         int lp = 0;
         while ((units >> (lp + 1)) * 16 >= 16384 && units % (2ll << lp) == 0 && (units >> (lp + 1)) % upr == 0)
             ++lp;
-        for_job_runs(n_jobs, static_cast<int64_t>(max_tiles) << lp, (units * 16) >> lp, kFusedRunsFrom,
+        for_job_runs(classes, 1ll << lp, (units * 16) >> lp, kFusedRunsFrom,
                      [&](int j0, const JobRuns& jr, unsigned blocks) {
 #define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_lane_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq, lp)
             if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
@@ -465,7 +451,7 @@ void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles, const Ro
     const RowParts rp(g.n_rows, upr);
     gd.parts = FastDiv(static_cast<uint32_t>(rp.parts));
     gd.part_rows = rp.part_rows;
-    for_job_runs(n_jobs, static_cast<int64_t>(max_tiles) * rp.parts, static_cast<int64_t>(rp.part_rows) * upr * 16,
+    for_job_runs(classes, rp.parts, static_cast<int64_t>(rp.part_rows) * upr * 16,
                  kFusedRunsFrom, [&](int j0, const JobRuns& jr, unsigned blocks) {
 #define DARIC_SR(K, N, A) DARIC_LAUNCH((scatter_rotate_rows_kernel<K, N, A>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq)
 #define DARIC_SRA(K, N) do { if (g.aligned) DARIC_SR(K, N, true); else DARIC_SR(K, N, false); } while (0)

@@ -69,31 +69,53 @@ int64_t daric_hosttest_layer_minor(int n_layers, int64_t n_items) {
     return bad ? -1 : launches;
 }
 
-// Walks the launches for_job_runs makes for n_jobs x units and decodes every
-// block with JobRuns::at_block. Returns the number of launches when every
-// (job, unit) pair is covered exactly once, every job lies in the launch and
-// no launch exceeds kMaxGridBlocks, else -1 or -2 (an oversized launch).
-// *log2_run gets the last launch's run length.
-int64_t daric_hosttest_job_runs(int n_jobs, int64_t units, int64_t unit_bytes, int64_t runs_from, int32_t* log2_run) {
-    std::vector<uint8_t> seen(static_cast<size_t>(n_jobs) * static_cast<size_t>(units), 0);
+// Walks the launches for_job_runs (gather 0) or for_job_rows (gather 1) makes for
+// jobs of tiles[i] tiles of `parts` units, ordered by order_jobs, and decodes
+// every block. Returns the number of launches when every unit of every job is
+// taken by exactly one block, every job lies in its launch and no launch exceeds
+// kMaxGridBlocks, else -1 or -2 (an oversized launch). *log2_run gets the last
+// launch's run length, *idle the blocks that no unit of a job answers to.
+int64_t daric_hosttest_job_grid(int gather, const int64_t* tiles, int64_t n, int64_t parts, int64_t unit_bytes,
+                                int64_t runs_from, int32_t* log2_run, int64_t* idle) {
+    struct Job { int64_t id, tiles; };
+    std::vector<Job> jobs;
+    for (int64_t i = 0; i < n; ++i) jobs.push_back({i, tiles[i]});
+    const daric::JobClasses classes = daric::order_jobs(jobs, [](const Job& j) { return j.tiles; });
+    std::vector<std::vector<uint8_t>> seen(static_cast<size_t>(n));
+    for (int64_t i = 0; i < n; ++i) seen[static_cast<size_t>(i)].assign(static_cast<size_t>(tiles[i] * parts), 0);
     int64_t launches = 0;
     bool bad = false, big = false;
-    daric::for_job_runs(n_jobs, units, unit_bytes, runs_from, [&](int j0, const daric::JobRuns& jr, unsigned blocks) {
+    *idle = 0;
+    int64_t at = 0;
+    for (int k = 0; k < classes.n; ++k) {    // longest class first, the jobs of a class in their order
+        for (int64_t i = at; i < at + classes[k].jobs; ++i) {
+            const int64_t t = jobs[static_cast<size_t>(i)].tiles;
+            if (t > classes[k].tiles || t <= 0 || (i > at && jobs[static_cast<size_t>(i)].id < jobs[static_cast<size_t>(i - 1)].id)) bad = true;
+        }
+        at += classes[k].jobs;
+        if (k > 0 && classes[k].tiles >= classes[k - 1].tiles) bad = true;
+    }
+    for (int64_t i = at; i < n; ++i) bad = bad || jobs[static_cast<size_t>(i)].tiles != 0;
+    const auto walk = [&](int j0, const auto& g, unsigned blocks) {
         ++launches;
-        *log2_run = static_cast<int32_t>(jr.log2_run);
+        *log2_run = static_cast<int32_t>(g.log2_run);
         if (static_cast<int64_t>(blocks) > daric::kMaxGridBlocks || blocks == 0) big = true;
         for (uint32_t b = 0; b < blocks; ++b) {
             int job, unit;
-            jr.at_block(b, job, unit);
-            if (job < 0 || job >= static_cast<int>(jr.jobs.d) || j0 + job >= n_jobs || unit < 0) { bad = true; continue; }
-            if (unit >= units) continue;   // past the job's end: the kernels' tile check drops it
-            uint8_t& s = seen[static_cast<size_t>(j0 + job) * static_cast<size_t>(units) + static_cast<size_t>(unit)];
+            g.at_block(b, job, unit);
+            if (job < 0 || j0 + job >= n || unit < 0) { bad = true; continue; }
+            const Job& j = jobs[static_cast<size_t>(j0 + job)];
+            if (unit >= j.tiles * parts) { ++*idle; continue; }   // the kernels' tile check drops it
+            uint8_t& s = seen[static_cast<size_t>(j.id)][static_cast<size_t>(unit)];
             if (s) bad = true;
             s = 1;
         }
-    });
-    for (uint8_t s : seen)
-        if (!s) bad = true;
+    };
+    if (gather) daric::for_job_rows(classes, parts, unit_bytes, walk);
+    else daric::for_job_runs(classes, parts, unit_bytes, runs_from, walk);
+    for (const auto& v : seen)
+        for (uint8_t s : v)
+            if (!s) bad = true;
     if (big) return -2;
     return bad ? -1 : launches;
 }

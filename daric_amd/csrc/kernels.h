@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <vector>
 
 #include <hip/hip_runtime_api.h>
 
@@ -103,22 +104,173 @@ void for_layer_minor(int n_layers, int64_t n_items, F&& launch) {
     }
 }
 
+// The jobs of a page copy by length: classes of consecutive jobs of `tiles`
+// tiles each (the longest of the class), longest first (order_jobs). A grid made
+// from them has workgroups for the tiles that are there; one sized by the
+// longest job gave every job as many, and a workgroup that finds nothing to do
+// still costs its place in the queue (about 0.7 ns on the whole chip). Same
+// process, MI355X, against the grid of the longest job, in 8 KiB parts: gather
+// into rows of 24 KiB pages 168 -> 157 us (three chunks of 1111 to 3000 tokens),
+// 48 KiB 411 -> 392 us (five of 1462 to 2629), 72 KiB 172 -> 161 us (six of 64
+// to 4000).
+struct JobClass {
+    int64_t jobs, tiles;
+};
+constexpr int kJobClasses = 8;
+struct JobClasses {
+    int n = 0;
+    JobClass c[kJobClasses];
+    bool empty() const { return n == 0; }
+    const JobClass& operator[](int k) const { return c[k]; }
+    int64_t jobs() const {
+        int64_t s = 0;
+        for (int k = 0; k < n; ++k) s += c[k].jobs;
+        return s;
+    }
+};
+
+// Joins neighbours of a descending list of lengths until at most kJobClasses
+// are left, each time those where that adds the fewest idle workgroups.
+// joined[i] is the class that entry i ends up in. Returns their number.
+inline int join_classes(JobClass* d, int n, int* joined) {
+    int at[64], live = n;
+    for (int i = 0; i < n; ++i) at[i] = i;     // the entry that starts live class k
+    while (live > kJobClasses) {
+        int best = 0;
+        int64_t least = -1;
+        for (int k = 0; k + 1 < live; ++k) {
+            const int64_t idle = (d[at[k]].tiles - d[at[k + 1]].tiles) * d[at[k + 1]].jobs;
+            if (least < 0 || idle < least) { least = idle; best = k; }
+        }
+        d[at[best]].jobs += d[at[best + 1]].jobs;
+        for (int k = best + 1; k + 1 < live; ++k) at[k] = at[k + 1];
+        --live;
+    }
+    for (int i = 0, k = -1; i < n; ++i) {
+        if (k + 1 < live && at[k + 1] == i) ++k;
+        joined[i] = k;
+    }
+    for (int k = 0; k < live; ++k) d[k] = d[at[k]];
+    return live;
+}
+
+// Sorts `jobs` by descending class of count(job), keeping the order within a
+// class, and returns the classes (jobs without tiles come last, in none).
+template <class Job, class Count>
+JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
+    JobClasses out;
+    const size_t n = jobs.size();
+    if (n == 0) return out;
+    constexpr int kLengths = 64;
+    JobClass d[kLengths];
+    int nd = 0, last = 0;
+    std::vector<uint8_t> of(n);
+    int64_t longest = 0;
+    for (size_t i = 0; i < n; ++i) longest = std::max<int64_t>(longest, count(jobs[i]));
+    if (longest == 0) return out;
+    // lengths in at most 63 steps of the longest (exact up to 63 tiles, or where
+    // no more than 64 lengths occur), rounded up
+    int64_t step = 1;
+    for (size_t i = 0; i < n; ++i) {
+        const int64_t t = (count(jobs[i]) + step - 1) / step * step;
+        if (nd == 0 || d[last].tiles != t) {
+            for (last = 0; last < nd && d[last].tiles != t;) ++last;
+            if (last == nd) {
+                if (nd == kLengths) {     // too many lengths: start again in coarser steps
+                    step = (longest + 62) / 63;
+                    nd = 0;
+                    i = static_cast<size_t>(-1);
+                    continue;
+                }
+                d[nd++] = {0, t};
+            }
+        }
+        ++d[last].jobs;
+        of[i] = static_cast<uint8_t>(last);
+    }
+    if (nd == 1) {
+        out.n = 1;
+        out.c[0] = {static_cast<int64_t>(n), longest};
+        return out;
+    }
+    int rank[kLengths], joined[kLengths];
+    JobClass s[kLengths];
+    int ns = 0;
+    for (int i = 0; i < nd; ++i) {
+        rank[i] = 0;
+        for (int k = 0; k < nd; ++k) rank[i] += d[k].tiles > d[i].tiles ? 1 : 0;
+        if (d[i].tiles > 0) ++ns;
+    }
+    for (int i = 0; i < nd; ++i)
+        if (d[i].tiles > 0) s[rank[i]] = d[i];
+    out.n = join_classes(s, ns, joined);
+    size_t at[kJobClasses + 1] = {0};
+    for (int k = 0; k < out.n; ++k) {
+        out.c[k] = {s[k].jobs, std::min(s[k].tiles, longest)};
+        at[k + 1] = at[k] + static_cast<size_t>(s[k].jobs);
+    }
+    std::vector<Job> sorted(n);
+    for (size_t i = 0; i < n; ++i) {
+        const int r = of[i];
+        sorted[at[d[r].tiles > 0 ? joined[rank[r]] : out.n]++] = jobs[i];
+    }
+    jobs.swap(sorted);
+    return out;
+}
+
+// Where the blocks of each class begin, and what they divide by. A block compares
+// its place with all the begins, without a branch before the last: returning
+// early for the first class ran the gathers of even jobs 2-4% slower and the
+// scatters up to 1% (MI355X).
+struct JobGrid {
+    struct Class {
+        uint32_t first = 0;
+        FastDiv div;
+    };
+    uint32_t begin[kJobClasses];
+    Class cls[kJobClasses];
+    uint32_t log2_run = 0;
+    JobGrid() {
+        for (uint32_t& b : begin) b = 0xffffffffu;
+        begin[0] = 0;
+    }
+    inline DARIC_HD Class find(uint32_t r, uint32_t& base) const {
+        uint32_t k = 0;
+        base = 0;
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+#endif
+        for (int i = 1; i < kJobClasses; ++i)
+            if (r >= begin[i]) { k = static_cast<uint32_t>(i); base = begin[i]; }
+#ifdef __HIP_DEVICE_COMPILE__
+        const DescPtr<uint32_t> p = (DescPtr<uint32_t>)(const uint32_t*)cls + 4 * k;
+        Class c;
+        c.first = p[0]; c.div.d = p[1]; c.div.m = p[2]; c.div.s = p[3];
+        return c;
+#else
+        return cls[k];
+#endif
+    }
+};
+static_assert(sizeof(JobGrid::Class) == 16, "JobGrid::Class layout");
+
 // Block order of the kernels that scatter from staging into the pages of many
 // jobs (one job per layer and chunk). Workgroups are dispatched to the 8 XCDs
 // in turn; block b is place b / 8 % run of the (b / 8 / run)-th run of XCD
 // b % 8, and the runs of `run` consecutive units are dealt to the XCDs job by
-// job: run r is unit block r / n of job (r + r / n) % n. So an XCD reads and
-// writes a job's consecutive parts while all jobs advance together, and the
-// shift by r / n moves a job on to the next XCD with each run, so that a call
-// of few jobs of unequal length still loads the XCDs alike.
+// job: round q takes unit block q of each of the n jobs that reach it, job
+// (i + q) % n being the i-th. So an XCD reads and writes a job's consecutive
+// parts while all jobs advance together, and the shift by q moves a job on to
+// the next XCD with each run, so that a call of few jobs still loads the XCDs
+// alike. A class's `first` is its first round, its divisor the jobs that reach
+// those rounds.
 // The scatters wait on HBM writes to random pages, whose rate depends on how
 // the concurrent writes fall on the memory channels. Runs of 128 KiB against
 // the plain job-minor order (run = 1), on MI355X, same process: fused scatter
 // of 256 jobs (32 layers x 8 chunks of 1024 tokens, bf16) 408 -> 391 us on
 // layers 256 MiB apart and 346 -> 341 us on layers 4 GiB apart, plain scatter
-// 404 -> 381 and 345 -> 332 us; fused fp8 scatter of 1280 jobs 2135 -> 2016 us;
-// two layers of 8 chunks of 1800 to 11800 tokens 214 -> 192 us, most of it the
-// shift. Runs of 64 KiB gained half as much and runs of 512 KiB nothing on the
+// 404 -> 381 and 345 -> 332 us; fused fp8 scatter of 1280 jobs 2135 -> 2016 us.
+// Runs of 64 KiB gained half as much and runs of 512 KiB nothing on the
 // fused scatter. Below `runs_from` bytes, where a call's traffic stays mostly in
 // the 256 MB Infinity Cache, runs gained nothing and cost up to 5%: fused scatter
 // 1.00-1.08x from 64 MiB and 0.96-1.02x below, plain scatter 1.00-1.05x above
@@ -127,80 +279,132 @@ void for_layer_minor(int n_layers, int64_t n_items, F&& launch) {
 // chunks). Fewer than 16 runs per XCD leave some XCDs idle at the end, so such
 // calls take shorter runs. Runs of one unit are not shifted: units of 72 KiB ran
 // 2.5% slower so.
-struct JobRuns {
+struct JobRuns : JobGrid {
     static constexpr uint32_t kXcds = 8;
     static constexpr int64_t kRunBytes = 128 * 1024;
     static constexpr int64_t kMinRuns = 16 * kXcds;
-    FastDiv jobs;
-    uint32_t log2_run = 0;
-    // runs of a job
-    static int64_t per_job(int64_t units, uint32_t log2) { return (units + (1ll << log2) - 1) >> log2; }
-    // blocks that cover n_jobs x units; units past a job's end come out as well
-    static int64_t blocks(int64_t n_jobs, int64_t units, uint32_t log2) {
-        const int64_t runs = n_jobs * per_job(units, log2);
-        return log2 == 0 ? runs : ((runs + kXcds - 1) / kXcds * kXcds) << log2;
-    }
     inline DARIC_HD void at_block(uint32_t b, int& job, int& unit) const {
         const uint32_t i = b >> 3;
         const uint32_t r = ((i >> log2_run) << 3) + (b & (kXcds - 1));
-        const uint32_t q = jobs.div(r);
-        uint32_t j = r - q * jobs.d;
+        uint32_t base;
+        const Class c = find(r, base);
+        const uint32_t q0 = c.div.div(r - base);
+        const uint32_t q = c.first + q0;
+        uint32_t j = r - base - q0 * c.div.d;
         if (log2_run != 0) {
-            j += q - jobs.div(q) * jobs.d;
-            if (j >= jobs.d) j -= jobs.d;
+            j += q - c.div.div(q) * c.div.d;
+            if (j >= c.div.d) j -= c.div.d;
         }
         job = static_cast<int>(j);
         unit = static_cast<int>((q << log2_run) + (i & ((1u << log2_run) - 1)));
     }
 };
 
-// Calls launch(first job, JobRuns, blocks) for launches that together cover
-// the units of every job, each of at most kMaxGridBlocks blocks. Runs longer
-// than one unit are used where the jobs' units make at least runs_from bytes.
-template <class F>
-void for_job_runs(int n_jobs, int64_t units, int64_t unit_bytes, int64_t runs_from, F&& launch) {
-    if (n_jobs <= 0 || units <= 0) return;
-    const int slice = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(n_jobs, kMaxGridBlocks / units)));
-    for (int j0 = 0; j0 < n_jobs; j0 += slice) {
-        const int nj = std::min(slice, n_jobs - j0);
-        JobRuns jr;
-        jr.jobs = FastDiv(static_cast<uint32_t>(nj));
-        if (static_cast<int64_t>(n_jobs) * units * unit_bytes >= runs_from)
-            while (jr.log2_run < 10 && (unit_bytes << (jr.log2_run + 1)) <= JobRuns::kRunBytes) ++jr.log2_run;
-        while (jr.log2_run > 0 && (nj * JobRuns::per_job(units, jr.log2_run) < JobRuns::kMinRuns ||
-                                   JobRuns::blocks(nj, units, jr.log2_run) > kMaxGridBlocks))
-            --jr.log2_run;
-        launch(j0, jr, static_cast<unsigned>(JobRuns::blocks(nj, units, jr.log2_run)));
+// Block order of the gathers: job by job, unit by unit, since consecutive units
+// write consecutive staging bytes. Workgroups are dispatched to the 8 XCDs in
+// turn, so neighbouring parts of the staging side would be written from
+// different XCDs: in rows of a multiple of 8 units (every job's row is padded to
+// one, except rows of fewer than 64) the units are permuted so that XCD x's i-th
+// unit becomes unit (i / run * 8 + x) * run + i % run: each XCD writes runs of
+// `run` consecutive units. Runs of ~256 KiB measured fastest on MI355X (gathers
+// 1-3% faster than the plain order); runs of 32-64 KiB were slower than the plain
+// order. Units past the last whole group keep their place. A class's `first` is
+// its first job, its divisor the units of a job's row.
+struct JobRows : JobGrid {
+    static constexpr uint32_t kXcds = 8;
+    static constexpr int64_t kRunBytes = 256 * 1024;
+    inline DARIC_HD void at_block(uint32_t b, int& job, int& unit) const {
+        uint32_t base;
+        const Class c = find(b, base);
+        const uint32_t j = c.div.div(b - base);
+        const uint32_t u = b - base - j * c.div.d;
+        job = static_cast<int>(c.first + j);
+        const uint32_t full = c.div.d % kXcds ? 0 : c.div.d >> (3 + log2_run) << (3 + log2_run);
+        const uint32_t i = u >> 3, x = u & (kXcds - 1);
+        unit = static_cast<int>(u >= full ? u : ((((i >> log2_run) << 3) + x) << log2_run) + (i & ((1u << log2_run) - 1)));
+    }
+};
+
+// Calls launch(first job, grid, blocks) for launches that together cover the
+// jobs' units, parts per tile, each launch of at most kMaxGridBlocks blocks:
+// slices of jobs where one launch cannot hold them all.
+template <class Grid, class Build, class F>
+void for_job_slices(const JobClasses& classes, int64_t parts, Build&& build, F&& launch) {
+    if (classes.empty() || parts <= 0) return;
+    const int64_t n = classes.jobs();
+    const int64_t row = classes[0].tiles * parts + 8;
+    const int64_t slice = std::max<int64_t>(1, std::min<int64_t>(n, kMaxGridBlocks / row));
+    for (int64_t j0 = 0; j0 < n; j0 += slice) {
+        JobClasses part;
+        int64_t at = 0;
+        for (int k = 0; k < classes.n; ++k) {
+            const int64_t lo = std::max(at, j0), hi = std::min(at + classes[k].jobs, j0 + slice);
+            if (hi > lo) part.c[part.n++] = {hi - lo, classes[k].tiles * parts};
+            at += classes[k].jobs;
+        }
+        Grid g;
+        const int64_t blocks = build(part, g);
+        launch(static_cast<int>(j0), g, static_cast<unsigned>(blocks));
     }
 }
 
-// XCD-aware unit order for grids whose consecutive units write consecutive
-// bytes (the gathers: staging is the contiguous side). Workgroups are
-// dispatched to the 8 XCDs round-robin, so with a grid row length divisible
-// by 8, unit u runs on XCD u % 8 and neighbouring parts of the staging side
-// would be written from different XCDs. map() permutes [0, full) so that XCD
-// x's i-th unit becomes unit (i / run * 8 + x) * run + i % run: each XCD
-// writes runs of `run` consecutive units. Runs of ~256 KiB measured fastest
-// on MI355X (gathers 1-3% faster than the plain order); runs of 32-64 KiB
-// were slower than the plain order. Units past `full` keep their place.
-struct XcdRuns {
-    static constexpr int kXcds = 8;
-    static constexpr int64_t kRunBytes = 256 * 1024;
-    int32_t log2_run = 0;   // 0: identity
-    int32_t full = 0;
-    XcdRuns() = default;
-    XcdRuns(int64_t grid_x, int64_t unit_bytes) {
-        if (grid_x % kXcds != 0 || unit_bytes <= 0) return;
-        while (log2_run < 10 && (unit_bytes << (log2_run + 1)) <= kRunBytes) ++log2_run;
-        const int64_t group = static_cast<int64_t>(kXcds) << log2_run;
-        full = static_cast<int32_t>(grid_x / group * group);
-    }
-    inline DARIC_HD int map(int u) const {
-        if (log2_run == 0 || u >= full) return u;
-        const int i = u >> 3, x = u & 7;
-        return ((((i >> log2_run) << 3) + x) << log2_run) + (i & ((1 << log2_run) - 1));
-    }
-};
+// JobRuns launches. Runs longer than one unit are used where the units make at
+// least runs_from bytes.
+template <class F>
+void for_job_runs(const JobClasses& classes, int64_t parts, int64_t unit_bytes, int64_t runs_from, F&& launch) {
+    int64_t total = 0;
+    for (int k = 0; k < classes.n; ++k) total += classes[k].jobs * classes[k].tiles * parts;
+    for_job_slices<JobRuns>(classes, parts, [&](const JobClasses& cl, JobRuns& g) {
+        const auto runs = [&](uint32_t log2) {
+            int64_t r = 0;
+            for (int k = 0; k < cl.n; ++k) r += cl[k].jobs * ((cl[k].tiles + (1ll << log2) - 1) >> log2);
+            return r;
+        };
+        const auto blocks = [&](uint32_t log2) {
+            return log2 == 0 ? runs(0) : ((runs(log2) + JobRuns::kXcds - 1) / JobRuns::kXcds * JobRuns::kXcds) << log2;
+        };
+        if (total * unit_bytes >= runs_from)
+            while (g.log2_run < 10 && (unit_bytes << (g.log2_run + 1)) <= JobRuns::kRunBytes) ++g.log2_run;
+        while (g.log2_run > 0 && (runs(g.log2_run) < JobRuns::kMinRuns || blocks(g.log2_run) > kMaxGridBlocks))
+            --g.log2_run;
+        // rounds [0, shortest class's runs) hold every job, the next ones the
+        // longer classes' jobs, and so on
+        int64_t n = cl.jobs(), at = 0, round = 0;
+        int k = 0;
+        for (int i = cl.n - 1; i >= 0; --i) {
+            const int64_t end = (cl[i].tiles + (1ll << g.log2_run) - 1) >> g.log2_run;
+            if (end > round) {
+                g.begin[k] = static_cast<uint32_t>(at);
+                g.cls[k].first = static_cast<uint32_t>(round);
+                g.cls[k].div = FastDiv(static_cast<uint32_t>(n));
+                ++k;
+                at += n * (end - round);
+                round = end;
+            }
+            n -= cl[i].jobs;
+        }
+        return blocks(g.log2_run);
+    }, launch);
+}
+
+// JobRows launches.
+template <class F>
+void for_job_rows(const JobClasses& classes, int64_t parts, int64_t unit_bytes, F&& launch) {
+    for_job_slices<JobRows>(classes, parts, [&](const JobClasses& cl, JobRows& g) {
+        while (g.log2_run < 10 && (unit_bytes << (g.log2_run + 1)) <= JobRows::kRunBytes) ++g.log2_run;
+        int64_t at = 0, job = 0;
+        for (int k = 0; k < cl.n; ++k) {
+            const int64_t padded = (cl[k].tiles + 7) / 8 * 8;
+            const int64_t row = cl[k].tiles < 64 || padded > kMaxGridBlocks ? cl[k].tiles : padded;
+            g.begin[k] = static_cast<uint32_t>(at);
+            g.cls[k].first = static_cast<uint32_t>(job);
+            g.cls[k].div = FastDiv(static_cast<uint32_t>(row));
+            at += row * cl[k].jobs;
+            job += cl[k].jobs;
+        }
+        return at;
+    }, launch);
+}
 
 // One token-major copy job: the pages idx[0 .. n_sel) of one layer to or from
 // staging laid out as [n_kv][n_sel * PS][H][row_bytes] (K rows, then V rows).
@@ -227,20 +431,21 @@ static_assert(sizeof(TokenJob) == 112, "TokenJob layout");
 
 // Token-major gather (staging <- cache) or scatter; lds selects the
 // LDS-staged transpose for head-major pages ([H, PS, D] dense); vw is 16 or 1.
-// part_bytes: the largest part's staging bytes (sets the XCD run length).
-void launch_token_copy(const DescArg& d, int n_jobs, int max_parts, int64_t part_bytes, int vw,
+// part_bytes: the largest part's staging bytes (sets the XCD run length). The
+// jobs are ordered by their parts (order_jobs).
+void launch_token_copy(const DescArg& d, const JobClasses& classes, int64_t part_bytes, int vw,
                        bool lds, bool gather, hipStream_t stream);
 
-// Plain page copies of the n_jobs CopyJobs in `d`. vw is the access width in
-// bytes (16, 4 or 1); max_span
-// is the largest page span (bytes) of the jobs.
-void launch_copy_pages(const DescArg& d, int n_jobs, int max_tiles, int64_t max_span, int vw,
+// Plain page copies of the CopyJobs in `d`, ordered by their tiles (order_jobs).
+// vw is the access width in bytes (16, 4 or 1); max_span is the largest page
+// span (bytes) of the jobs.
+void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t max_span, int vw,
                        bool gather, hipStream_t stream);
 
-// Fused scatter + K re-rotation of the n_jobs CopyJobs in `d`; kind is an
-// ElemKind. All jobs share `geom`.
-void launch_scatter_rotate(const DescArg& d, int n_jobs, int max_tiles, const RowGeom& geom, int kind, bool neox,
-                           const float* inv_freq, hipStream_t stream);
+// Fused scatter + K re-rotation of the CopyJobs in `d`, ordered by their tiles
+// (order_jobs); kind is an ElemKind. All jobs share `geom`.
+void launch_scatter_rotate(const DescArg& d, const JobClasses& classes, const RowGeom& geom, int kind,
+                           bool neox, const float* inv_freq, hipStream_t stream);
 
 // In-place K re-rotation over segments of tokens. `d` holds the n_segs
 // RopeSegs, then (at byte layer_off) the n_layers K base pointers. `path`:

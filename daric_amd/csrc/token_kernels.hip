@@ -29,7 +29,8 @@
 //    pages (5.9 TB/s), 16 KiB parts were no faster; part-major order within
 //    a job beat a job-minor order (5.3 TB/s);
 //  - scatter: job-minor order 6.4-6.6 TB/s against 5.5-5.9 TB/s part-major;
-//    it now takes the jobs' 128 KiB runs per XCD of JobRuns (kernels.h).
+//    it now takes the jobs' 128 KiB runs per XCD of JobRuns, the gather the
+//    order of JobRows (kernels.h).
 // The physical-span gather_pages of the same pages ran 6.2-6.4 TB/s, so the
 // transpose costs about 1%.
 //
@@ -51,7 +52,6 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kRowUnroll = 8;
 constexpr int kLdsUnits = 512;   // 16-byte units of LDS per workgroup (8 KiB)
-constexpr int kMaxY = 65535;
 constexpr int64_t kRunsFrom = 512ll << 20;   // JobRuns
 
 template <typename T>
@@ -84,24 +84,12 @@ __device__ __forceinline__ bool resolve_part(const TokenJob& j, int q, uint8_t*&
     return true;
 }
 
-// Workgroup -> (job, part). Gather: part-major within a job (grid.y = job), in
-// the order of `xr`; scatter: the order of `jr`.
-template <bool GATHER>
-__device__ __forceinline__ void block_part(const JobRuns& jr, const XcdRuns& xr, int& job, int& q) {
-    if (GATHER) {
-        job = static_cast<int>(blockIdx.y);
-        q = xr.map(static_cast<int>(blockIdx.x));
-    } else {
-        jr.at_block(blockIdx.x, job, q);
-    }
-}
-
-template <int VW, bool GATHER>
-__global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job0, JobRuns jr, XcdRuns xr) {
+template <int VW, bool GATHER, class Grid>
+__global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job0, Grid grid) {
     using T = typename Unit<VW>::T;
-    DARIC_ARGS_TOGETHER4(d.ptr, job0, jr.jobs.d, xr.full);
+    DARIC_ARGS_TOGETHER4(d.ptr, job0, grid.begin[1], grid.cls[0].div.d);
     int jb, q;
-    block_part<GATHER>(jr, xr, jb, q);
+    grid.at_block(blockIdx.x, jb, q);
     const TokenJob j = desc_load(desc_at<TokenJob>(d, 0) + job0 + jb);
     uint8_t *cache, *stage;
     int n_tok;
@@ -136,12 +124,12 @@ __global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job
 
 // Head-major pages: the cache side of a part is H runs of n_tok rows, each
 // run contiguous (token stride == row bytes, head stride == PS * row bytes).
-template <bool GATHER>
-__global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0, JobRuns jr, XcdRuns xr) {
+template <bool GATHER, class Grid>
+__global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0, Grid grid) {
     __shared__ u32x4 sm[kLdsUnits];
-    DARIC_ARGS_TOGETHER4(d.ptr, job0, jr.jobs.d, xr.full);
+    DARIC_ARGS_TOGETHER4(d.ptr, job0, grid.begin[1], grid.cls[0].div.d);
     int jb, q;
-    block_part<GATHER>(jr, xr, jb, q);
+    grid.at_block(blockIdx.x, jb, q);
     const TokenJob j = desc_load(desc_at<TokenJob>(d, 0) + job0 + jb);
     uint8_t *cache, *stage;
     int n_tok;
@@ -213,27 +201,20 @@ __global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0
 
 }  // namespace
 
-void launch_token_copy(const DescArg& d, int n_jobs, int max_parts, int64_t part_bytes, int vw,
+void launch_token_copy(const DescArg& d, const JobClasses& classes, int64_t part_bytes, int vw,
                        bool lds, bool gather, hipStream_t stream) {
-#define DARIC_TOK(G, GRID, JR, XR)                                                                     \
+#define DARIC_TOK(G, GRID)                                                                              \
     do {                                                                                               \
-        if (lds) DARIC_LAUNCH((token_lds_kernel<G>), GRID, kThreads, 0, stream, d, j0, JR, XR);          \
-        else if (vw == 16) DARIC_LAUNCH((token_rows_kernel<16, G>), GRID, kThreads, 0, stream, d, j0, JR, XR); \
-        else DARIC_LAUNCH((token_rows_kernel<1, G>), GRID, kThreads, 0, stream, d, j0, JR, XR);          \
+        if (lds) DARIC_LAUNCH((token_lds_kernel<G, GRID>), blocks, kThreads, 0, stream, d, j0, g);       \
+        else if (vw == 16) DARIC_LAUNCH((token_rows_kernel<16, G, GRID>), blocks, kThreads, 0, stream, d, j0, g); \
+        else DARIC_LAUNCH((token_rows_kernel<1, G, GRID>), blocks, kThreads, 0, stream, d, j0, g);       \
         check_launch(G ? "gather_tokens" : "scatter_tokens");                                         \
     } while (0)
-    if (!gather) {
-        for_job_runs(n_jobs, max_parts, part_bytes, kRunsFrom, [&](int j0, const JobRuns& jr, unsigned blocks) {
-            DARIC_TOK(false, blocks, jr, XcdRuns());
-        });
-        return;
-    }
-    const XcdRuns xr(max_parts, part_bytes);
-    for (int j0 = 0; j0 < n_jobs; j0 += kMaxY) {
-        const int nj = std::min(kMaxY, n_jobs - j0);
-        const dim3 grid(static_cast<unsigned>(max_parts), static_cast<unsigned>(nj));
-        DARIC_TOK(true, grid, JobRuns(), xr);
-    }
+    if (gather)
+        for_job_rows(classes, 1, part_bytes, [&](int j0, const JobRows& g, unsigned blocks) { DARIC_TOK(true, JobRows); });
+    else
+        for_job_runs(classes, 1, part_bytes, kRunsFrom,
+                     [&](int j0, const JobRuns& g, unsigned blocks) { DARIC_TOK(false, JobRuns); });
 #undef DARIC_TOK
 }
 

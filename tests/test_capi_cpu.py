@@ -512,13 +512,23 @@ def test_layer_minor_grid_covers_every_pair_once(hosttest, n_layers, n_items, la
     assert hosttest.daric_hosttest_layer_minor(n_layers, n_items) == launches
 
 
+def job_grid(hosttest, gather, tiles, parts, unit_bytes, runs_from=0):
+    t = np.asarray(tiles, dtype=np.int64)
+    log2_run, idle = ctypes.c_int32(-1), ctypes.c_int64(-1)
+    hosttest.daric_hosttest_job_grid.restype = ctypes.c_int64
+    launches = hosttest.daric_hosttest_job_grid(
+        gather, ctypes.c_void_p(t.ctypes.data), ctypes.c_int64(t.size), ctypes.c_int64(parts),
+        ctypes.c_int64(unit_bytes), ctypes.c_int64(runs_from), ctypes.byref(log2_run), ctypes.byref(idle))
+    return launches, log2_run.value, idle.value
+
+
 # (jobs, units, unit bytes, launches, log2 run): 256 and 1280 jobs of 16 KiB
 # parts, 8 KiB parts, jobs and units that divide nothing, calls too small for
 # whole runs, units past 128 KiB, and grids past 2^24 - 1 blocks.
 @pytest.mark.parametrize("n_jobs,units,unit_bytes,launches,log2_run", [
     (256, 256, 16384, 1, 3), (1280, 256, 16384, 1, 3), (32, 2049, 8192, 1, 4), (7, 333, 8192, 1, 4),
     (61, 97, 9216, 1, 3), (1, 1, 16384, 1, 0), (3, 5, 16384, 1, 0), (9, 100, 16384, 1, 2),
-    (2, 70, 512, 1, 0), (13, 40, 1 << 18, 1, 0), (2, (1 << 24) - 1, 16384, 2, 0), (70_001, 300, 16384, 2, 3),
+    (2, 70, 512, 1, 0), (13, 40, 1 << 18, 1, 0), (2, (1 << 24) - 9, 16384, 2, 0), (70_001, 300, 16384, 2, 3),
     (1, (1 << 24) - 9, 16384, 1, 0),
 ])
 def test_job_runs_grid_covers_every_unit_once(hosttest, n_jobs, units, unit_bytes, launches, log2_run):
@@ -528,7 +538,28 @@ def test_job_runs_grid_covers_every_unit_once(hosttest, n_jobs, units, unit_byte
     runs_from bytes."""
     total = n_jobs * units * unit_bytes
     for runs_from, want in ((total, log2_run), (total + 1, 0)):
-        got = ctypes.c_int32(-1)
-        assert hosttest.daric_hosttest_job_runs(n_jobs, ctypes.c_int64(units), ctypes.c_int64(unit_bytes),
-                                                ctypes.c_int64(runs_from), ctypes.byref(got)) == launches
-        assert got.value == want
+        assert job_grid(hosttest, 0, [units] * n_jobs, 1, unit_bytes, runs_from)[:2] == (launches, want)
+    assert job_grid(hosttest, 1, [units] * n_jobs, 1, unit_bytes)[0] >= 1
+
+
+# Job lengths (tiles), parts per tile, and the most idle blocks the grids may
+# have: uneven chunks over several layers, jobs without pages, one long job among
+# many short ones, more lengths than classes, very many lengths.
+@pytest.mark.parametrize("tiles,parts", [
+    ([126] * 48 + [192] * 48 + [8] * 48 + [256] * 48 + [42] * 48, 9),
+    ([5, 0, 7, 0, 5, 3, 0], 1), ([0, 0], 4), ([1], 1), ([4000] + [3] * 700, 2),
+    (list(range(1, 30)) * 3, 5), ([(i * 7919) % 1009 for i in range(1500)], 3), ([2, 1, 2, 1], 64),
+])
+def test_job_grids_of_uneven_jobs(hosttest, tiles, parts):
+    """Uneven jobs: both block orders still take every unit once, the jobs of a
+    class keep their order, and the idle blocks stay few: up to 8 per job's row
+    for the gathers, up to one run per job and class joined for the scatters."""
+    live = [t for t in tiles if t]
+    spread = 0                      # what joining lengths into 8 classes may add
+    if len(set(live)) > 8:
+        spread = len(live) * (max(live) - min(live)) * parts // 8
+    for gather in (0, 1):
+        launches, log2_run, idle = job_grid(hosttest, gather, tiles, parts, 8192)
+        assert launches == (1 if live else 0)
+        if live:
+            assert idle <= spread + len(live) * (8 if gather else 1 << log2_run) + 8 * (1 << log2_run)
