@@ -1141,6 +1141,18 @@ Chunks build_chunks(const daric_chunk* chunks, int64_t n, int64_t PS, int64_t bt
     return c;
 }
 
+// Sets each chunk's first batch of `rows` selected rows; returns all batches.
+int64_t merge_batches(std::vector<SelChunk>& chunks, int64_t kmax, int rows) {
+    int64_t n = 0;
+    for (SelChunk& c : chunks) {
+        DARIC_CHECK(n <= kIntMax, "too many selected rows in one call");
+        c.tile_begin = static_cast<int32_t>(n);
+        n += (std::min<int64_t>({c.k, c.n_tokens, kmax}) + rows - 1) / rows;
+    }
+    DARIC_CHECK(n <= kIntMax, "too many selected rows in one call");
+    return n;
+}
+
 void check_rows_tensor(const daric_tensor* x, const daric_tensor& layer, int64_t n_layers,
                        int64_t H, int64_t D, const char* what, int64_t* T) {
     check_tensor_struct(x, what);
@@ -1190,7 +1202,7 @@ int daric_kv_deviation(const daric_tensor* layers, int64_t n_layers, int page_fi
                     (g.sh * ces) % need == 0 && aligned(t.data, need),
                     "kv_deviation needs head_dim % 8 == 0 and aligned K rows");
         for (int64_t i = 1; i < n_layers; ++i) DARIC_CHECK(aligned(layers[i].data, need), "misaligned layer ", i);
-        Chunks c = build_chunks(chunks, n_chunks, g.PS, numel(*block_table), T, deviation_tile_tokens(ck));
+        Chunks c = build_chunks(chunks, n_chunks, g.PS, numel(*block_table), T, deviation_tile_tokens(ck, g));
         if (c.tiles == 0) return;
         DARIC_CHECK(c.tiles <= kMaxTiles, "too many tokens in one kv_deviation call");
         DeviceGuard guard(t.device);
@@ -1299,6 +1311,7 @@ int daric_merge_rows(const daric_tensor* layers, int64_t n_layers, int page_firs
         // index slots): no launch, so empty k_new / v_new (whose data pointer
         // may be null) are never read.
         if (kmax == 0 || T == 0 || c.max_k == 0) return;
+        const int64_t batches = merge_batches(c.v, kmax, merge_rows_per_block(g, t.elem_size, quant));
         DeviceGuard guard(t.device);
         const hipStream_t st = as_stream(stream);
         const size_t cb = c.v.size() * sizeof(SelChunk);
@@ -1307,11 +1320,11 @@ int daric_merge_rows(const daric_tensor* layers, int64_t n_layers, int page_firs
         const auto ptrs = layer_ptrs(layers, n_layers);
         std::memcpy(blob.data() + cb, ptrs.data(), n_layers * sizeof(uint8_t*));
         DescHandOver ho(t.device, blob.data(), blob.size(), st);
-        launch_merge(ho.arg(), static_cast<int>(cb), static_cast<int>(n_layers), g, t.elem_size,
+        launch_merge(ho.arg(), 0, static_cast<int>(cb), static_cast<int>(n_layers), g, t.elem_size,
                      static_cast<const int32_t*>(block_table->data),
                      static_cast<const uint8_t*>(k_new->data),
                      g.v_off >= 0 ? static_cast<const uint8_t*>(v_new->data) : nullptr, T,
-                     static_cast<int>(n_chunks), static_cast<const int32_t*>(sel_idx->data),
+                     static_cast<int>(n_chunks), batches, static_cast<const int32_t*>(sel_idx->data),
                      static_cast<int>(kmax), quant ? nk : -1,
                      quant ? static_cast<const float*>(k_scales->data) : nullptr,
                      quant && g.v_off >= 0 ? static_cast<const float*>(v_scales->data) : nullptr, st);
@@ -1385,17 +1398,29 @@ int daric_select_merge(const daric_tensor* layers, int64_t n_layers, int page_fi
                     sel_idx->sizes[1] == n_chunks && is_contiguous(*sel_idx),
                     "sel_idx must be a contiguous int32 [n_layers, n_chunks, kmax] tensor");
         const int64_t kmax = sel_idx->sizes[2];
-        Chunks c = build_chunks(chunks, n_chunks, g.PS, numel(*block_table), T, deviation_tile_tokens(ck));
+        Chunks c = build_chunks(chunks, n_chunks, g.PS, numel(*block_table), T, deviation_tile_tokens(ck, g));
         DARIC_CHECK(c.max_k <= kmax, "sel_idx kmax (", kmax, ") is smaller than a chunk's k (", c.max_k, ")");
         DARIC_CHECK(c.tiles <= kMaxTiles && n_chunks <= kMaxTiles, "too many tokens in one select_merge call");
         if (c.tiles == 0 && kmax == 0) return;   // no tokens to read, no index rows to fill
         DeviceGuard guard(t.device);
         const hipStream_t st = as_stream(stream);
         const size_t cb = c.v.size() * sizeof(SelChunk);
-        std::vector<uint8_t> blob(cb + n_layers * sizeof(uint8_t*));
+        const bool fused = kmax > 0 && select_merge_fits(g, t.elem_size, quant, c.max_tokens, kmax, one_pass);
+        // The merge kernel has its own batches of the chunks: beside the chunks
+        // where they travel through the ring anyway, in a second argument block
+        // where that keeps both inline.
+        const bool merges = !fused && kmax > 0 && c.max_k > 0;
+        const size_t layers_end = cb + static_cast<size_t>(n_layers) * sizeof(uint8_t*);
+        const size_t chunks2 = (layers_end + 15) / 16 * 16;
+        const bool both = merges && (chunks2 + cb <= static_cast<size_t>(kInlineDescBytes) ||
+                                     layers_end > static_cast<size_t>(kInlineDescBytes));
+        std::vector<uint8_t> blob(both ? chunks2 + cb : layers_end);
         std::memcpy(blob.data(), c.v.data(), cb);
         const auto ptrs = layer_ptrs(layers, n_layers);
         std::memcpy(blob.data() + cb, ptrs.data(), n_layers * sizeof(uint8_t*));
+        int64_t batches = 0;
+        if (merges) batches = merge_batches(c.v, kmax, merge_rows_per_block(g, t.elem_size, quant));
+        if (both) std::memcpy(blob.data() + chunks2, c.v.data(), cb);
         DescHandOver ho(t.device, blob.data(), blob.size(), st);
         const float* ksc = quant ? static_cast<const float*>(k_scales->data) : nullptr;
         const float* vsc = quant && g.v_off >= 0 ? static_cast<const float*>(v_scales->data) : nullptr;
@@ -1404,7 +1429,7 @@ int daric_select_merge(const daric_tensor* layers, int64_t n_layers, int page_fi
         const auto* kn = static_cast<const uint8_t*>(k_new->data);
         const auto* vn = g.v_off >= 0 ? static_cast<const uint8_t*>(v_new->data) : nullptr;
         const auto* btp = static_cast<const int32_t*>(block_table->data);
-        if (kmax > 0 && select_merge_fits(g, t.elem_size, quant, c.max_tokens, kmax, one_pass)) {
+        if (fused) {
             // the keys by the deviation kernel (unless given, or one_pass), then
             // one workgroup per (layer, chunk) for its top-k and merge
             if (!keys_ready && !one_pass && c.tiles > 0)
@@ -1424,9 +1449,19 @@ int daric_select_merge(const daric_tensor* layers, int64_t n_layers, int page_fi
         if (kmax == 0) return;
         launch_topk(kd, static_cast<int>(n_layers), T, ho.arg(), static_cast<int>(n_chunks),
                     static_cast<int>(std::max<int64_t>(c.max_tokens, 1)), sd, static_cast<int>(kmax), st);
-        if (c.max_k == 0) return;
-        launch_merge(ho.arg(), static_cast<int>(cb), static_cast<int>(n_layers), g, t.elem_size, btp, kn, vn, T,
-                     static_cast<int>(n_chunks), sd, static_cast<int>(kmax), quant ? nk : -1, ksc, vsc, st);
+        if (!merges) return;
+        const auto merge = [&](const DescArg& arg, size_t chunk_off) {
+            launch_merge(arg, static_cast<int>(chunk_off), static_cast<int>(cb), static_cast<int>(n_layers), g,
+                         t.elem_size, btp, kn, vn, T, static_cast<int>(n_chunks), batches, sd, static_cast<int>(kmax),
+                         quant ? nk : -1, ksc, vsc, st);
+        };
+        if (both) {
+            merge(ho.arg(), chunks2);
+        } else {
+            std::memcpy(blob.data(), c.v.data(), cb);
+            DescHandOver ho2(t.device, blob.data(), blob.size(), st);   // inline: copied by value
+            merge(ho2.arg(), 0);
+        }
     });
 }
 

@@ -460,7 +460,7 @@ void launch_rerotate_inplace(const DescArg& d, int layer_off, int n_layers, cons
 
 // Selection kernels. deviation_tile_tokens: tokens per deviation workgroup
 // (the tiling launch_deviation expects in SelChunk::tile_begin).
-int deviation_tile_tokens(int cache_kind);
+int deviation_tile_tokens(int cache_kind, const KVGeom& g);
 // Selection launchers: `d` holds the n_chunks SelChunks, then (deviation and
 // merge, at byte layer_off) the n_layers layer base pointers.
 void launch_deviation(const DescArg& d, int layer_off, int n_layers, const KVGeom& g, int cache_kind,
@@ -469,16 +469,18 @@ void launch_deviation(const DescArg& d, int layer_off, int n_layers, const KVGeo
                       const float* k_scales, float* keys, hipStream_t stream);
 void launch_topk(const float* keys, int n_layers, int64_t T, const DescArg& d,
                  int n_chunks, int max_tokens, int32_t* out_idx, int kmax, hipStream_t stream);
-// merge: quant_from is -1 (rows are copied as bytes) or the ElemKind of
+// merge: the SelChunks at byte chunk_off have their first batch of
+// merge_rows_per_block selected rows in tile_begin, n_batches in all. quant_from is -1 (rows are copied as bytes) or the ElemKind of
 // bf16 / fp16 rows quantised into an e4m3 cache with the [n_layers, H] fp32
 // k_scales / v_scales. merge_fits_rows: whether the row kernel takes the
 // geometry (required for quantising); merge_max_row_bytes: the most bytes of
 // recomputed K+V values per token it takes.
 bool merge_fits_rows(const KVGeom& g, int elem_size, bool quant);
 int64_t merge_max_row_bytes();
-void launch_merge(const DescArg& d, int layer_off, int n_layers, const KVGeom& g, int elem_size,
+int merge_rows_per_block(const KVGeom& g, int elem_size, bool quant);
+void launch_merge(const DescArg& d, int chunk_off, int layer_off, int n_layers, const KVGeom& g, int elem_size,
                   const int32_t* block_table, const uint8_t* k_new, const uint8_t* v_new,
-                  int64_t T, int n_chunks, const int32_t* sel_idx, int kmax, int quant_from,
+                  int64_t T, int n_chunks, int64_t n_batches, const int32_t* sel_idx, int kmax, int quant_from,
                   const float* k_scales, const float* v_scales, hipStream_t stream);
 // Fused selection, one workgroup per (layer, chunk): top-k on the chunk's
 // keys held in LDS and the merge of its selected rows, with (with_keys) or

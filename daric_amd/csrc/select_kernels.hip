@@ -26,13 +26,12 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-// Tokens per wavefront in the deviation kernel: 8 for 16-bit caches (16 loads
+// Tokens a lane group sums in the deviation kernel: 8 for 16-bit caches (16 loads
 // of 16 bytes in flight per lane; 3-4% faster than 4 at config 3), 4 for fp8
 // caches, where the 8-token form measured slower (config 5).
-template <int CK> constexpr int dev_tok_per_wave() { return CK == kE4M3 ? 4 : 8; }
+template <int CK> constexpr int dev_tok_per_group() { return CK == kE4M3 ? 4 : 8; }
 constexpr int kMergeTok = 8;                       // selected tokens per merge workgroup
 constexpr int kMaxGridYZ = 65535;                  // grid.y / grid.z limit; larger counts are sliced
-constexpr int kTopkLdsTokens = 8192;               // top-k keys staged in LDS up to this chunk length
 
 // 8 elements: 16 bytes for 2-byte types, 8 bytes for fp8. Loaded raw (so a
 // lane keeps few registers per load in flight) and converted when summed.
@@ -76,26 +75,30 @@ __device__ __forceinline__ void unpack8(const Raw8<KIND>& r, float* x, float sca
     }
 }
 
-// Keys of tokens j0 .. j0 + TPW - 1 of chunk c in layer l, summed by one
-// wavefront in the fixed order above; the butterfly leaves every key in every
-// lane. A token past the chunk's end, or whose block id lies outside
-// [0, num_blocks), is not read and gets key 0; a NaN key is 0x7FC00000.
-template <int CK, int NK, int TPW>
-__device__ __forceinline__ void wave_keys(const SelChunk& c, int j0, int lane, const KVGeom& g,
-                                          const uint8_t* __restrict__ base, const int32_t* __restrict__ bt,
-                                          const uint8_t* __restrict__ k_new, int64_t T, int l,
-                                          const float* __restrict__ ksc, float* key) {
+// Keys of tokens of chunk c in layer l in the fixed order above. A group of G
+// lanes sums TPG consecutive tokens, the first of them j0. G is 64, or the power
+// of two that holds a token's vectors where they are fewer (heads split over
+// GPUs, small models): the lanes of the fixed order that have no vector add
+// +0 to sums that are not -0, so leaving them out gives the same bits, and a
+// wavefront's loads serve 64 / G times the tokens. The butterfly leaves a key in
+// every lane of its group. A token past the chunk's end, or whose block id lies
+// outside [0, num_blocks), is not read and gets key 0; a NaN key is 0x7FC00000.
+template <int CK, int NK, int TPG, int G>
+__device__ __forceinline__ void group_keys(const SelChunk& c, int j0, int sub, const KVGeom& g,
+                                           const uint8_t* __restrict__ base, const int32_t* __restrict__ bt,
+                                           const uint8_t* __restrict__ k_new, int64_t T, int l,
+                                           const float* __restrict__ ksc, float* key) {
 #pragma clang fp contract(off)
     constexpr int CES = CK == kE4M3 ? 1 : 2;
     const int N = g.H * g.D;
     const int n_vec = N >> 3;
-    const int rounds = (n_vec + 63) >> 6;
+    const int rounds = G == 64 ? (n_vec + 63) >> 6 : 1;
 
-    int64_t cache_row[TPW];
-    const uint8_t* new_row[TPW];
-    bool valid[TPW];
+    int64_t cache_row[TPG];
+    const uint8_t* new_row[TPG];
+    bool valid[TPG];
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
+    for (int i = 0; i < TPG; ++i) {
         const int j = j0 + i;
         const int p = c.tok0 + j;                  // position in the chunk's block list
         int blk = -1;
@@ -105,27 +108,27 @@ __device__ __forceinline__ void wave_keys(const SelChunk& c, int j0, int lane, c
         new_row[i] = k_new + ((static_cast<int64_t>(l) * T + c.row_offset + j) * N) * 2;
     }
 
-    float acc[TPW];
+    float acc[TPG];
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) acc[i] = 0.0f;
+    for (int i = 0; i < TPG; ++i) acc[i] = 0.0f;
 
     for (int r = 0; r < rounds; ++r) {
-        const int v = r * 64 + lane;
+        const int v = r * 64 + sub;
         if (v >= n_vec) break;
         const int e0 = v << 3;
         const int h = e0 / g.D;
         const int d0 = e0 - h * g.D;
         const float scale = (CK == kE4M3 && ksc) ? ksc[h] : 1.0f;
-        Raw8<NK> ra[TPW];
-        Raw8<CK> rb[TPW];
+        Raw8<NK> ra[TPG];
+        Raw8<CK> rb[TPG];
 #pragma unroll
-        for (int i = 0; i < TPW; ++i) {
+        for (int i = 0; i < TPG; ++i) {
             if (!valid[i]) continue;
             ra[i] = load_raw8<NK>(new_row[i] + static_cast<int64_t>(e0) * 2);
             rb[i] = load_raw8<CK>(base + (cache_row[i] + static_cast<int64_t>(h) * g.sh + d0) * CES);
         }
 #pragma unroll
-        for (int i = 0; i < TPW; ++i) {
+        for (int i = 0; i < TPG; ++i) {
             if (!valid[i]) continue;
             float a[8], b[8];
             unpack8<NK>(ra[i], a, 1.0f);
@@ -139,17 +142,24 @@ __device__ __forceinline__ void wave_keys(const SelChunk& c, int j0, int lane, c
         }
     }
 #pragma unroll
-    for (int i = 0; i < TPW; ++i) {
+    for (int i = 0; i < TPG; ++i) {
         float s = acc[i];
 #pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) s = s + __shfl_xor(s, off, 64);
+        for (int off = G / 2; off >= 1; off >>= 1) s = s + __shfl_xor(s, off, 64);
         float k = valid[i] ? s : 0.0f;
         if (k != k) k = u2f(0x7fc00000u);
         key[i] = k;
     }
 }
 
-template <int CK, int NK>
+// Lanes per token: see group_keys.
+inline int dev_group(int n_vec) { return n_vec > 32 ? 64 : n_vec > 16 ? 32 : n_vec > 8 ? 16 : 8; }
+
+// Bound by HBM. G = 64 takes tokens of more than 256 values. A group of 16 lanes
+// against it, MI355X: 8 chunks of 700 tokens of 80 values in one layer 8.7 -> 5.7
+// us; with groups of 32 and 16 lanes the whole selection of 23 layers of 2 x 64
+// (16 x 5 chunks) went from 268 to 116 us, of 59 layers of 1 x 256 from 390 to 233.
+template <int CK, int NK, int G>
 __global__ __launch_bounds__(kThreads) void deviation_kernel(
     DescArg d, int layer_off, KVGeom g, const int32_t* __restrict__ bt,
     const uint8_t* __restrict__ k_new, int64_t T, int n_chunks,
@@ -159,18 +169,17 @@ __global__ __launch_bounds__(kThreads) void deviation_kernel(
     const int l = static_cast<int>(blockIdx.y) + l0;
     const int tile = static_cast<int>(blockIdx.x);
     const SelChunk c = desc_load(chunks + find_by_tile(chunks, n_chunks, tile));
-    const int lane = static_cast<int>(threadIdx.x) & 63;
-    const int wave = static_cast<int>(threadIdx.x) >> 6;
-    constexpr int kTokPerWave = dev_tok_per_wave<CK>();
-    constexpr int kTileTokens = kWaves * kTokPerWave;
-    const int j0 = (tile - c.tile_begin) * kTileTokens + wave * kTokPerWave;
+    const int sub = static_cast<int>(threadIdx.x) & (G - 1);
+    const int group = static_cast<int>(threadIdx.x) / G;
+    constexpr int kTok = dev_tok_per_group<CK>();
+    const int j0 = ((tile - c.tile_begin) * (kThreads / G) + group) * kTok;
     const float* ksc = k_scales ? k_scales + static_cast<int64_t>(l) * g.H : nullptr;
-    float key[kTokPerWave];
-    wave_keys<CK, NK, kTokPerWave>(c, j0, lane, g, layers[l], bt, k_new, T, l, ksc, key);
+    float key[kTok];
+    group_keys<CK, NK, kTok, G>(c, j0, sub, g, layers[l], bt, k_new, T, l, ksc, key);
 #pragma unroll
-    for (int i = 0; i < kTokPerWave; ++i) {
+    for (int i = 0; i < kTok; ++i) {
         const int j = j0 + i;
-        if (lane == 0 && j < c.n_tokens) keys[static_cast<int64_t>(l) * T + c.row_offset + j] = key[i];
+        if (sub == i % G && j < c.n_tokens) keys[static_cast<int64_t>(l) * T + c.row_offset + j] = key[i];
     }
 }
 
@@ -180,140 +189,194 @@ __device__ __forceinline__ uint32_t order_key(float f) {
     return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
 }
 
-// Exclusive prefix count of `flag` over the workgroup; *total gets the sum.
-__device__ __forceinline__ int block_excl_count(bool flag, int* s_wave, int* total) {
-    const int lane = static_cast<int>(threadIdx.x) & 63;
-    const int wave = static_cast<int>(threadIdx.x) >> 6;
-    const unsigned long long m = __ballot(flag);
-    const int below = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) s_wave[wave] = __popcll(m);
-    __syncthreads();
-    int before = 0, sum = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; ++w) {
-        const int cnt = s_wave[w];
-        before += w < wave ? cnt : 0;
-        sum += cnt;
+// Per-chunk top-k by a workgroup of T lanes: the k largest of n order keys, ties
+// to the lower index, written in ascending index order to orow[0 .. k-1] (when
+// not null) and, when s_sel is not null, to the LDS array s_sel (visible to the
+// other lanes after the caller's next barrier).
+//
+// Bound by latency: a chain of passes with barriers between them, so the passes
+// are few and each pass is short. Wavefront w takes the consecutive keys of
+// slots [w * slots, (w + 1) * slots) of 64, slot by slot, and holds them in
+// registers (KPT slots; KPT = 0: it reads them again in each pass, for chunks
+// longer than any register file). Radix passes find the k-th largest key: three
+// of 11, 11 and 10 bits, or for a single wavefront, which would spend itself on
+// 2048 bins, four of 8. A pass whose digit holds exactly the keys still wanted
+// is the last. Lanes add to the LDS histogram one by one, except where all keys
+// of a wavefront share the digit (ties, zeros), which one lane adds. The last
+// step needs one barrier: the wavefronts' counts give each its place in the
+// output.
+// Against 256 lanes with four 8-bit passes over keys in LDS (from 8192 tokens,
+// in memory), MI355X, 15% of the tokens selected: one chunk of 500 tokens 6.0 ->
+// 4.6 us, 16 of 5000 29.2 -> 9.5 us, one of 12000 78 -> 18 us, 6 of 30000 194 ->
+// 36 us, 6144 of 512 31.2 -> 23.6 us; all keys equal 6-440 -> 6-94 us.
+template <int T>
+struct TopkLds {
+    static constexpr int kBits = T == 64 ? 8 : 11;
+    static constexpr int kBins = 1 << kBits;
+    static constexpr int kPerLane = kBins / T;
+    // Bin x lies at (x % kPerLane) * T + x / kPerLane, so that the lanes, which
+    // sum kPerLane neighbouring bins each, read consecutive words.
+    static __device__ __forceinline__ uint32_t at(uint32_t x) {
+        return (x % kPerLane) * T + x / kPerLane;
     }
-    __syncthreads();
-    *total = sum;
-    return before + below;
-}
+    uint32_t hist[kBins];
+    uint32_t wave_a[T / 64], wave_b[T / 64];
+    uint32_t digit, above, count;
+};
 
-// LDS_KEYS: the chunk's order keys are staged in LDS (chunks of at most
-// kTopkLdsTokens tokens); otherwise every pass reads them from global memory,
-// where a chunk's keys (4 bytes per token) stay in L2 across the five passes.
-// Per-chunk top-k by the workgroup (kThreads lanes): the k largest of the n
-// order keys key_at(0 .. n-1), ties to the lower index, written in ascending
-// index order to orow[0 .. k-1] (when not null) and, when s_sel is not null,
-// to the LDS array s_sel (visible to the other lanes after the caller's next
-// barrier). Four
-// 8-bit radix passes over LDS histograms find the k-th largest key.
-template <typename KeyAt>
-__device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* __restrict__ orow,
-                                           int32_t* s_sel, uint32_t* hist, uint32_t* s_digit,
-                                           uint32_t* s_above, int* s_wave) {
+template <int T, int KPT, typename KeyAt>
+__device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* __restrict__ orow, int32_t* s_sel,
+                                           TopkLds<T>& sm) {
+    constexpr int W = T / 64;
+    using Lds = TopkLds<T>;
+    constexpr int BPT = Lds::kPerLane;
+    constexpr int R = KPT > 0 ? KPT : 1;
     const int tid = static_cast<int>(threadIdx.x);
-    uint32_t prefix = 0, mask = 0, krem = static_cast<uint32_t>(k);
-    for (int pass = 0; pass < 4; ++pass) {
-        const int shift = 24 - 8 * pass;
-        hist[tid] = 0;
-        __syncthreads();
-        // Lanes of a wavefront whose keys share a digit are found with eight
-        // ballots, and one of them adds the group's count: one LDS atomic per
-        // distinct digit instead of up to 64 colliding ones (the leading
-        // digits of one chunk's keys are nearly all equal).
-        for (int b = 0; b < n; b += kThreads) {
-            const int i = b + tid;
-            const uint32_t key = i < n ? key_at(i) : 0u;
-            const bool act = i < n && (key & mask) == prefix;
-            const uint32_t dig = (key >> shift) & 255u;
-            unsigned long long same = __ballot(act);
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int slots = (n + T - 1) / T;
+    const int i0 = wave * slots * 64 + lane;
+    uint32_t key[R];
+    if constexpr (KPT > 0) {
 #pragma unroll
-            for (int bit = 0; bit < 8; ++bit) {
-                const unsigned long long ones = __ballot((dig >> bit) & 1u);
-                same &= ((dig >> bit) & 1u) ? ones : ~ones;
-            }
-            if (act && (tid & 63) == __ffsll(static_cast<long long>(same)) - 1)
-                atomicAdd(&hist[dig], static_cast<uint32_t>(__popcll(same)));
+        for (int s = 0; s < KPT; ++s) {
+            key[s] = 0;
+            if (s < slots && i0 + s * 64 < n) key[s] = key_at(i0 + s * 64);
         }
+    }
+    // f(slot, key, whether there is one) for the wavefront's slots
+    const auto each = [&](auto&& f) {
+        if constexpr (KPT > 0) {
+#pragma unroll
+            for (int s = 0; s < KPT; ++s)
+                if (s < slots) f(s, key[s], i0 + s * 64 < n);
+        } else {
+            for (int s = 0; s < slots; ++s) {
+                const bool in = i0 + s * 64 < n;
+                f(s, in ? key_at(i0 + s * 64) : 0u, in);
+            }
+        }
+    };
+#pragma unroll
+    for (int b = 0; b < BPT; ++b) sm.hist[b * T + tid] = 0;
+    __syncthreads();
+
+    uint32_t prefix = 0, mask = 0, krem = static_cast<uint32_t>(k);
+    bool whole = k >= n;      // every key from `prefix` up is taken
+    int left_bits = 32;
+    for (int pass = 0; left_bits > 0 && !whole; ++pass) {
+        const int width = min(left_bits, Lds::kBits);
+        const int shift = left_bits - width;
+        left_bits = shift;
+        const uint32_t dmask = (1u << width) - 1u;
+        each([&](int, uint32_t v, bool in) {
+            const bool act = in && (v & mask) == prefix;
+            const uint32_t dig = (v >> shift) & dmask;
+            const unsigned long long some = __ballot(act);
+            if (some == 0) return;
+            const int lead = __ffsll(static_cast<long long>(some)) - 1;
+            const uint32_t d0 = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(dig), lead));
+            if (__ballot(act && dig != d0) == 0) {
+                if (lane == lead) atomicAdd(&sm.hist[Lds::at(d0)], static_cast<uint32_t>(__popcll(some)));
+            } else if (act) {
+                atomicAdd(&sm.hist[Lds::at(dig)], 1u);
+            }
+        });
         __syncthreads();
-        // suffix sums over digits (from 255 down): thread t holds digit 255 - t
-        const uint32_t cnt = hist[255 - tid];
-        uint32_t incl = cnt;
-        const int lane = tid & 63;
-        const int wave = tid >> 6;
+        // Lane t sums bins [kBins - (t + 1) * BPT, kBins - t * BPT), highest first,
+        // and leaves them empty for the next pass.
+        uint32_t c[BPT], mine = 0;
+#pragma unroll
+        for (int b = 0; b < BPT; ++b) {
+            const int at = (BPT - 1 - b) * T + (T - 1 - tid);
+            c[b] = sm.hist[at];
+            sm.hist[at] = 0;
+            mine += c[b];
+        }
+        uint32_t incl = mine;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
             const uint32_t o = __shfl_up(incl, off, 64);
             if (lane >= off) incl += o;
         }
-        if (lane == 63) s_wave[wave] = static_cast<int>(incl);
-        __syncthreads();
-        uint32_t before = 0;
+        if constexpr (W > 1) {
+            if (lane == 63) sm.wave_a[wave] = incl;
+            __syncthreads();
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) before += w < wave ? static_cast<uint32_t>(s_wave[w]) : 0u;
-        incl += before;
-        const uint32_t excl = incl - cnt;  // keys with a larger digit
-        if (excl < krem && incl >= krem) {
-            *s_digit = static_cast<uint32_t>(255 - tid);
-            *s_above = excl;
+            for (int w = 0; w < W; ++w) incl += w < wave ? sm.wave_a[w] : 0u;
+        }
+        uint32_t above = incl - mine;          // keys with a larger digit
+        if (above < krem && incl >= krem) {
+#pragma unroll
+            for (int b = 0; b < BPT; ++b) {
+                if (above < krem && above + c[b] >= krem) {
+                    sm.digit = static_cast<uint32_t>(Lds::kBins - 1 - tid * BPT - b);
+                    sm.above = above;
+                    sm.count = c[b];
+                }
+                above += c[b];
+            }
         }
         __syncthreads();
-        prefix |= *s_digit << shift;
-        mask |= 255u << shift;
-        krem -= *s_above;
-        __syncthreads();
+        prefix |= sm.digit << shift;
+        mask |= dmask << shift;
+        krem -= sm.above;
+        whole = sm.count == krem;
     }
-    // prefix is the k-th largest key; take every larger key and the first
-    // krem keys equal to it, in index order.
-    int running = 0, eq_seen = 0;
-    for (int b = 0; b < n; b += kThreads) {
-        const int i = b + tid;
-        const uint32_t key = i < n ? key_at(i) : 0u;
-        const bool gt = i < n && key > prefix;
-        const bool eq = i < n && key == prefix;
-        int eq_total, sel_total;
-        const int eq_rank = eq_seen + block_excl_count(eq, s_wave, &eq_total);
-        const bool sel = gt || (eq && eq_rank < static_cast<int>(krem));
-        const int pos = running + block_excl_count(sel, s_wave, &sel_total);
-        if (sel && pos < k) {
+    // Take every key with a larger prefix and, of those equal to it, all
+    // (whole) or the first krem in index order.
+    uint32_t n_gt = 0, n_eq = 0;
+    const auto over = [&](uint32_t v, bool in) { return in && (whole ? v >= prefix : v > prefix); };
+    each([&](int, uint32_t v, bool in) {
+        n_gt += static_cast<uint32_t>(__popcll(__ballot(over(v, in))));
+        n_eq += static_cast<uint32_t>(__popcll(__ballot(in && !whole && v == prefix)));
+    });
+    uint32_t gt = 0, eq = 0;                   // of the wavefronts before
+    if constexpr (W > 1) {
+        if (lane == 0) {
+            sm.wave_a[wave] = n_gt;
+            sm.wave_b[wave] = n_eq;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            gt += w < wave ? sm.wave_a[w] : 0u;
+            eq += w < wave ? sm.wave_b[w] : 0u;
+        }
+    }
+    const unsigned long long below = (1ull << lane) - 1ull;
+    each([&](int s, uint32_t v, bool in) {
+        const bool g = over(v, in), e = in && !whole && v == prefix;
+        const unsigned long long mg = __ballot(g), me = __ballot(e);
+        const uint32_t eq_rank = eq + static_cast<uint32_t>(__popcll(me & below));
+        const uint32_t pos = gt + static_cast<uint32_t>(__popcll(mg & below)) + min(eq_rank, krem);
+        if ((g || (e && eq_rank < krem)) && pos < static_cast<uint32_t>(k)) {
+            const int i = i0 + s * 64;
             if (orow != nullptr) orow[pos] = i;
             if (s_sel != nullptr) s_sel[pos] = i;
         }
-        running += sel_total;
-        eq_seen += eq_total;
-    }
+        gt += static_cast<uint32_t>(__popcll(mg));
+        eq += static_cast<uint32_t>(__popcll(me));
+    });
 }
 
-// LDS_KEYS: the chunk's order keys are staged in LDS (chunks of at most
-// kTopkLdsTokens tokens); otherwise every pass reads them from global memory,
-// where a chunk's keys (4 bytes per token) stay in L2 across the five passes.
-template <bool LDS_KEYS>
-__global__ __launch_bounds__(kThreads) void topk_kernel(const float* __restrict__ keys, int64_t T,
-                                                        DescArg d, int n_chunks,
-                                                        int32_t* __restrict__ out, int kmax, int l0) {
+// One workgroup per (layer, chunk). T and KPT by the longest chunk, see
+// launch_topk.
+template <int T, int KPT>
+__global__ __launch_bounds__(T) void topk_kernel(const float* __restrict__ keys, int64_t stride, DescArg d,
+                                                 int n_chunks, int32_t* __restrict__ out, int kmax, int l0) {
     const DescPtr<SelChunk> chunks = desc_at<SelChunk>(d, 0);
-    extern __shared__ uint32_t s_keys[];
-    __shared__ uint32_t hist[256];
-    __shared__ uint32_t s_digit, s_above;
-    __shared__ int s_wave[kWaves];
-
+    __shared__ TopkLds<T> sm;
     const int l = static_cast<int>(blockIdx.y) + l0;
     const int ci = static_cast<int>(blockIdx.x);
     const SelChunk c = desc_load(chunks + ci);
     const int n = c.n_tokens;
     const int k = min(max(c.k, 0), n);
     int32_t* __restrict__ orow = out + (static_cast<int64_t>(l) * n_chunks + ci) * kmax;
-    const int tid = static_cast<int>(threadIdx.x);
-
-    for (int i = k + tid; i < kmax; i += kThreads) orow[i] = -1;
+    for (int i = k + static_cast<int>(threadIdx.x); i < kmax; i += T) orow[i] = -1;
     if (k == 0) return;
-    const float* krow = keys + static_cast<int64_t>(l) * T + c.row_offset;
-    if (LDS_KEYS)
-        for (int i = tid; i < n; i += kThreads) s_keys[i] = order_key(krow[i]);
-    const auto key_at = [&](int i) -> uint32_t { return LDS_KEYS ? s_keys[i] : order_key(krow[i]); };
-    chunk_topk(key_at, n, k, orow, nullptr, hist, &s_digit, &s_above, s_wave);
+    const float* krow = keys + static_cast<int64_t>(l) * stride + c.row_offset;
+    chunk_topk<T, KPT>([&](int i) -> uint32_t { return order_key(krow[i]); }, n, k, orow, nullptr, sm);
 }
 
 template <int VW>
@@ -474,24 +537,28 @@ __device__ __forceinline__ void merge_units(
     }
 }
 
+// A chunk's row batches begin at its tile_begin: the chunks' counts differ (the
+// recompute policy gives a prompt's last document most of its budget), and a
+// grid of the largest count times the chunks left most workgroups idle (MI355X,
+// counts of 2% to 90% of 8 chunks of 3000 tokens, 22 layers of 4 x 96: 80 -> 60 us).
 template <int MODE, bool DENSE>
 __global__ __launch_bounds__(kMergeThreads) void merge_rows_kernel(
-    DescArg d, int layer_off, KVGeom g, int ces, const int32_t* __restrict__ bt,
+    DescArg d, int chunk_off, int layer_off, KVGeom g, int ces, const int32_t* __restrict__ bt,
     const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t T,
     int n_chunks, const int32_t* __restrict__ sel, int kmax, int tpb, int units,
     FastDiv d_tok_units, FastDiv d_upr, const float* __restrict__ k_scales,
-    const float* __restrict__ v_scales, LayerMinor lm, int64_t nbx) {
+    const float* __restrict__ v_scales, LayerMinor lm) {
     __shared__ int64_t s_src[kMergeMaxTok];   // byte offset of the token's recomputed rows (-1: skip)
     __shared__ int64_t s_dst[kMergeMaxTok];   // byte offset of the token's K row in the layer
-    const DescPtr<SelChunk> chunks = desc_at<SelChunk>(d, 0);
+    const DescPtr<SelChunk> chunks = desc_at<SelChunk>(d, chunk_off);
     const DescPtr<uint8_t*> layers = desc_at<uint8_t*>(d, layer_off);
     // work item = (chunk, row batch), the batches of a chunk consecutive
     int l;
     int64_t item;
     lm.at(l, item);
-    const int ci = static_cast<int>(item / nbx);
-    const int bx = static_cast<int>(item - static_cast<int64_t>(ci) * nbx);
+    const int ci = find_by_tile(chunks, n_chunks, static_cast<int>(item));
     const SelChunk c = desc_load(chunks + ci);
+    const int bx = static_cast<int>(item) - c.tile_begin;
     const int tid = static_cast<int>(threadIdx.x);
     const int ses = MODE == kMergeCopy ? ces : 2;                    // source element size
     const int64_t row_bytes = static_cast<int64_t>(g.H) * g.D * ses;
@@ -506,13 +573,14 @@ __global__ __launch_bounds__(kMergeThreads) void merge_rows_kernel(
 }
 
 // The whole selection of one (layer, chunk) in one workgroup: the chunk's
-// deviation keys (wave_keys, the fixed order of deviation_kernel; WITH_KEYS
-// false: read from `keys` instead), its top-k on the keys held in LDS
-// (chunk_topk), then the slots of all its selected tokens (merge_slot) and
-// the merge of their rows (merge_units). Keys and indices are written out as
-// kv_deviation and topk_per_chunk write them. Dynamic LDS (select_merge_lds):
-// n_max order keys, kmax selected indices, kmax source and kmax destination
-// offsets.
+// deviation keys (group_keys, the fixed order of deviation_kernel; WITH_KEYS
+// false: read from `keys` instead), its top-k (chunk_topk), then the slots of all
+// its selected tokens (merge_slot) and the merge of their rows (merge_units).
+// Keys and indices are written out as kv_deviation and topk_per_chunk write
+// them. Dynamic LDS (select_merge_lds): n_max order keys (WITH_KEYS), kmax
+// selected indices, kmax source and kmax destination offsets.
+constexpr int kFusedSlots = 8;                          // key slots per wavefront
+constexpr int kFusedMaxTokens = kThreads * kFusedSlots;
 template <int CK, int NK, int MODE, bool DENSE, bool WITH_KEYS>
 __global__ __launch_bounds__(kThreads) void select_merge_kernel(
     DescArg d, int layer_off, KVGeom g, int ces, const int32_t* __restrict__ bt,
@@ -521,9 +589,7 @@ __global__ __launch_bounds__(kThreads) void select_merge_kernel(
     int n_max, int units, FastDiv d_tok_units, FastDiv d_upr, const float* __restrict__ k_scales,
     const float* __restrict__ v_scales, LayerMinor lm) {
     extern __shared__ __align__(16) uint32_t s_dyn[];   // keys, indices, then 8-byte offsets
-    __shared__ uint32_t hist[256];
-    __shared__ uint32_t s_digit, s_above;
-    __shared__ int s_wave[kWaves];
+    __shared__ TopkLds<kThreads> sm;
     uint32_t* s_keys = s_dyn;
     int32_t* s_sel = reinterpret_cast<int32_t*>(s_dyn + n_max);
     int64_t* s_src = reinterpret_cast<int64_t*>(s_dyn + ((n_max + kmax + 1) & ~1));
@@ -536,20 +602,20 @@ __global__ __launch_bounds__(kThreads) void select_merge_kernel(
     const int ci = static_cast<int>(item);
     const SelChunk c = desc_load(chunks + ci);
     const int tid = static_cast<int>(threadIdx.x);
-    const int lane = tid & 63;
-    const int wave = tid >> 6;
     const int n = c.n_tokens;
     const int k = min(max(c.k, 0), n);
     uint8_t* __restrict__ base = layers[l];
     float* krow = keys + static_cast<int64_t>(l) * T + c.row_offset;
     if constexpr (WITH_KEYS) {
-        constexpr int TPW = dev_tok_per_wave<CK>();
+        constexpr int TPG = dev_tok_per_group<CK>();
+        const int lane = tid & 63;
+        const int wave = tid >> 6;
         const float* ksc = dev_scales ? dev_scales + static_cast<int64_t>(l) * g.H : nullptr;
-        for (int j0 = wave * TPW; j0 < n; j0 += kWaves * TPW) {
-            float key[TPW];
-            wave_keys<CK, NK, TPW>(c, j0, lane, g, base, bt, k_new, T, l, ksc, key);
+        for (int j0 = wave * TPG; j0 < n; j0 += kWaves * TPG) {
+            float key[TPG];
+            group_keys<CK, NK, TPG, 64>(c, j0, lane, g, base, bt, k_new, T, l, ksc, key);
 #pragma unroll
-            for (int i = 0; i < TPW; ++i) {
+            for (int i = 0; i < TPG; ++i) {
                 const int j = j0 + i;
                 if (lane == i && j < n) {
                     krow[j] = key[i];
@@ -557,15 +623,13 @@ __global__ __launch_bounds__(kThreads) void select_merge_kernel(
                 }
             }
         }
-    } else {
-        for (int i = tid; i < n; i += kThreads) s_keys[i] = order_key(krow[i]);
+        __syncthreads();
     }
     int32_t* __restrict__ orow = sel + (static_cast<int64_t>(l) * n_chunks + ci) * kmax;
     for (int i = k + tid; i < kmax; i += kThreads) orow[i] = -1;
     if (k == 0) return;
-    __syncthreads();
-    chunk_topk([&](int i) -> uint32_t { return s_keys[i]; }, n, k, orow, s_sel, hist, &s_digit, &s_above,
-               s_wave);
+    chunk_topk<kThreads, kFusedSlots>(
+        [&](int i) -> uint32_t { return WITH_KEYS ? s_keys[i] : order_key(krow[i]); }, n, k, orow, s_sel, sm);
     __syncthreads();
     const int ses = MODE == kMergeCopy ? ces : 2;
     const int64_t row_bytes = static_cast<int64_t>(g.H) * g.D * ses;
@@ -577,41 +641,49 @@ __global__ __launch_bounds__(kThreads) void select_merge_kernel(
 
 }  // namespace
 
-int deviation_tile_tokens(int cache_kind) {
-    return kWaves * (cache_kind == kE4M3 ? dev_tok_per_wave<kE4M3>() : dev_tok_per_wave<kBF16>());
+int deviation_tile_tokens(int cache_kind, const KVGeom& g) {
+    const int group = dev_group(g.H * g.D / 8);
+    return kThreads / group * (cache_kind == kE4M3 ? dev_tok_per_group<kE4M3>() : dev_tok_per_group<kBF16>());
 }
 
 void launch_deviation(const DescArg& d, int layer_off, int n_layers, const KVGeom& g, int cache_kind,
                       const int32_t* block_table, const uint8_t* k_new, int new_kind,
                       int64_t T, int n_chunks, int n_tiles,
                       const float* k_scales, float* keys, hipStream_t stream) {
+    const int group = dev_group(g.H * g.D / 8);
     for (int l0 = 0; l0 < n_layers; l0 += kMaxGridYZ) {
         const dim3 grid(static_cast<unsigned>(n_tiles), static_cast<unsigned>(std::min(kMaxGridYZ, n_layers - l0)));
-#define DARIC_DV(C, N) DARIC_LAUNCH((deviation_kernel<C, N>), grid, kThreads, 0, stream, d, layer_off, g, block_table, k_new, T, n_chunks, k_scales, keys, l0)
+#define DARIC_DV(C, N, G) DARIC_LAUNCH((deviation_kernel<C, N, G>), grid, kThreads, 0, stream, d, layer_off, g, block_table, k_new, T, n_chunks, k_scales, keys, l0)
+#define DARIC_DVG(C, N) do { if (group == 64) DARIC_DV(C, N, 64); else if (group == 32) DARIC_DV(C, N, 32); \
+                             else if (group == 16) DARIC_DV(C, N, 16); else DARIC_DV(C, N, 8); } while (0)
         if (new_kind == kBF16) {
-            if (cache_kind == kBF16) DARIC_DV(kBF16, kBF16);
-            else if (cache_kind == kF16) DARIC_DV(kF16, kBF16);
-            else DARIC_DV(kE4M3, kBF16);
+            if (cache_kind == kBF16) DARIC_DVG(kBF16, kBF16);
+            else if (cache_kind == kF16) DARIC_DVG(kF16, kBF16);
+            else DARIC_DVG(kE4M3, kBF16);
         } else {
-            if (cache_kind == kBF16) DARIC_DV(kBF16, kF16);
-            else if (cache_kind == kF16) DARIC_DV(kF16, kF16);
-            else DARIC_DV(kE4M3, kF16);
+            if (cache_kind == kBF16) DARIC_DVG(kBF16, kF16);
+            else if (cache_kind == kF16) DARIC_DVG(kF16, kF16);
+            else DARIC_DVG(kE4M3, kF16);
         }
+#undef DARIC_DVG
 #undef DARIC_DV
         check_launch("kv_deviation");
     }
 }
 
+// The fewest lanes whose registers hold the longest chunk's keys in a few slots:
+// more wavefronts only add to the barriers.
 void launch_topk(const float* keys, int n_layers, int64_t T, const DescArg& d,
                  int n_chunks, int max_tokens, int32_t* out_idx, int kmax, hipStream_t stream) {
-    const bool lds = max_tokens <= kTopkLdsTokens;
-    const size_t lds_bytes = lds ? static_cast<size_t>(max_tokens) * sizeof(uint32_t) : 0;
     for (int l0 = 0; l0 < n_layers; l0 += kMaxGridYZ) {
         const dim3 grid(static_cast<unsigned>(n_chunks), static_cast<unsigned>(std::min(kMaxGridYZ, n_layers - l0)));
-        if (lds)
-            DARIC_LAUNCH((topk_kernel<true>), grid, kThreads, lds_bytes, stream, keys, T, d, n_chunks, out_idx, kmax, l0);
-        else
-            DARIC_LAUNCH((topk_kernel<false>), grid, kThreads, 0, stream, keys, T, d, n_chunks, out_idx, kmax, l0);
+#define DARIC_TK(TH, KPT) DARIC_LAUNCH((topk_kernel<TH, KPT>), grid, TH, 0, stream, keys, T, d, n_chunks, out_idx, kmax, l0)
+        if (max_tokens <= 256) DARIC_TK(64, 4);
+        else if (max_tokens <= 2048) DARIC_TK(256, 8);
+        else if (max_tokens <= 8192) DARIC_TK(1024, 8);
+        else if (max_tokens <= 32768) DARIC_TK(1024, 32);
+        else DARIC_TK(1024, 0);
+#undef DARIC_TK
         check_launch("topk_per_chunk");
     }
 }
@@ -629,9 +701,15 @@ bool merge_fits_rows(const KVGeom& g, int elem_size, bool quant) {
 
 int64_t merge_max_row_bytes() { return static_cast<int64_t>(kMergeThreads) * kMergeUnits * 16; }
 
-void launch_merge(const DescArg& d, int layer_off, int n_layers, const KVGeom& g, int elem_size,
+int merge_rows_per_block(const KVGeom& g, int elem_size, bool quant) {
+    if (!merge_fits_rows(g, elem_size, quant)) return 1;
+    const int tok_units = (g.v_off >= 0 ? 2 : 1) * g.H * (g.D * (quant ? 2 : elem_size) / 16);
+    return std::min(kMergeMaxTok, std::max(1, kMergeThreads * kMergeUnits / tok_units));
+}
+
+void launch_merge(const DescArg& d, int chunk_off, int layer_off, int n_layers, const KVGeom& g, int elem_size,
                   const int32_t* block_table, const uint8_t* k_new, const uint8_t* v_new,
-                  int64_t T, int n_chunks, const int32_t* sel_idx, int kmax, int quant_from,
+                  int64_t T, int n_chunks, int64_t n_batches, const int32_t* sel_idx, int kmax, int quant_from,
                   const float* k_scales, const float* v_scales, hipStream_t stream) {
     const bool quant = quant_from >= 0;
     if (merge_fits_rows(g, elem_size, quant)) {
@@ -640,14 +718,13 @@ void launch_merge(const DescArg& d, int layer_off, int n_layers, const KVGeom& g
         const int upr = g.D * ses / 16;                              // source units per head row
         const int units = g.H * upr;                                 // per K (or V) token row
         const int tok_units = (g.v_off >= 0 ? 2 : 1) * units;
-        const int tpb = std::min(kMergeMaxTok, std::max(1, kMergeThreads * kMergeUnits / tok_units));
-        const int64_t nbx = (static_cast<int64_t>(kmax) + tpb - 1) / tpb;
+        const int tpb = merge_rows_per_block(g, elem_size, quant);
         const FastDiv dtu(static_cast<uint32_t>(tok_units)), dupr(static_cast<uint32_t>(upr));
         const bool dense = g.sh == g.D;
-        for_layer_minor(n_layers, nbx * n_chunks, [&](const LayerMinor& lm, unsigned blocks) {
-#define DARIC_MR(M, DN) DARIC_LAUNCH((merge_rows_kernel<M, DN>), blocks, kMergeThreads, 0, stream, d, layer_off, g, \
-                                     elem_size, block_table, k_new, v_new, T, n_chunks, sel_idx, kmax, tpb, units, \
-                                     dtu, dupr, k_scales, v_scales, lm, nbx)
+        for_layer_minor(n_layers, n_batches, [&](const LayerMinor& lm, unsigned blocks) {
+#define DARIC_MR(M, DN) DARIC_LAUNCH((merge_rows_kernel<M, DN>), blocks, kMergeThreads, 0, stream, d, chunk_off, \
+                                     layer_off, g, elem_size, block_table, k_new, v_new, T, n_chunks, sel_idx, kmax, \
+                                     tpb, units, dtu, dupr, k_scales, v_scales, lm)
             if (!quant) { if (dense) DARIC_MR(kMergeCopy, true); else DARIC_MR(kMergeCopy, false); }
             else if (quant_from == kBF16) { if (dense) DARIC_MR(kMergeFromBF16, true); else DARIC_MR(kMergeFromBF16, false); }
             else { if (dense) DARIC_MR(kMergeFromF16, true); else DARIC_MR(kMergeFromF16, false); }
@@ -677,14 +754,15 @@ void launch_merge(const DescArg& d, int layer_off, int n_layers, const KVGeom& g
     }
 }
 
-// Dynamic LDS of the fused kernel: keys and indices (4 bytes each), then the
-// source and destination offsets of the selected tokens (8 bytes each).
-size_t select_merge_lds(int64_t max_tokens, int64_t kmax) {
-    const int64_t n = std::max<int64_t>(max_tokens, 1), k = std::max<int64_t>(kmax, 1);
+// Dynamic LDS of the fused kernel: keys (one pass only) and indices (4 bytes
+// each), then the source and destination offsets of the selected tokens (8 bytes
+// each).
+size_t select_merge_lds(int64_t max_tokens, int64_t kmax, bool one_pass) {
+    const int64_t n = one_pass ? std::max<int64_t>(max_tokens, 1) : 0, k = std::max<int64_t>(kmax, 1);
     return static_cast<size_t>(((n + k + 1) & ~int64_t(1)) * 4 + 2 * k * 8);
 }
 
-constexpr size_t kSelectMergeMaxLds = 48 * 1024;
+constexpr size_t kSelectMergeMaxLds = 40 * 1024;   // beside the 8 KiB of the top-k
 // A fused workgroup merges its chunk's selected rows alone, in rounds of
 // kMergeThreads x kMergeUnits 16-byte units. Up to this many rounds per chunk
 // the fused top-k + merge beat topk_kernel + merge_rows_kernel on MI355X
@@ -696,8 +774,8 @@ constexpr int64_t kFusedMaxRounds = 12;
 
 bool select_merge_fits(const KVGeom& g, int elem_size, bool quant, int64_t max_tokens, int64_t kmax,
                        bool one_pass) {
-    if (!merge_fits_rows(g, elem_size, quant) || max_tokens > kTopkLdsTokens ||
-        select_merge_lds(max_tokens, kmax) > kSelectMergeMaxLds)
+    if (!merge_fits_rows(g, elem_size, quant) || max_tokens > kFusedMaxTokens ||
+        select_merge_lds(max_tokens, kmax, one_pass) > kSelectMergeMaxLds)
         return false;
     const int ses = quant ? 2 : elem_size;
     const int64_t tok_units = static_cast<int64_t>(g.v_off >= 0 ? 2 : 1) * g.H * (g.D * ses / 16);
@@ -717,8 +795,8 @@ void launch_select_merge(const DescArg& d, int layer_off, int n_layers, const KV
     const int tok_units = (g.v_off >= 0 ? 2 : 1) * units;
     const FastDiv dtu(static_cast<uint32_t>(tok_units)), dupr(static_cast<uint32_t>(upr));
     const bool dense = g.sh == g.D;
-    const int n_max = std::max(max_tokens, 1);
-    const size_t lds = select_merge_lds(max_tokens, kmax);
+    const int n_max = with_keys ? std::max(max_tokens, 1) : 0;
+    const size_t lds = select_merge_lds(max_tokens, kmax, with_keys);
     // deviation scales: per-head K scales of an fp8 cache (the quantising
     // merge's K scales are the same ones)
     const float* dev_scales = cache_kind == kE4M3 ? k_scales : nullptr;

@@ -331,8 +331,8 @@ int daric_kv_deviation(const daric_tensor* layers, int64_t n_layers, int page_fi
  * (ties: lower token index first) and write their chunk-local token indices
  * in ascending order to out_idx[l, c, 0:k]; slots k..kmax-1 are set to -1.
  * keys: [n_layers, T] fp32; out_idx: [n_layers, n_chunks, kmax] int32.
- * Chunks of any length: keys of chunks up to 8192 tokens are staged in LDS,
- * longer chunks are read from global memory in each radix pass. */
+ * Chunks of any length: a workgroup holds the keys of chunks up to 32768 tokens
+ * in registers, longer chunks are read from memory in each radix pass. */
 int daric_topk_per_chunk(const daric_tensor* keys, const daric_chunk* chunks,
                          int64_t n_chunks, daric_tensor* out_idx, uint64_t stream);
 
@@ -364,8 +364,8 @@ int daric_merge_rows(const daric_tensor* layers, int64_t n_layers, int page_firs
  * dequantise the cached K for the keys and quantise the merged K rows) and
  * v_scales the V scales; k_new and v_new are bfloat16 or float16 rows. Other
  * caches take rows of their own type and NULL scales.
- * Where every chunk has at most 8192 tokens, its keys and kmax row slots fit
- * in 48 KiB of LDS, the merge kernel takes the rows, and kmax selected K and
+ * Where every chunk has at most 2048 tokens, its keys and kmax row slots fit
+ * in 40 KiB of LDS, the merge kernel takes the rows, and kmax selected K and
  * V rows make at most 12 rounds of 2048 16-byte units (e.g. 77 of 512 rows
  * of 8 x 128 bf16, not 205 of 2048): the keys come from the deviation
  * kernel, then one workgroup per (layer, chunk) runs the chunk's top-k on

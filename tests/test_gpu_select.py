@@ -154,6 +154,83 @@ def test_topk_random_distinct(dev):
     assert np.array_equal(got.cpu().numpy(), want)
 
 
+def topk_keys(kind, rng, n):
+    if kind == "spread":
+        return (rng.standard_t(3, n) ** 2).astype(np.float32)
+    if kind == "few":                                  # ties at the k-th key
+        return rng.integers(0, 3, n).astype(np.float32)
+    if kind == "near":                                 # one exponent: the last bits decide
+        return (np.float32(1.0) + rng.integers(0, 500, n).astype(np.float32) * np.float32(2.0 ** -23))
+    return np.zeros(n, np.float32)                     # every key the same
+
+
+# Chunk lengths at the edges of the top-k's workgroups (1, 4 and 16 wavefronts,
+# 4, 8 and 32 keys per lane, keys from memory), each with small, half, nearly all
+# and all tokens wanted, and more than there are.
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 255, 256, 257, 2047, 2048, 2049, 8192, 8193, 32767, 32768, 32769])
+@pytest.mark.parametrize("kind", ["spread", "few", "near", "zero"])
+def test_topk_workgroup_edges(dev, n, kind):
+    rng = np.random.default_rng(n)
+    short = max(1, n // 3)
+    keys = np.stack([topk_keys(kind, rng, n + short) for _ in range(2)])
+    if kind == "spread" and n > 8:
+        keys[0, n // 2] = np.inf
+        keys[1, 3] = np.array([0x7FC00000], np.uint32).view(np.float32)[0]
+    ks = sorted({1, 2, n // 2, n - 1, n, n + 3} - {0})
+    chunks = [(0, 0, n, k) for k in ks] + [(0, n, short, max(1, short // 5)), (0, n, short, 0)]
+    kmax = max(min(c[2], c[3]) for c in chunks) + 2
+    want = osel.topk_per_chunk(keys, chunks, kmax)
+    got = cache_ops.topk_per_chunk(torch.from_numpy(keys).to(dev), chunks, kmax=kmax)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
+# Rows of 1, 8, 9, 16, 17, 32, 33 and 64 vectors of 8: the lanes that share a
+# token in the deviation kernel, whole and partly filled.
+@pytest.mark.parametrize("h,d", [(1, 8), (1, 64), (3, 24), (1, 128), (1, 136), (2, 128), (3, 88), (4, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.uint8])
+def test_deviation_lane_groups(dev, h, d, dtype):
+    layers, pf, bt, chunks, k_new, _v = setup_case(dev, "nhd", nb=60, h=h, d=d, L=2, dtype=dtype,
+                                                   chunk_tokens=(133, 1, 70), seed=11)
+    scales = None
+    if dtype == torch.uint8:
+        k_new = k_new.to(torch.bfloat16) if k_new.dtype == torch.uint8 else k_new
+        scales = (0.5 + torch.rand(2, h, generator=torch.Generator().manual_seed(5))).float()
+    want = osel.deviation([t for t, _ in layers], pf, bt, k_new, chunks,
+                          **({} if scales is None else {"k_scales": scales.numpy()}))
+    got = cache_ops.kv_deviation([to_dev(t, dev) for t, _ in layers], pf, torch.from_numpy(bt).to(dev),
+                                 k_new.to(dev), chunks, k_scales=None if scales is None else scales.to(dev))
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
+
+
+@pytest.mark.parametrize("quant", [False, True])
+def test_merge_of_uneven_counts(dev, quant):
+    """Chunks that select none, one, a few and nearly all of their tokens: the
+    row batches follow each chunk's own count, in merge_rows and select_merge."""
+    dtype = torch.uint8 if quant else torch.bfloat16
+    layers, pf, bt, chunks, k_new, v_new = setup_case(dev, "nhd", nb=400, h=2, d=64, L=2, dtype=dtype,
+                                                      chunk_tokens=(40, 2300, 17, 64, 900), seed=13)
+    ks = (0, 2250, 17, 1, 130)
+    chunks = [tuple(c[:3]) + (k,) + tuple(c[4:]) for c, k in zip(chunks, ks)]
+    if k_new.dtype == torch.uint8:
+        g = torch.Generator().manual_seed(3)
+        k_new, v_new = (torch.randn(k_new.shape, generator=g).to(torch.bfloat16) for _ in range(2))
+    sc = [torch.full((2, 2), 0.5 + 0.25 * i) for i in range(2)] if quant else [None, None]
+    kw = dict(k_scales=sc[0].numpy(), v_scales=sc[1].numpy()) if quant else {}
+    cpu = [t.clone() for t, _ in layers]
+    keys = osel.deviation(cpu, pf, bt, k_new, chunks, **({"k_scales": sc[0].numpy()} if quant else {}))
+    sel = osel.topk_per_chunk(np.asarray(keys, np.float32), chunks, max(ks))
+    osel.merge_rows(cpu, pf, bt, k_new, v_new, chunks, sel, **kw)
+    gpu = [to_dev(t, dev) for t, _ in layers]
+    gk = dict(k_scales=sc[0].to(dev), v_scales=sc[1].to(dev)) if quant else {}
+    _, got = cache_ops.select_merge(gpu, pf, torch.from_numpy(bt).to(dev), k_new.to(dev), v_new.to(dev), chunks, **gk)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), sel)
+    for t, td in zip(cpu, gpu):
+        assert same_bytes(td, t)
+
+
 def test_deviation_llama_shape(dev):
     # H*D = 1024 (two reduction rounds per lane), as benchmark configuration 3
     layers, pf, bt, chunks, k_new, v_new = setup_case(dev, "nhd", nb=80, h=8, d=128, L=2,
