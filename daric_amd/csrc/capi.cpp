@@ -688,6 +688,11 @@ std::vector<uint8_t*> layer_ptrs(const daric_tensor* layers, int64_t n) {
     return v;
 }
 
+// Fewest rotated units of a page for which the page tiles of the rows kernel
+// beat the element kernel's runs across pages: 48 (one head, 16 tokens) ran 28 ->
+// 36 us, 320 (64 tokens) 41 -> 22 us on MI355X.
+constexpr int64_t kRowsPageUnits = 128;
+
 // A validated in-place rotation: the geometry, kernel path and descriptor
 // bytes (segments, then the layer pointer table) of one call.
 struct InplacePlan {
@@ -729,9 +734,9 @@ InplacePlan plan_inplace(const daric_tensor* layers, int64_t n_layers, int page_
     const int64_t e = t.elem_size;
     const int64_t VE = kind == kE4M3 ? 16 : 8;
     const int64_t half = rope->rotary_dim / 2;
-    bool vec = (L.sb * e) % 16 == 0 && (L.ss * e) % 16 == 0 && (L.sh * e) % 16 == 0 &&
-               (neox ? half % VE == 0 : rope->rotary_dim % VE == 0);
-    for (int64_t i = 0; i < n_layers && vec; ++i) vec = aligned(layers[i].data, 16);
+    bool rows16 = (L.sb * e) % 16 == 0 && (L.ss * e) % 16 == 0 && (L.sh * e) % 16 == 0;
+    for (int64_t i = 0; i < n_layers && rows16; ++i) rows16 = aligned(layers[i].data, 16);
+    const bool vec = rows16 && (neox ? half % VE == 0 : rope->rotary_dim % VE == 0);
 
     InplaceGeom& g = plan.g;
     g.min_block = min_block;
@@ -745,18 +750,20 @@ InplacePlan plan_inplace(const daric_tensor* layers, int64_t n_layers, int page_
     // about 1024 items (vector path) or 2048 pairs (element path) per tile
     const int64_t tile_items = vec ? 1024 : 2048;
     g.tile_tokens = static_cast<int32_t>(std::max<int64_t>(1, tile_items / std::max<int64_t>(per_tok, 1)));
-    // Page tiles (rerotate_lane_kernel) when a page's K rows are dense
-    // rows of a power-of-two number (<= 64) of 16-byte units.
+    // Page tiles when a page's K rows are dense: rerotate_lane_kernel for rows of
+    // a power-of-two number (<= 64) of 16-byte units and pair halves of whole
+    // units, rerotate_rows_kernel for e4m3 halves that end inside a unit.
     int path = vec ? kRotVec : kRotElem;
-    if (vec) {
+    if (rows16) {
         const int64_t W = L.row_width;
         const int64_t upr = W * e / 16;
         int64_t tok_div = 0;
         if (L.H == 1 && L.ss == W) tok_div = 1;
         else if (L.H > 1 && L.ss == L.H * W && L.sh == W) tok_div = L.H;     // [PS, H, W] rows
         else if (L.H > 1 && L.sh == L.PS * W && L.ss == W) tok_div = 1;      // [H, PS, W] rows
-        if (tok_div > 0 && (W * e) % 16 == 0 && upr > 0 && upr <= 64 && (upr & (upr - 1)) == 0 &&
-            L.PS * L.H * upr <= kIntMax) {
+        const int64_t walk = (rope->rotary_dim * e + 15) / 16;
+        const bool page_rows = tok_div > 0 && (W * e) % 16 == 0 && upr > 0 && L.PS * L.H * upr <= kIntMax;
+        if (page_rows && vec && upr <= 64 && (upr & (upr - 1)) == 0) {
             path = kRotLane;
             g.upr = static_cast<int32_t>(upr);
             g.tok_div = static_cast<int32_t>(tok_div);
@@ -768,6 +775,14 @@ InplacePlan plan_inplace(const daric_tensor* layers, int64_t n_layers, int page_
                    (units >> (lp + 1)) % upr == 0)
                 ++lp;
             g.log2_parts = lp;
+        } else if (page_rows && !vec && kind == kE4M3 && L.PS * L.H * walk >= kRowsPageUnits) {
+            path = kRotRows;
+            const RowParts rp(L.PS * L.H, walk);
+            g.upr = static_cast<int32_t>(upr);
+            g.tok_div = static_cast<int32_t>(tok_div);
+            g.walk = static_cast<int32_t>(walk);
+            g.parts = rp.parts;
+            g.part_rows = rp.part_rows;
         }
     }
 
@@ -791,6 +806,8 @@ InplacePlan plan_inplace(const daric_tensor* layers, int64_t n_layers, int page_
         rs.tile_begin = static_cast<int32_t>(tiles);
         if (path == kRotLane)
             tiles += (last_block - s.tok_start / L.PS + 1) << g.log2_parts;   // the pages the segment touches
+        else if (path == kRotRows)
+            tiles += (last_block - s.tok_start / L.PS + 1) * g.parts;
         else
             tiles += (s.n_tokens + g.tile_tokens - 1) / g.tile_tokens;
         segs.push_back(rs);

@@ -134,10 +134,14 @@ struct InplaceGeom {
     int32_t num_blocks;
     int32_t n_rot;     // rotated items per head row (lane path: rotated units per pair half)
     int32_t tile_tokens;
-    int32_t upr;       // lane path: 16-byte units per K row (a power of two dividing 64)
-    int32_t tok_div;   // lane path: rows per token step (H: token-major rows, 1: head-major)
+    int32_t upr;       // lane and rows paths: 16-byte units per K row (lane: a power of two dividing 64)
+    int32_t tok_div;   // lane and rows paths: rows per token step (H: token-major rows, 1: head-major)
     int32_t log2_parts;  // lane path: parts per page tile
     int32_t min_block;   // block ids below it are skipped: 0, or 1 to skip the null block too
+    int32_t walk;        // rows path: units of a row that hold rotated values
+    int32_t parts;       // rows path: parts per page, each but the last of part_rows rows
+    int32_t part_rows;
+    int32_t pad0;
 };
 
 struct RopeSeg {

@@ -450,10 +450,10 @@ void launch_scatter_rotate(const DescArg& d, const JobClasses& classes, const Ro
 // In-place K re-rotation over segments of tokens. `d` holds the n_segs
 // RopeSegs, then (at byte layer_off) the n_layers K base pointers. `path`:
 // kRotElem (per-element access), kRotVec (16-byte items, tiles of
-// g.tile_tokens tokens) or kRotLane (one tile per page of dense K rows, see
-// rerotate_lane_kernel). fp8 codes are rotated as stored (a per-head scale
+// g.tile_tokens tokens), kRotLane or kRotRows (tiles of pages of dense K rows, see
+// rerotate_lane_kernel and rerotate_rows_kernel). fp8 codes are rotated as stored (a per-head scale
 // cancels in a linear rotation).
-enum RotPath { kRotElem = 0, kRotVec = 1, kRotLane = 2 };
+enum RotPath { kRotElem = 0, kRotVec = 1, kRotLane = 2, kRotRows = 3 };
 void launch_rerotate_inplace(const DescArg& d, int layer_off, int n_layers, const InplaceGeom& g,
                              int n_segs, int n_tiles, const int32_t* block_table,
                              const float* inv_freq, int kind, bool neox, int path, hipStream_t stream);

@@ -209,6 +209,17 @@ def inplace_case(dev, layout, dtype, neox, rotary_dim, nb=40, ps=16, h=4, d=64, 
     return worst
 
 
+# (layout, page, heads, head dim, NeoX, rotary dim): e4m3 rows whose halves end
+# inside a unit, one part per page and several, whole and partly rotated rows,
+# segments that start and end inside pages.
+@pytest.mark.parametrize("layout,ps,h,d,neox,rotary_dim", [
+    ("nhd", 16, 8, 80, True, 80), ("hnd", 16, 8, 80, True, 40), ("pf", 16, 8, 80, False, 72),
+    ("packed", 64, 8, 96, True, 48), ("nhd", 64, 8, 144, True, 136), ("mla", 64, 1, 576, True, 72),
+])
+def test_inplace_fp8_rows_kernel(dev, layout, ps, h, d, neox, rotary_dim):
+    inplace_case(dev, layout, torch.uint8, neox, rotary_dim, nb=40, ps=ps, h=h, d=d, L=3, seed=43)
+
+
 # Shifts of long-context models, both signs: 128K positions and past 1M. The
 # first pair's fp32 angle, shift x inv_freq[0] = shift, reaches 10^6 radians,
 # where only sincosf's argument reduction keeps cos and sin accurate.
