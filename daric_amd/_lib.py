@@ -9,6 +9,7 @@ from __future__ import annotations
 import array
 import ctypes
 import os
+import struct
 from ctypes import POINTER, c_char_p, c_double, c_int, c_int32, c_int64, c_uint64, c_void_p
 
 import torch
@@ -90,8 +91,7 @@ SIGNATURES = {
                                                             P(DaricRope), c_uint64]),
     "daric_batched_memcpy_d2h": (c_int, [T, T, I64P, I64P, I64P, c_int64, c_uint64]),
     "daric_batched_memcpy_h2d": (c_int, [T, T, I64P, I64P, I64P, c_int64, c_uint64]),
-    "daric_rerotate_pages": (c_int, [T, c_int64, c_int, T, P(DaricRopeSegment), c_int64, P(DaricRope), T,
-                                     c_uint64]),
+    "daric_rerotate_pages": (c_int, [T, c_int64, c_int, T, I64P, c_int64, P(DaricRope), T, c_uint64]),
     "daric_kv_deviation": (c_int, [T, c_int64, c_int, T, T, P(DaricChunk), c_int64, T, T, c_uint64]),
     "daric_topk_per_chunk": (c_int, [T, P(DaricChunk), c_int64, T, c_uint64]),
     "daric_merge_rows": (c_int, [T, c_int64, c_int, T, T, T, P(DaricChunk), c_int64, T, T, T, c_uint64]),
@@ -132,24 +132,18 @@ def check(status: int) -> None:
         raise (ValueError if status == ERR_VALUE else RuntimeError)(text)
 
 
+# daric_tensor of rank n in one pack: field by field assignment of the ctypes
+# structure took 0.9 us per tensor against 0.6 us (MI355X host).
+_DESC = [struct.Struct(f"@Piiii{n}q{8 * (MAX_DIMS - n)}x{n}q{8 * (MAX_DIMS - n)}x") for n in range(MAX_DIMS + 1)]
+
+
 def desc(t: torch.Tensor) -> DaricTensor:
     n = t.dim()
     if n > MAX_DIMS:
         raise RuntimeError(f"tensor rank {n} exceeds {MAX_DIMS}")
-    d = DaricTensor()
-    d.data = t.data_ptr()
-    d.ndim = n
-    d.elem_size = t.element_size()
-    dv = t.device
-    if dv.type == "cuda":
-        d.device = dv.index if dv.index is not None else torch.cuda.current_device()
-    else:
-        d.device = -1
-    d.dtype = DTYPE_CODES.get(t.dtype, 15)
-    if n:
-        d.sizes[:n] = tuple(t.shape)
-        d.strides[:n] = t.stride()
-    return d
+    return DaricTensor.from_buffer_copy(_DESC[n].pack(
+        t.data_ptr(), n, t.element_size(), t.get_device() if t.is_cuda else -1, DTYPE_CODES.get(t.dtype, 15),
+        *t.shape, *t.stride()))
 
 
 class I64:

@@ -345,9 +345,9 @@ class Adapter:
 
     def _device_inv_freq(self, rotary, device) -> torch.Tensor:
         hit = self._host_inv_freq(rotary)
-        dev = hit[2].get(str(device))
+        dev = hit[2].get(device)
         if dev is None:
-            dev = hit[2][str(device)] = hit[1].to(device).contiguous()
+            dev = hit[2][device] = hit[1].to(device).contiguous()
         return dev
 
     def _group_idx(self, name: str, topo) -> int:

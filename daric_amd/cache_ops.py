@@ -20,15 +20,18 @@ temporary inputs on the launch stream (kernels.cu:202, copier.cpp:69).
 """
 from __future__ import annotations
 
+import array
 import ctypes
 from collections.abc import Sequence
+from contextlib import nullcontext
+from itertools import chain
 from typing import Optional
 
 import numpy as np
 import torch
 
 from . import _lib
-from ._lib import I64, DaricChunk, DaricRope, DaricRopeSegment, check, desc, load, str_array
+from ._lib import I64, DaricChunk, DaricRope, check, desc, load, str_array
 
 __all__ = [
     "CacheCopier", "batched_memcpy_d2h", "batched_memcpy_h2d", "rerotate_pages",
@@ -66,14 +69,21 @@ def _ext_stream(stream: int, device: torch.device):
     return s
 
 
+def _on_stream(stream: int, device: torch.device):
+    """Context in which torch allocates and launches on `stream`; none to enter
+    where that is the current stream already (entering two of them was most of
+    what made a selection over 96 chunks 80 us on the host, now 63 us)."""
+    if stream == _resolve_stream(0, device):
+        return nullcontext()
+    return torch.cuda.stream(_ext_stream(stream, device))
+
+
 def _record(stream: int, device: torch.device, *tensors) -> None:
     """Keep caching-allocator memory of temporaries alive until `stream` has
     consumed them (the reference's record_tensor_on_external_stream). Not
     while a graph is being captured: a captured graph's inputs must outlive
     its replays, which is the caller's to ensure, as for any graph."""
-    if device is None or device.type != "cuda":
-        return
-    if torch.cuda.is_current_stream_capturing():
+    if device is None or device.type != "cuda" or torch.cuda.is_current_stream_capturing():
         return
     ext = _ext_stream(stream, device)
     for t in tensors:
@@ -145,7 +155,7 @@ class CacheCopier:
         return t.device if t is not None else None
 
     def _copy(self, fn, layer_names, offsets, byte_sizes, indices_flat, indices_offsets, stream,
-              extra=()):
+              extra=(), record=()):
         names = list(layer_names)
         dev = self._device(names)
         st = _resolve_stream(stream, dev)
@@ -155,7 +165,7 @@ class CacheCopier:
                     ctypes.byref(idx), ioff.ptr, ioff.n, *extra, ctypes.c_uint64(st))
         check(status)
         if names:
-            _record(st, dev, indices_flat)
+            _record(st, dev, indices_flat, *record)
 
     def gather_pages(self, layer_names: Sequence[str], offsets: Sequence[int],
                      byte_sizes: Sequence[int], indices_flat: torch.Tensor,
@@ -222,9 +232,7 @@ class CacheCopier:
         rope = _rope(inv_freq, rotary_dim, is_neox_style, dev) if names else DaricRope()
         dl, nt = I64(deltas), I64(num_tokens)
         self._copy(fn, names, offsets, byte_sizes, indices_flat, indices_offsets, stream,
-                   extra=(dl.ptr, nt.ptr, ctypes.byref(rope)))
-        if names and dev is not None:
-            _record(_resolve_stream(stream, dev), dev, inv_freq)
+                   extra=(dl.ptr, nt.ptr, ctypes.byref(rope)), record=(inv_freq,))
 
 
 def _memcpy(fn, dev_t, host_t, dev_offsets, host_offsets, sizes, stream, d2h):
@@ -274,6 +282,20 @@ def _layer_array(layers: Sequence[torch.Tensor]):
     return arr
 
 
+def _segments(segs):
+    """(address of daric_rope_segment[n], n, keep-alive) of a list of 4-tuples
+    of ints (0.4 us for four of them; through numpy 1.8 us), or of what else
+    numpy takes as rows of four int64 values."""
+    if all(type(s) is tuple and len(s) == 4 for s in segs):
+        try:
+            flat = array.array("q", chain.from_iterable(segs))
+            return flat.buffer_info()[0], len(segs), flat
+        except TypeError:       # not ints: numpy converts or refuses them
+            pass
+    a = np.ascontiguousarray(np.asarray(segs, dtype=np.int64).reshape(-1, 4))
+    return a.ctypes.data, len(segs), a
+
+
 def rerotate_pages(layers: Sequence[torch.Tensor], page_first: bool, block_table: torch.Tensor,
                    segments: Sequence[tuple[int, int, int, int]], inv_freq: torch.Tensor,
                    rotary_dim: int, is_neox_style: bool = True,
@@ -291,12 +313,11 @@ def rerotate_pages(layers: Sequence[torch.Tensor], page_first: bool, block_table
     dev = layers[0].device
     st = _resolve_stream(stream, dev)
     rope = _rope(inv_freq, rotary_dim, is_neox_style, dev)
-    seg_np = np.ascontiguousarray(np.asarray(segs, dtype=np.int64).reshape(-1, 4))
-    sarr = ctypes.cast(seg_np.ctypes.data, ctypes.POINTER(DaricRopeSegment))
+    sarr, n_segs, _keep = _segments(segs)
     bt = desc(block_table)
     ks = desc(k_scales) if k_scales is not None else None
     check(load().daric_rerotate_pages(_layer_array(layers), len(layers), 1 if page_first else 0,
-                                      ctypes.byref(bt), sarr, len(segs), ctypes.byref(rope),
+                                      ctypes.byref(bt), sarr, n_segs, ctypes.byref(rope),
                                       ctypes.byref(ks) if ks is not None else None,
                                       ctypes.c_uint64(st)))
     _record(st, dev, block_table, inv_freq, k_scales)
@@ -332,12 +353,8 @@ def kv_deviation(layers: Sequence[torch.Tensor], page_first: bool, block_table: 
     if keys is None:
         # zeroed on the launch stream: rows outside every chunk stay 0, and the
         # fill is ordered before the kernel whatever stream the caller passed
-        shape = (len(layers), k_new.shape[1])
-        if st == _resolve_stream(0, dev):
-            keys = torch.zeros(shape, dtype=torch.float32, device=dev)
-        else:
-            with torch.cuda.stream(_ext_stream(st, dev)):
-                keys = torch.zeros(shape, dtype=torch.float32, device=dev)
+        with _on_stream(st, dev):
+            keys = torch.zeros((len(layers), k_new.shape[1]), dtype=torch.float32, device=dev)
     carr, n, _keep = _chunks(chunks)
     bt, kn, kd = desc(block_table), desc(k_new), desc(keys)
     ks = desc(k_scales) if k_scales is not None else None
@@ -409,19 +426,17 @@ def select_merge(layers: Sequence[torch.Tensor], page_first: bool, block_table: 
     layers = list(layers)
     dev = layers[0].device
     st = _resolve_stream(stream, dev)
-    ch = list(chunks) if not isinstance(chunks, np.ndarray) else chunks.tolist()
+    carr, n, ch = _chunks(chunks if isinstance(chunks, np.ndarray) else list(chunks))
     if kmax is None:
-        kmax = max([min(int(c[3]), int(c[2])) for c in ch] + [0])
-    carr, n, _keep = _chunks(ch)
-    shape = (len(layers), k_new.shape[1])
+        kmax = max(0, int(np.minimum(ch[:, 2], ch[:, 3]).max()))
     if keys is None:
         if keys_ready:
             raise ValueError("keys_ready needs keys")
         # zeroed on the launch stream: rows outside every chunk stay 0
-        with torch.cuda.stream(_ext_stream(st, dev)):
-            keys = torch.zeros(shape, dtype=torch.float32, device=dev)
+        with _on_stream(st, dev):
+            keys = torch.zeros((len(layers), k_new.shape[1]), dtype=torch.float32, device=dev)
     if sel_idx is None:
-        with torch.cuda.stream(_ext_stream(st, dev)):
+        with _on_stream(st, dev):
             sel_idx = torch.empty(len(layers), n, kmax, dtype=torch.int32, device=dev)
     bt, kn, kd, si = desc(block_table), desc(k_new), desc(keys), desc(sel_idx)
     vn = desc(v_new) if v_new is not None else None

@@ -563,3 +563,18 @@ def test_job_grids_of_uneven_jobs(hosttest, tiles, parts):
         assert launches == (1 if live else 0)
         if live:
             assert idle <= spread + len(live) * (8 if gather else 1 << log2_run) + 8 * (1 << log2_run)
+
+
+def test_segment_forms():
+    """Tuples of ints take the short way; every other form numpy's, with the same values and errors."""
+    from daric_amd.cache_ops import _segments
+    want = [(0, 0, 512, 5), (32, 1, 300, -6), (51, 15, 41, (1 << 24) - 1)]
+    forms = [want, [list(s) for s in want], list(np.array(want)), [tuple(np.array(s)) for s in want],
+             [tuple(float(x) + (0.5 if x > 0 else 0) for x in s) if i == 0 else s for i, s in enumerate(want)]]
+    for form in forms:
+        addr, n, keep = _segments(form)
+        got = ctypes.cast(addr, ctypes.POINTER(_lib.DaricRopeSegment))
+        assert [(got[i].bt_offset, got[i].tok_start, got[i].n_tokens, got[i].delta) for i in range(n)] == want
+    for bad in ([(1, 2, 3), (1, 2, 3, 4, 5)], [(1, 2, 3)], [("a", 0, 0, 0)]):
+        with pytest.raises(ValueError):
+            _segments(bad)
