@@ -339,6 +339,20 @@ def _chunks(chunks):
     return ctypes.cast(a.ctypes.data, ctypes.POINTER(DaricChunk)), a.shape[0], a
 
 
+def _new_keys(st: int, dev, n_layers: int, rows: int, chunks: np.ndarray) -> torch.Tensor:
+    """Deviation keys [n_layers, rows] allocated on stream `st`. Rows outside
+    every chunk are 0, by a fill ordered before the kernel; chunks that follow
+    each other over all rows, as a batch's plan does, leave none, and the kernel
+    writes every row of a chunk (0 for a block id out of range): no fill then
+    (a call over 294 rows of 17 layers 43.2 -> 41.4 us, over 49152 rows of 32
+    layers 1335 -> 1332 us on MI355X)."""
+    begin = chunks[:, 1]
+    end = begin + chunks[:, 2]
+    whole = begin[0] == 0 and end[-1] == rows and bool((begin[1:] == end[:-1]).all())
+    with _on_stream(st, dev):
+        return (torch.empty if whole else torch.zeros)((n_layers, rows), dtype=torch.float32, device=dev)
+
+
 def kv_deviation(layers: Sequence[torch.Tensor], page_first: bool, block_table: torch.Tensor,
                  k_new: torch.Tensor, chunks, keys: Optional[torch.Tensor] = None,
                  stream: int = 0, k_scales: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -350,12 +364,9 @@ def kv_deviation(layers: Sequence[torch.Tensor], page_first: bool, block_table: 
     layers = list(layers)
     dev = layers[0].device
     st = _resolve_stream(stream, dev)
+    carr, n, ch = _chunks(chunks)
     if keys is None:
-        # zeroed on the launch stream: rows outside every chunk stay 0, and the
-        # fill is ordered before the kernel whatever stream the caller passed
-        with _on_stream(st, dev):
-            keys = torch.zeros((len(layers), k_new.shape[1]), dtype=torch.float32, device=dev)
-    carr, n, _keep = _chunks(chunks)
+        keys = _new_keys(st, dev, len(layers), k_new.shape[1], ch)
     bt, kn, kd = desc(block_table), desc(k_new), desc(keys)
     ks = desc(k_scales) if k_scales is not None else None
     check(load().daric_kv_deviation(_layer_array(layers), len(layers), 1 if page_first else 0,
@@ -432,9 +443,7 @@ def select_merge(layers: Sequence[torch.Tensor], page_first: bool, block_table: 
     if keys is None:
         if keys_ready:
             raise ValueError("keys_ready needs keys")
-        # zeroed on the launch stream: rows outside every chunk stay 0
-        with _on_stream(st, dev):
-            keys = torch.zeros((len(layers), k_new.shape[1]), dtype=torch.float32, device=dev)
+        keys = _new_keys(st, dev, len(layers), k_new.shape[1], ch)
     if sel_idx is None:
         with _on_stream(st, dev):
             sel_idx = torch.empty(len(layers), n, kmax, dtype=torch.int32, device=dev)

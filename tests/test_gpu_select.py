@@ -310,6 +310,34 @@ def test_deviation_allocated_keys_on_a_side_stream(dev):
     assert not keys[:, :10].any() and not keys[:, 10 + k_new.shape[1]:].any()
 
 
+@pytest.mark.parametrize("moved", [
+    lambda c: c,                                            # one after another over all rows: no fill
+    lambda c: [c[2], c[0], c[1]],                           # all rows, another order
+    lambda c: c[:2],                                        # rows after the last
+    lambda c: c[1:],                                        # rows before the first
+    lambda c: [c[0], c[2]],                                 # a gap
+    lambda c: [c[0][:2] + (97,) + c[0][3:], c[1], c[2]],    # a gap of three rows
+])
+@pytest.mark.parametrize("one_call", [False, True])
+def test_allocated_keys_cover_rows(dev, moved, one_call):
+    layers, pf, bt, chunks, k_new, v_new = setup_case(dev, "nhd", chunk_tokens=(100, 64, 37))
+    chunks = moved(chunks)
+    bt = bt.copy()
+    bt[0] = 1 << 20             # a block id out of range: key 0, nothing read
+    cpu = [t for t, _ in layers]
+    gpu = [to_dev(t, dev) for t in cpu]
+    btd, knd, vnd = torch.from_numpy(bt).to(dev), k_new.to(dev), v_new.to(dev)
+    want = osel.deviation(cpu, pf, bt, k_new, chunks)
+    for _ in range(4):          # memory that held NaN before
+        torch.full((len(gpu), k_new.shape[1]), float("nan"), device=dev)
+    if one_call:
+        keys, _ = cache_ops.select_merge(gpu, pf, btd, knd, vnd, chunks)
+    else:
+        keys = cache_ops.kv_deviation(gpu, pf, btd, knd, chunks)
+    torch.cuda.synchronize()
+    assert np.array_equal(keys.cpu().numpy().view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
+
+
 def test_topk_chunk_longer_than_lds_budget(dev):
     """A 20000-token chunk (past the 8192 tokens whose keys the kernel stages
     in LDS) and a short one in the same call: the long chunk's keys are read
