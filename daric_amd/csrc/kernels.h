@@ -164,15 +164,26 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
     constexpr int kLengths = 64;
     JobClass d[kLengths];
     int nd = 0, last = 0;
-    std::vector<uint8_t> of(n);
-    int64_t longest = 0;
-    for (size_t i = 0; i < n; ++i) longest = std::max<int64_t>(longest, count(jobs[i]));
+    int64_t longest = count(jobs[0]);
+    bool even = true;
+    for (size_t i = 1; i < n; ++i) {
+        const int64_t t = count(jobs[i]);
+        even = even && t == longest;
+        longest = std::max(longest, t);
+    }
     if (longest == 0) return out;
+    if (even) {
+        out.n = 1;
+        out.c[0] = {static_cast<int64_t>(n), longest};
+        return out;
+    }
+    std::vector<uint32_t> to(n);      // a job's length, then its place
     // lengths in at most 63 steps of the longest (exact up to 63 tiles, or where
     // no more than 64 lengths occur), rounded up
     int64_t step = 1;
     for (size_t i = 0; i < n; ++i) {
-        const int64_t t = (count(jobs[i]) + step - 1) / step * step;
+        const int64_t tiles = count(jobs[i]);
+        const int64_t t = step == 1 ? tiles : (tiles + step - 1) / step * step;
         if (nd == 0 || d[last].tiles != t) {
             for (last = 0; last < nd && d[last].tiles != t;) ++last;
             if (last == nd) {
@@ -186,7 +197,7 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
             }
         }
         ++d[last].jobs;
-        of[i] = static_cast<uint8_t>(last);
+        to[i] = static_cast<uint32_t>(last);
     }
     if (nd == 1) {
         out.n = 1;
@@ -209,12 +220,20 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
         out.c[k] = {s[k].jobs, std::min(s[k].tiles, longest)};
         at[k + 1] = at[k] + static_cast<size_t>(s[k].jobs);
     }
-    std::vector<Job> sorted(n);
+    uint32_t cls[kLengths];
+    for (int i = 0; i < nd; ++i) cls[i] = d[i].tiles > 0 ? joined[rank[i]] : out.n;
+    for (size_t i = 0; i < n; ++i) to[i] = static_cast<uint32_t>(at[cls[to[i]]]++);
+    // in place: a second array of jobs cost as much again
     for (size_t i = 0; i < n; ++i) {
-        const int r = of[i];
-        sorted[at[d[r].tiles > 0 ? joined[rank[r]] : out.n]++] = jobs[i];
+        if (to[i] == i) continue;
+        Job held = jobs[i];
+        for (uint32_t k = static_cast<uint32_t>(i); to[k] != k;) {
+            const uint32_t next = to[k];
+            to[k] = k;
+            std::swap(held, jobs[next]);
+            k = next;
+        }
     }
-    jobs.swap(sorted);
     return out;
 }
 
