@@ -223,7 +223,9 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
     uint32_t cls[kLengths];
     for (int i = 0; i < nd; ++i) cls[i] = d[i].tiles > 0 ? joined[rank[i]] : out.n;
     for (size_t i = 0; i < n; ++i) to[i] = static_cast<uint32_t>(at[cls[to[i]]]++);
-    // in place: a second array of jobs cost as much again
+    // In place: with a second, zeroed array of jobs and a division per job 432 uneven
+    // jobs of 112 bytes took 9.8 us instead of 4.5, 1280 took 72 instead of 16 (one
+    // host core).
     for (size_t i = 0; i < n; ++i) {
         if (to[i] == i) continue;
         Job held = jobs[i];
