@@ -97,6 +97,14 @@ def test_token_row_parts(dev, layout, ps, h, d, gather):
     _case(dev, [layout, layout], torch.uint8, d=d, h=h, ps=ps, gather=gather, seed=9)
 
 
+# 112 bytes a job: the most that travel inline (25), the fewest and most that the
+# kernels read from the pinned slot (26, 146), and the fewest that are uploaded.
+@pytest.mark.parametrize("gather", [True, False])
+@pytest.mark.parametrize("n_jobs", [25, 26, 146, 147])
+def test_token_copies_job_list_hand_over(dev, n_jobs, gather):
+    _case(dev, ["nhd"] * n_jobs, torch.bfloat16, gather=gather, seed=n_jobs)
+
+
 @pytest.mark.parametrize("n_sel", [33, 35, 40])
 def test_token_gather_xcd_runs_with_tail(dev, n_sel):
     # 8 KiB parts, 2 * n_sel * 4 per job: runs of 32 parts per XCD cover the
