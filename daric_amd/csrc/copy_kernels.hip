@@ -388,8 +388,7 @@ void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t max_
     // lanes. Tiles above 64 KiB ran 1.1-1.25x faster than in eight parts each, and
     // 72 KiB ones 1.1x faster than in eight parts of 9 KiB; parts of 4 KiB ran
     // 0.88-1.05x of these rates (MI355X, tiles of 4 to 256 KiB).
-    int64_t part = 8192;
-    while ((max_span + part - 1) / part * classes[0].tiles > kMaxGridBlocks - 8) part *= 2;
+    const int64_t part = page_part_bytes(max_span, classes[0].tiles);
     const FastDiv parts(static_cast<uint32_t>((max_span + part - 1) / part));
     const int part_units = static_cast<int>(part / vw);
     if (gather) {

@@ -120,4 +120,8 @@ int64_t daric_hosttest_job_grid(int gather, const int64_t* tiles, int64_t n, int
     return bad ? -1 : launches;
 }
 
+int64_t daric_hosttest_page_part_bytes(int64_t max_span, int64_t tiles) {
+    return daric::page_part_bytes(max_span, tiles);
+}
+
 }

@@ -239,6 +239,17 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
     return out;
 }
 
+// Bytes of the parts that a page copy cuts its tiles into, the last part of a
+// tile what is left, for tiles of up to max_span bytes and at most `tiles` of
+// them in a job: 8 KiB, and more where a job's parts would not fit in one launch.
+// A part as long as the tile ends the doubling: a job of up to kMaxGridBlocks
+// tiles then has a workgroup per tile.
+inline int64_t page_part_bytes(int64_t max_span, int64_t tiles) {
+    int64_t part = 8192;
+    while (part < max_span && (max_span + part - 1) / part * tiles > kMaxGridBlocks) part *= 2;
+    return part;
+}
+
 // Where the blocks of each class begin, and what they divide by. A block compares
 // its place with all the begins, without a branch before the last: returning
 // early for the first class ran the gathers of even jobs 2-4% slower and the

@@ -565,6 +565,22 @@ def test_job_grids_of_uneven_jobs(hosttest, tiles, parts):
             assert idle <= spread + len(live) * (8 if gather else 1 << log2_run) + 8 * (1 << log2_run)
 
 
+@pytest.mark.parametrize("span", [1, 16, 8192, 8193, 9216, 73728, (1 << 31) - 1])
+@pytest.mark.parametrize("tiles", [1, 300, (1 << 24) // 9 + 1, (1 << 24) - 9, (1 << 24) - 8, (1 << 24) - 1])
+def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
+    """Up to 2^24 - 1 pages of any span, which is what the copies accept in a
+    job: the choice of a part ends, a launch holds the job's parts, and a block
+    order over them takes every one once."""
+    hosttest.daric_hosttest_page_part_bytes.restype = ctypes.c_int64
+    part = hosttest.daric_hosttest_page_part_bytes(ctypes.c_int64(span), ctypes.c_int64(tiles))
+    parts = -(-span // part)
+    assert part >= 8192 and 1 <= parts and parts * tiles < 1 << 24
+    if tiles >= (1 << 24) - 9 and span == 16:
+        for gather in (0, 1):
+            assert job_grid(hosttest, gather, [tiles], parts, part, 64 << 20)[0] == 1
+            assert job_grid(hosttest, gather, [tiles, 3], parts, part, 64 << 20)[0] == 2
+
+
 def test_segment_forms():
     """Tuples of ints take the short way; every other form numpy's, with the same values and errors."""
     from daric_amd.cache_ops import _segments

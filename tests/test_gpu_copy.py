@@ -130,6 +130,29 @@ def test_gather_xcd_runs_with_tail(dev, n_sel):
     assert same_bytes(sd, oc.store)
 
 
+@pytest.mark.parametrize("n_sel", [(1 << 24) - 9, (1 << 24) - 8, (1 << 24) - 1])
+def test_as_many_pages_as_a_job_may_have(dev, n_sel):
+    """Jobs of 2^24 - 9 to 2^24 - 1 pages of 16 bytes, the longest the copies
+    accept, gathered and scattered back (an id's copies all hold its page)."""
+    nb = 257
+    layer = torch.randint(0, 256, (nb, 1, 16), dtype=torch.uint8, device=dev)
+    idx = (torch.arange(n_sel, device=dev) % (nb - 1) + 1).to(torch.int32)
+    store = torch.zeros(n_sel * 16, dtype=torch.uint8, device=dev)
+    c = cache_ops.CacheCopier()
+    c.register_layer("l", layer, True)
+    c.register_store(store)
+    c.gather_pages(["l"], [0], [n_sel * 16], idx, [0, n_sel])
+    assert torch.equal(store.view(n_sel, 16), layer[idx.long(), 0])
+    want = layer.clone()
+    layer[1:].zero_()
+    c.scatter_pages(["l"], [0], [n_sel * 16], idx, [0, n_sel])
+    assert torch.equal(layer, want)
+    with pytest.raises(RuntimeError, match="too many pages in one job"):
+        more = torch.zeros(1 << 24, dtype=torch.int32, device=dev)
+        c.register_store(torch.zeros(16 << 24, dtype=torch.uint8, device=dev))
+        c.gather_pages(["l"], [0], [16 << 24], more, [0, 1 << 24])
+
+
 def test_errors_surface_as_runtime_error(dev):
     gc = cache_ops.CacheCopier()
     t = torch.zeros(2, 4, 16, 2, 8, dtype=torch.bfloat16, device=dev)
