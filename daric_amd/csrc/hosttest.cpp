@@ -120,6 +120,10 @@ int64_t daric_hosttest_job_grid(int gather, const int64_t* tiles, int64_t n, int
     return bad ? -1 : launches;
 }
 
+void daric_hosttest_store_unit_head(uint8_t* dst, const uint32_t* words, int n) {
+    daric::store_unit_head(dst, words, n);
+}
+
 int64_t daric_hosttest_page_part_bytes(int64_t max_span, int64_t tiles) {
     return daric::page_part_bytes(max_span, tiles);
 }

@@ -58,6 +58,20 @@ struct RowParts {
     }
 };
 
+// Stores the first n bytes (even; all 16 from 16 up) of a 16-byte unit, w its four
+// words, and leaves the rest of dst alone: in place, the bytes past a row's rotary
+// dims may be V, or a tail that another stream writes meanwhile.
+template <class Words>
+inline DARIC_HD void store_unit_head(uint8_t* dst, const Words& w, int n) {
+#ifdef __HIP_DEVICE_COMPILE__
+#pragma unroll
+#endif
+    for (int i = 0; i < 4; ++i) {
+        if (4 * i + 4 <= n) *reinterpret_cast<uint32_t*>(dst + 4 * i) = w[i];
+        else if (4 * i + 2 <= n) *reinterpret_cast<uint16_t*>(dst + 4 * i) = static_cast<uint16_t>(w[i]);
+    }
+}
+
 // Layer-minor block order for kernels over (layer, work item) pairs: block b
 // of a launch takes layer l0 + b % nl and work item w0 + b / nl. Workgroups
 // are dispatched to the 8 XCDs in turn, so with nl a multiple of 8 each XCD

@@ -7,10 +7,11 @@
 // segment's rotary_dim/2 cos/sin values once in fp32 into LDS, and streams
 // the tile's K head rows with 16-byte accesses. A tile is the segment's
 // tokens in one page, or in a part of it, when the page's K rows are dense
-// (rerotate_lane_kernel, rerotate_rows_kernel), else a run of about 1024 16-byte items (rerotate_vec_kernel), or of pairs
-// with per-element accesses when the layout is not 16-byte aligned
-// (rerotate_elem_kernel). Only the rotated [0, R) part of each head row is
-// read and written; V and the rotary tail are never touched.
+// (rerotate_lane_kernel, rerotate_rows_kernel), else a run of about 1024 16-byte
+// items (rerotate_vec_kernel), or of pairs with per-element accesses when the
+// layout is not 16-byte aligned (rerotate_elem_kernel). Only the rotated [0, R)
+// part of each head row is written: V and the rotary tail may be written by
+// others meanwhile. rerotate_rows_kernel reads up to 15 bytes past it.
 #include <hip/hip_runtime.h>
 
 #include "elem.h"
@@ -326,10 +327,10 @@ __global__ __launch_bounds__(kThreads) void rerotate_lane_kernel(
 // Page-tile variant for dense e4m3 rows whose rotary halves end inside a 16-byte
 // unit (rotate_rows.h): a workgroup takes the rotated units of the segment's
 // tokens in a part of one page, whole rows of up to 16 KiB of them. Only the
-// units that hold rotated values are read and written; all of a part's loads come
-// before its first store, and pairs lie in one row, so nothing is read after it
-// was rotated. Layer-minor, nontemporal loads and plain stores as in the lane
-// kernel.
+// units that hold rotated values are read, and only their rotated bytes are
+// written (store_unit_head); all of a part's loads come before its first store,
+// and pairs lie in one row, so nothing is read after it was rotated. Layer-minor,
+// nontemporal loads and plain stores as in the lane kernel.
 // Against the element kernel, which moves single bytes (MI355X, 24 layers, 8
 // heads of 80, two prompts of 4450 tokens): 293 -> 101 us with all 80 values
 // rotated, 165 -> 85 us with 40. For 16-bit values the element kernel stays: with
@@ -392,8 +393,11 @@ __global__ __launch_bounds__(kThreads) void rerotate_rows_kernel(
         const int i = u * kThreads + tid;
         const int row = static_cast<int>(d_walk.div(static_cast<uint32_t>(i)));
         const int k = i - row * walk;
-        pg[static_cast<int64_t>(r0 + row) * g.upr + k] =
-            RR::turn(v[u], s_row + (NEOX ? i - k : 0), k, s_cs, g.R / 2);
+        const u32x4 out = RR::turn(v[u], s_row + (NEOX ? i - k : 0), k, s_cs, g.R / 2);
+        u32x4* dst = pg + static_cast<int64_t>(r0 + row) * g.upr + k;
+        const int bytes = g.R - k * RR::VE;
+        if (bytes >= RR::VE) *dst = out;
+        else store_unit_head(reinterpret_cast<uint8_t*>(dst), out, bytes);
     }
 }
 

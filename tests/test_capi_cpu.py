@@ -581,6 +581,18 @@ def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
             assert job_grid(hosttest, gather, [tiles, 3], parts, part, 64 << 20)[0] == 2
 
 
+@pytest.mark.parametrize("n", range(2, 20, 2))
+def test_store_unit_head_leaves_the_rest_alone(hosttest, n):
+    """The in-place rotation of e4m3 rows writes a unit's rotated bytes only:
+    what follows them may be V, or a tail that another stream writes."""
+    words = np.arange(1, 17, dtype=np.uint8)
+    row = np.full(32, 0xEE, np.uint8)
+    hosttest.daric_hosttest_store_unit_head(ctypes.c_void_p(row.ctypes.data), ctypes.c_void_p(words.ctypes.data),
+                                            ctypes.c_int(n))
+    k = min(n, 16)
+    assert row[:k].tolist() == words[:k].tolist() and (row[k:] == 0xEE).all()
+
+
 def test_segment_forms():
     """Tuples of ints take the short way; every other form numpy's, with the same values and errors."""
     from daric_amd.cache_ops import _segments

@@ -215,9 +215,36 @@ def inplace_case(dev, layout, dtype, neox, rotary_dim, nb=40, ps=16, h=4, d=64, 
 @pytest.mark.parametrize("layout,ps,h,d,neox,rotary_dim", [
     ("nhd", 16, 8, 80, True, 80), ("hnd", 16, 8, 80, True, 40), ("pf", 16, 8, 80, False, 72),
     ("packed", 64, 8, 96, True, 48), ("nhd", 64, 8, 144, True, 136), ("mla", 64, 1, 576, True, 72),
+    ("packed", 16, 8, 72, True, 72), ("packed", 16, 8, 72, False, 70),
 ])
 def test_inplace_fp8_rows_kernel(dev, layout, ps, h, d, neox, rotary_dim):
     inplace_case(dev, layout, torch.uint8, neox, rotary_dim, nb=40, ps=ps, h=h, d=d, L=3, seed=43)
+
+
+def test_inplace_fp8_rows_beside_a_writer_of_v(dev):
+    """Packed e4m3 rows of 72 K values and 72 V values: the last K unit holds
+    eight V values. V written on another stream while K is rotated stays as it
+    was written, and K is what the rotation alone makes of it."""
+    nb, ps, h, d = 2048, 16, 8, 72
+    rows = torch.randint(0, 0x38, (nb, h, ps, 2 * d), dtype=torch.uint8, device=dev)
+    alone = rows.clone()
+    bt = (torch.randperm(nb - 1, device=dev) + 1).to(torch.int32)
+    inv = torch.from_numpy(orope.default_inv_freq(d, THETA)).to(dev)
+    segs = [(0, 0, (nb - 1) * ps, 3)]
+
+    def rotate(t, stream=0):
+        cache_ops.rerotate_pages([t.view(torch.float8_e4m3fn)], True, bt, segs, inv, d, stream=stream)
+    for _ in range(6):
+        rotate(alone)
+    torch.cuda.synchronize()
+    writer, mover = torch.cuda.Stream(), torch.cuda.Stream()
+    for i in range(6):
+        rotate(rows, mover.cuda_stream)
+        with torch.cuda.stream(writer):
+            rows[..., d:] = i + 1
+    torch.cuda.synchronize()
+    assert (rows[..., d:] == 6).all()
+    assert torch.equal(rows[..., :d], alone[..., :d])
 
 
 # Shifts of long-context models, both signs: 128K positions and past 1M. The
