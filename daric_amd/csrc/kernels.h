@@ -516,11 +516,13 @@ void launch_deviation(const DescArg& d, int layer_off, int n_layers, const KVGeo
 void launch_topk(const float* keys, int n_layers, int64_t T, const DescArg& d,
                  int n_chunks, int max_tokens, int32_t* out_idx, int kmax, hipStream_t stream);
 // merge: the SelChunks at byte chunk_off have their first batch of
-// merge_rows_per_block selected rows in tile_begin, n_batches in all. quant_from is -1 (rows are copied as bytes) or the ElemKind of
-// bf16 / fp16 rows quantised into an e4m3 cache with the [n_layers, H] fp32
-// k_scales / v_scales. merge_fits_rows: whether the row kernel takes the
-// geometry (required for quantising); merge_max_row_bytes: the most bytes of
-// recomputed K+V values per token it takes.
+// merge_rows_per_block index slots in tile_begin, n_batches in all (0 rows and
+// batches where the row kernel does not take the geometry). quant_from is -1
+// (rows are copied as bytes) or the ElemKind of bf16 / fp16 rows quantised into
+// an e4m3 cache with the [n_layers, H] fp32 k_scales / v_scales.
+// merge_fits_rows: whether the row kernel takes the geometry (required for
+// quantising); merge_max_row_bytes: the most bytes of recomputed K+V values per
+// token it takes.
 bool merge_fits_rows(const KVGeom& g, int elem_size, bool quant);
 int64_t merge_max_row_bytes();
 int merge_rows_per_block(const KVGeom& g, int elem_size, bool quant);

@@ -702,7 +702,7 @@ bool merge_fits_rows(const KVGeom& g, int elem_size, bool quant) {
 int64_t merge_max_row_bytes() { return static_cast<int64_t>(kMergeThreads) * kMergeUnits * 16; }
 
 int merge_rows_per_block(const KVGeom& g, int elem_size, bool quant) {
-    if (!merge_fits_rows(g, elem_size, quant)) return 1;
+    if (!merge_fits_rows(g, elem_size, quant)) return 0;
     const int tok_units = (g.v_off >= 0 ? 2 : 1) * g.H * (g.D * (quant ? 2 : elem_size) / 16);
     return std::min(kMergeMaxTok, std::max(1, kMergeThreads * kMergeUnits / tok_units));
 }

@@ -108,6 +108,29 @@ def test_quantising_merge_parity(dev, layout, row_dtype):
         assert same_bytes(td, t)
 
 
+@pytest.mark.parametrize("h,d", [(8, 128), (4, 60)])
+def test_merge_of_indices_in_any_slot(dev, h, d):
+    """merge_rows takes a caller's own indices: a chunk's first min(k, kmax)
+    slots may hold them in any place, also past as many slots as it has tokens
+    (row kernel: batches of 8 slots; 120-byte rows: element kernel)."""
+    layers, pf, bt, chunks, k_new, v_new = setup_case(dev, "nhd", h=h, d=d, chunk_tokens=(3, 20, 1, 40))
+    chunks = [c[:3] + (k,) for c, k in zip(chunks, (60, 33, 9, 17))]
+    cpu = [t for t, _ in layers]
+    gpu = [to_dev(t, dev) for t in cpu]
+    sel = np.full((len(cpu), len(chunks), 60), -1, np.int32)
+    for l in range(len(cpu)):
+        sel[l, 0, [0, 30, 59]] = [2, 0, 1]
+        sel[l, 1, [32, 5, 24]] = [19, 0, 7]
+        sel[l, 2, 8] = 0
+        sel[l, 3, :17] = np.arange(17)
+    osel.merge_rows(cpu, pf, bt, k_new, v_new, chunks, sel)
+    cache_ops.merge_rows(gpu, pf, torch.from_numpy(bt).to(dev), k_new.to(dev), v_new.to(dev), chunks,
+                         torch.from_numpy(sel).to(dev))
+    torch.cuda.synchronize()
+    for t, td in zip(cpu, gpu):
+        assert same_bytes(td, t)
+
+
 def test_quantising_merge_argument_errors(dev):
     layers, pf, bt, chunks, _k, _v = setup_case(dev, "nhd", dtype=torch.uint8, L=1)
     gpu = [to_dev(t, dev) for t, _ in layers]
