@@ -124,6 +124,8 @@ void daric_hosttest_store_unit_head(uint8_t* dst, const uint32_t* words, int n) 
     daric::store_unit_head(dst, words, n);
 }
 
+int daric_hosttest_topk_slots(int n, int lanes) { return daric::topk_slots(n, lanes); }
+
 int64_t daric_hosttest_page_part_bytes(int64_t max_span, int64_t tiles) {
     return daric::page_part_bytes(max_span, tiles);
 }

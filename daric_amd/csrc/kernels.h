@@ -504,6 +504,12 @@ void launch_rerotate_inplace(const DescArg& d, int layer_off, int n_layers, cons
                              int n_segs, int n_tiles, const int32_t* block_table,
                              const float* inv_freq, int kind, bool neox, int path, hipStream_t stream);
 
+// Slots of 64 keys a wavefront of the top-k takes of a chunk of n tokens, with T
+// lanes in the workgroup: T * topk_slots(n, T) may pass 2^31 - 1, but not 2^32.
+inline DARIC_HD int topk_slots(int n, int T) {
+    return static_cast<int>((static_cast<uint32_t>(n) + static_cast<uint32_t>(T) - 1) / static_cast<uint32_t>(T));
+}
+
 // Selection kernels. deviation_tile_tokens: tokens per deviation workgroup
 // (the tiling launch_deviation expects in SelChunk::tile_begin).
 int deviation_tile_tokens(int cache_kind, const KVGeom& g);

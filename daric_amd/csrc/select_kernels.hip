@@ -234,14 +234,15 @@ __device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* 
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int slots = (n + T - 1) / T;
-    const int i0 = wave * slots * 64 + lane;
+    const int slots = topk_slots(n, T);
+    const uint32_t un = static_cast<uint32_t>(n);
+    const uint32_t i0 = static_cast<uint32_t>(wave * slots * 64 + lane);
     uint32_t key[R];
     if constexpr (KPT > 0) {
 #pragma unroll
         for (int s = 0; s < KPT; ++s) {
             key[s] = 0;
-            if (s < slots && i0 + s * 64 < n) key[s] = key_at(i0 + s * 64);
+            if (s < slots && i0 + s * 64 < un) key[s] = key_at(static_cast<int>(i0 + s * 64));
         }
     }
     // f(slot, key, whether there is one) for the wavefront's slots
@@ -249,11 +250,11 @@ __device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* 
         if constexpr (KPT > 0) {
 #pragma unroll
             for (int s = 0; s < KPT; ++s)
-                if (s < slots) f(s, key[s], i0 + s * 64 < n);
+                if (s < slots) f(s, key[s], i0 + s * 64 < un);
         } else {
             for (int s = 0; s < slots; ++s) {
-                const bool in = i0 + s * 64 < n;
-                f(s, in ? key_at(i0 + s * 64) : 0u, in);
+                const uint32_t i = i0 + static_cast<uint32_t>(s) * 64;
+                f(s, i < un ? key_at(static_cast<int>(i)) : 0u, i < un);
             }
         }
     };
@@ -351,7 +352,7 @@ __device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* 
         const uint32_t eq_rank = eq + static_cast<uint32_t>(__popcll(me & below));
         const uint32_t pos = gt + static_cast<uint32_t>(__popcll(mg & below)) + min(eq_rank, krem);
         if ((g || (e && eq_rank < krem)) && pos < static_cast<uint32_t>(k)) {
-            const int i = i0 + s * 64;
+            const int i = static_cast<int>(i0 + static_cast<uint32_t>(s) * 64);
             if (orow != nullptr) orow[pos] = i;
             if (s_sel != nullptr) s_sel[pos] = i;
         }

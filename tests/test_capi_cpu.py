@@ -593,6 +593,15 @@ def test_store_unit_head_leaves_the_rest_alone(hosttest, n):
     assert row[:k].tolist() == words[:k].tolist() and (row[k:] == 0xEE).all()
 
 
+@pytest.mark.parametrize("lanes", [64, 256, 1024])
+@pytest.mark.parametrize("n", [0, 1, 63, 64, 65, 1024, 1025, 32769, (1 << 31) - 1024, (1 << 31) - 1023, (1 << 31) - 1])
+def test_topk_slots_cover_the_chunk(hosttest, n, lanes):
+    """A workgroup's slots hold every key of a chunk of any accepted length, the
+    last of them not past it, and a key's place fits 32 bits."""
+    slots = hosttest.daric_hosttest_topk_slots(ctypes.c_int(n), ctypes.c_int(lanes))
+    assert (slots - 1) * lanes < n <= slots * lanes < 1 << 32
+
+
 def test_segment_forms():
     """Tuples of ints take the short way; every other form numpy's, with the same values and errors."""
     from daric_amd.cache_ops import _segments
