@@ -209,6 +209,7 @@ __device__ __forceinline__ uint32_t order_key(float f) {
 // in memory), MI355X, 15% of the tokens selected: one chunk of 500 tokens 6.0 ->
 // 4.6 us, 16 of 5000 29.2 -> 9.5 us, one of 12000 78 -> 18 us, 6 of 30000 194 ->
 // 36 us, 6144 of 512 31.2 -> 23.6 us; all keys equal 6-440 -> 6-94 us.
+constexpr int kTopkWave = 256, kTopkGroup = 2048;   // longest chunks of one and of four wavefronts
 template <int T>
 struct TopkLds {
     static constexpr int kBits = T == 64 ? 8 : 11;
@@ -234,15 +235,16 @@ __device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* 
     const int tid = static_cast<int>(threadIdx.x);
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int slots = topk_slots(n, T);
-    const uint32_t un = static_cast<uint32_t>(n);
-    const uint32_t i0 = static_cast<uint32_t>(wave * slots * 64 + lane);
+    // Places past 2^31 - 1 occur where KPT is 0 only; unsigned places ran the
+    // register forms 2% slower.
+    const int slots = KPT > 0 ? (n + T - 1) / T : topk_slots(n, T);
+    const int i0 = wave * slots * 64 + lane;
     uint32_t key[R];
     if constexpr (KPT > 0) {
 #pragma unroll
         for (int s = 0; s < KPT; ++s) {
             key[s] = 0;
-            if (s < slots && i0 + s * 64 < un) key[s] = key_at(static_cast<int>(i0 + s * 64));
+            if (s < slots && i0 + s * 64 < n) key[s] = key_at(i0 + s * 64);
         }
     }
     // f(slot, key, whether there is one) for the wavefront's slots
@@ -250,11 +252,12 @@ __device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* 
         if constexpr (KPT > 0) {
 #pragma unroll
             for (int s = 0; s < KPT; ++s)
-                if (s < slots) f(s, key[s], i0 + s * 64 < un);
+                if (s < slots) f(s, key[s], i0 + s * 64 < n);
         } else {
             for (int s = 0; s < slots; ++s) {
-                const uint32_t i = i0 + static_cast<uint32_t>(s) * 64;
-                f(s, i < un ? key_at(static_cast<int>(i)) : 0u, i < un);
+                const uint32_t i = static_cast<uint32_t>(i0) + static_cast<uint32_t>(s) * 64;
+                const bool in = i < static_cast<uint32_t>(n);
+                f(s, in ? key_at(static_cast<int>(i)) : 0u, in);
             }
         }
     };
@@ -352,7 +355,7 @@ __device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* 
         const uint32_t eq_rank = eq + static_cast<uint32_t>(__popcll(me & below));
         const uint32_t pos = gt + static_cast<uint32_t>(__popcll(mg & below)) + min(eq_rank, krem);
         if ((g || (e && eq_rank < krem)) && pos < static_cast<uint32_t>(k)) {
-            const int i = static_cast<int>(i0 + static_cast<uint32_t>(s) * 64);
+            const int i = KPT > 0 ? i0 + s * 64 : static_cast<int>(static_cast<uint32_t>(i0) + static_cast<uint32_t>(s) * 64);
             if (orow != nullptr) orow[pos] = i;
             if (s_sel != nullptr) s_sel[pos] = i;
         }
@@ -361,23 +364,39 @@ __device__ __forceinline__ void chunk_topk(KeyAt key_at, int n, int k, int32_t* 
     });
 }
 
-// One workgroup per (layer, chunk). T and KPT by the longest chunk, see
-// launch_topk.
+// One workgroup per (layer, chunk), of T lanes and KPT slots for the call's longest
+// chunk (launch_topk). A shorter chunk is done by the first lanes alone, with the
+// fewest that hold it in registers, and the other wavefronts end at once (a
+// barrier counts the live ones): the short chunks beside a long one would each
+// pay for the barriers of 16 wavefronts. One chunk of 3000 tokens and 40 of 200 in
+// 32 layers 28.5 -> 15.4 us, one of 9000 and 40 of 500 51.6 -> 24.9 us, calls of
+// even chunks unchanged (MI355X).
 template <int T, int KPT>
 __global__ __launch_bounds__(T) void topk_kernel(const float* __restrict__ keys, int64_t stride, DescArg d,
                                                  int n_chunks, int32_t* __restrict__ out, int kmax, int l0) {
     const DescPtr<SelChunk> chunks = desc_at<SelChunk>(d, 0);
-    __shared__ TopkLds<T> sm;
+    static_assert(T <= 256 || sizeof(TopkLds<T>) >= sizeof(TopkLds<256>), "the short forms' LDS fits");
+    __shared__ __align__(16) uint8_t s_mem[sizeof(TopkLds<T>)];
     const int l = static_cast<int>(blockIdx.y) + l0;
     const int ci = static_cast<int>(blockIdx.x);
     const SelChunk c = desc_load(chunks + ci);
     const int n = c.n_tokens;
     const int k = min(max(c.k, 0), n);
     int32_t* __restrict__ orow = out + (static_cast<int64_t>(l) * n_chunks + ci) * kmax;
-    for (int i = k + static_cast<int>(threadIdx.x); i < kmax; i += T) orow[i] = -1;
-    if (k == 0) return;
+    const int tid = static_cast<int>(threadIdx.x);
     const float* krow = keys + static_cast<int64_t>(l) * stride + c.row_offset;
-    chunk_topk<T, KPT>([&](int i) -> uint32_t { return order_key(krow[i]); }, n, k, orow, nullptr, sm);
+    const auto key_at = [&](int i) -> uint32_t { return order_key(krow[i]); };
+    const auto form = [&](auto lanes, auto slots) {
+        constexpr int N = decltype(lanes)::value;
+        if (tid >= N) return;
+        for (int i = k + tid; i < kmax; i += N) orow[i] = -1;
+        if (k == 0) return;
+        chunk_topk<N, decltype(slots)::value>(key_at, n, k, orow, nullptr, *reinterpret_cast<TopkLds<N>*>(s_mem));
+    };
+    using std::integral_constant;
+    if (T > 64 && n <= kTopkWave) form(integral_constant<int, 64>(), integral_constant<int, kTopkWave / 64>());
+    else if (T > 256 && n <= kTopkGroup) form(integral_constant<int, 256>(), integral_constant<int, kTopkGroup / 256>());
+    else form(integral_constant<int, T>(), integral_constant<int, KPT>());
 }
 
 template <int VW>
@@ -679,8 +698,8 @@ void launch_topk(const float* keys, int n_layers, int64_t T, const DescArg& d,
     for (int l0 = 0; l0 < n_layers; l0 += kMaxGridYZ) {
         const dim3 grid(static_cast<unsigned>(n_chunks), static_cast<unsigned>(std::min(kMaxGridYZ, n_layers - l0)));
 #define DARIC_TK(TH, KPT) DARIC_LAUNCH((topk_kernel<TH, KPT>), grid, TH, 0, stream, keys, T, d, n_chunks, out_idx, kmax, l0)
-        if (max_tokens <= 256) DARIC_TK(64, 4);
-        else if (max_tokens <= 2048) DARIC_TK(256, 8);
+        if (max_tokens <= kTopkWave) DARIC_TK(64, kTopkWave / 64);
+        else if (max_tokens <= kTopkGroup) DARIC_TK(256, kTopkGroup / 256);
         else if (max_tokens <= 8192) DARIC_TK(1024, 8);
         else if (max_tokens <= 32768) DARIC_TK(1024, 32);
         else DARIC_TK(1024, 0);

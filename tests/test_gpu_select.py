@@ -208,6 +208,25 @@ def test_topk_workgroup_edges(dev, n, kind):
     assert np.array_equal(got.cpu().numpy(), want)
 
 
+# A long chunk beside short ones at the edges of the forms that a part of its
+# workgroup does.
+@pytest.mark.parametrize("long", [257, 2049, 8192, 8193, 32769])
+@pytest.mark.parametrize("kind", ["spread", "few", "zero"])
+def test_topk_of_uneven_lengths(dev, long, kind):
+    rng = np.random.default_rng(long)
+    lens = [long, 1, 64, 256, 257, 0, 2047, 2048, 2049, 300]
+    keys = np.stack([topk_keys(kind, rng, long + 300) for _ in range(3)])
+    chunks = []
+    for n in lens:
+        n = min(n, long)
+        chunks += [(0, long + 300 - n, n, k) for k in sorted({0, 1, n // 3, n, n + 2})]
+    kmax = long + 1
+    want = osel.topk_per_chunk(keys, chunks, kmax)
+    got = cache_ops.topk_per_chunk(torch.from_numpy(keys).to(dev), chunks, kmax=kmax)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
 # Rows of 1, 8, 9, 16, 17, 32, 33 and 64 vectors of 8: the lanes that share a
 # token in the deviation kernel, whole and partly filled.
 @pytest.mark.parametrize("h,d", [(1, 8), (1, 64), (3, 24), (1, 128), (1, 136), (2, 128), (3, 88), (4, 128)])
