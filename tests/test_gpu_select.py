@@ -208,6 +208,21 @@ def test_topk_workgroup_edges(dev, n, kind):
     assert np.array_equal(got.cpu().numpy(), want)
 
 
+# More chunks than CUs, where those of up to 8192 tokens take fewer lanes; they
+# share rows.
+@pytest.mark.parametrize("n_chunks,longest", [(128, 4097), (129, 2049), (129, 4097), (129, 8192), (129, 8193)])
+def test_topk_of_many_long_chunks(dev, n_chunks, longest):
+    rng = np.random.default_rng(longest)
+    keys = np.stack([topk_keys(kind, rng, longest + n_chunks) for kind in ("spread", "few")])
+    chunks = [(0, c, longest if c == 3 else int(rng.integers(1, longest + 1)), int(rng.integers(0, 400)))
+              for c in range(n_chunks)]
+    kmax = 401
+    want = osel.topk_per_chunk(keys, chunks, kmax)
+    got = cache_ops.topk_per_chunk(torch.from_numpy(keys).to(dev), chunks, kmax=kmax)
+    torch.cuda.synchronize()
+    assert np.array_equal(got.cpu().numpy(), want)
+
+
 # A long chunk beside short ones at the edges of the forms that a part of its
 # workgroup does.
 @pytest.mark.parametrize("long", [257, 2049, 8192, 8193, 32769])
