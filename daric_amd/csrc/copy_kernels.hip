@@ -383,14 +383,13 @@ constexpr int64_t kScatterRunsFrom = (128ll << 20) + 1, kFusedRunsFrom = 64ll <<
 void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t max_span, int vw,
                        bool gather, hipStream_t stream) {
     if (classes.empty()) return;
-    // Tiles cut into parts of 8 KiB (two accesses of 16 bytes per lane), the last
-    // part of a tile what is left, so that every part but that one fills its
-    // lanes. Tiles above 64 KiB ran 1.1-1.25x faster than in eight parts each, and
-    // 72 KiB ones 1.1x faster than in eight parts of 9 KiB; parts of 4 KiB ran
-    // 0.88-1.05x of these rates (MI355X, tiles of 4 to 256 KiB).
+    // The last part of a tile is what is left, so that every part but that one
+    // fills its lanes. Tiles above 64 KiB ran 1.1-1.25x faster in 8 KiB parts than
+    // in eight parts each; parts of 4 KiB ran 0.88-1.05x of these rates (MI355X,
+    // tiles of 4 to 256 KiB).
     const int64_t part = page_part_bytes(max_span, classes[0].tiles);
     const FastDiv parts(static_cast<uint32_t>((max_span + part - 1) / part));
-    const int part_units = static_cast<int>(part / vw);
+    const int part_units = static_cast<int>((part + vw - 1) / vw);
     if (gather) {
         for_job_rows(classes, parts.d, part, [&](int j0, const JobRows& g, unsigned blocks) {
 #define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, true, JobRows>), blocks, kThreads, 0, stream, d, j0, g, parts, part_units)

@@ -255,11 +255,19 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
 
 // Bytes of the parts that a page copy cuts its tiles into, the last part of a
 // tile what is left, for tiles of up to max_span bytes and at most `tiles` of
-// them in a job: 8 KiB, and more where a job's parts would not fit in one launch.
-// A part as long as the tile ends the doubling: a job of up to kMaxGridBlocks
-// tiles then has a workgroup per tile.
+// them in a job: one up to 11 KiB, two equal ones up to 16 KiB, then 8 KiB (two
+// accesses of 16 bytes per lane), and more where a job's parts would not fit in
+// one launch. A part as long as the tile ends the doubling: a job of up to
+// kMaxGridBlocks tiles then has a workgroup per tile.
+// Exact 8 KiB parts left pages of 8.5 to 15 KiB a small second part: gathers of
+// 300 MiB in pages of 8.5, 9, 10 and 12 KiB ran at 0.79, 0.81, 0.88 and 0.97 of
+// the rate of one part per page, scatters at 0.87, 0.91, 0.95 and 1.01, and by
+// this rule at 1.02, 0.99, 0.99 and 1.00, and 1.00, 0.98, 1.00 and 1.03. From
+// 16 KiB up exact parts are 0.99-1.05 of parts of 8 to 16 KiB, and equal parts
+// 0.97-1.03 of exact ones (MI355X).
 inline int64_t page_part_bytes(int64_t max_span, int64_t tiles) {
-    int64_t part = 8192;
+    int64_t part = max_span <= 11 * 1024 ? std::max<int64_t>(max_span, 8192)
+                 : max_span <= 16 * 1024 ? ((max_span + 1) / 2 + 255) / 256 * 256 : 8192;
     while (part < max_span && (max_span + part - 1) / part * tiles > kMaxGridBlocks) part *= 2;
     return part;
 }

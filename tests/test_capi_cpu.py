@@ -565,7 +565,7 @@ def test_job_grids_of_uneven_jobs(hosttest, tiles, parts):
             assert idle <= spread + len(live) * (8 if gather else 1 << log2_run) + 8 * (1 << log2_run)
 
 
-@pytest.mark.parametrize("span", [1, 16, 8192, 8193, 9216, 73728, (1 << 31) - 1])
+@pytest.mark.parametrize("span", [1, 16, 8192, 8193, 9216, 11264, 11265, 12288, 16383, 16384, 73728, (1 << 31) - 1])
 @pytest.mark.parametrize("tiles", [1, 300, (1 << 24) // 9 + 1, (1 << 24) - 9, (1 << 24) - 8, (1 << 24) - 1])
 def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
     """Up to 2^24 - 1 pages of any span, which is what the copies accept in a
@@ -574,7 +574,9 @@ def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
     hosttest.daric_hosttest_page_part_bytes.restype = ctypes.c_int64
     part = hosttest.daric_hosttest_page_part_bytes(ctypes.c_int64(span), ctypes.c_int64(tiles))
     parts = -(-span // part)
-    assert part >= 8192 and 1 <= parts and parts * tiles < 1 << 24
+    assert part >= 5632 and 1 <= parts and parts * tiles < 1 << 24
+    if span > 8192:           # no small last part beside one large one
+        assert parts == 1 or span - (parts - 1) * part >= (5120 if parts == 2 else 1)
     if tiles >= (1 << 24) - 9 and span == 16:
         for gather in (0, 1):
             assert job_grid(hosttest, gather, [tiles], parts, part, 64 << 20)[0] == 1
