@@ -250,7 +250,6 @@ struct ResolvedJobs {
     std::vector<daric_copier::Layer*> layers;
     int64_t max_tiles = 0;
     int64_t max_elements = 0;
-    int64_t max_span = 0;
     int vw = 16;
     int device = -1;
 };
@@ -331,7 +330,7 @@ ResolvedJobs resolve_jobs(daric_copier* c, const char* const* names, int64_t n_j
         j.idx = idx + indices_offsets[i];
         j.prefix_stride = s.prefix_stride;
         j.page_stride = s.page_stride;
-        j.span = s.suffix;
+        j.span = static_cast<int32_t>(s.suffix);
         j.n_sel = static_cast<int32_t>(n_sel);
         j.prefix = static_cast<int32_t>(s.prefix_size);
         j.num_pages = static_cast<int32_t>(s.num_pages);
@@ -339,7 +338,6 @@ ResolvedJobs resolve_jobs(daric_copier* c, const char* const* names, int64_t n_j
         j.delta = 0.0f;
         r.max_tiles = std::max(r.max_tiles, s.prefix_size * n_sel);
         r.max_elements = std::max(r.max_elements, num);
-        r.max_span = std::max(r.max_span, s.suffix);
         const auto al = [&](int64_t a) {
             return s.suffix % a == 0 && s.page_stride % a == 0 && s.prefix_stride % a == 0 &&
                    offsets[i] % a == 0 && aligned(t.data, a);
@@ -522,12 +520,13 @@ int copy_pages(daric_copier* c, const char* const* names, int64_t n_jobs, const 
         ResolvedJobs r = resolve_jobs(c, names, n_jobs, offsets, n_offsets, byte_sizes, n_byte_sizes,
                                       indices, indices_offsets, n_indices_offsets, gather);
         if (r.jobs.empty() || r.max_elements == 0) return;
-        const JobClasses classes = order_jobs(r.jobs, tiles_of);
+        int64_t part = 0;
+        const JobClasses classes = cut_pages(r.jobs, r.vw, &part);
         DeviceGuard guard(r.device);
         const hipStream_t st = as_stream(stream);
         const size_t bytes = r.jobs.size() * sizeof(CopyJob);
         DescHandOver ho(r.device, r.jobs.data(), bytes, st, bytes <= kDirectDescBytes);
-        launch_copy_pages(ho.arg(), classes, r.max_span, r.vw, gather, st);
+        launch_copy_pages(ho.arg(), classes, part, r.vw, gather, st);
     });
 }
 
@@ -898,12 +897,13 @@ void scatter_then_rotate(ResolvedJobs& r, const daric_tensor* indices, const int
                                      static_cast<int64_t>(sv.size()), rope, nullptr, 1);
         if (p.n_segs > 0) plans.push_back(std::move(p));
     }
-    const JobClasses classes = order_jobs(r.jobs, tiles_of);   // the plans hold what they need of the jobs
+    int64_t part = 0;
+    const JobClasses classes = cut_pages(r.jobs, r.vw, &part);   // the plans hold what they need of the jobs
     DeviceGuard guard(r.device);
     const hipStream_t st = as_stream(stream);
     {
         DescHandOver ho(r.device, r.jobs.data(), r.jobs.size() * sizeof(CopyJob), st);
-        launch_copy_pages(ho.arg(), classes, r.max_span, r.vw, false, st);
+        launch_copy_pages(ho.arg(), classes, part, r.vw, false, st);
     }
     for (const InplacePlan& p : plans) launch_inplace(p, st);
 }

@@ -85,18 +85,17 @@ __device__ __forceinline__ bool resolve_tile(const CopyJob& j, int t, int& p, in
 // A unit is a part of a tile: part_units accesses of VW bytes, the last part of a
 // tile what is left.
 template <int VW, bool GATHER, class Grid>
-__global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job0, Grid grid, FastDiv parts,
-                                                              int part_units) {
-    DARIC_ARGS_TOGETHER6(d.ptr, job0, grid.begin[1], grid.cls[0].div.d, parts.d, part_units);
+__global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job0, Grid grid) {
+    DARIC_ARGS_TOGETHER4(d.ptr, job0, grid.begin[1], grid.cls[0].div.d);
     int jb, unit;
     grid.at_block(blockIdx.x, jb, unit);
     const CopyJob j = desc_load(desc_at<CopyJob>(d, 0) + job0 + jb);
-    const int tile = static_cast<int>(parts.div(static_cast<uint32_t>(unit)));
+    const int tile = static_cast<int>(j.parts.div(static_cast<uint32_t>(unit)));
     int p, s;
     uint8_t *cache, *stage;
     if (!resolve_tile(j, tile, p, s, cache, stage)) return;
-    const int u0 = (unit - tile * static_cast<int>(parts.d)) * part_units;
-    const int cnt = min(part_units, static_cast<int>(j.span / VW) - u0);
+    const int u0 = (unit - tile * static_cast<int>(j.parts.d)) * j.part_units;
+    const int cnt = min(j.part_units, j.span / VW - u0);
     if (cnt <= 0) return;
     const int64_t b0 = static_cast<int64_t>(u0) * VW;
     if (GATHER)
@@ -226,7 +225,7 @@ __global__ __launch_bounds__(kThreads) void scatter_rotate_lane_kernel(
     int p, s;
     uint8_t *cache, *stage;
     if (!resolve_tile(j, unit >> log2_parts, p, s, cache, stage)) return;
-    const int n_units = static_cast<int>(j.span / 16);
+    const int n_units = j.span / 16;
     const int per = n_units >> log2_parts;
     const int u0 = (unit & ((1 << log2_parts) - 1)) * per;
     const int u1 = u0 + per;
@@ -380,27 +379,20 @@ __global__ __launch_bounds__(kThreads) void upload_kernel(const u32x4* __restric
 
 constexpr int64_t kScatterRunsFrom = (128ll << 20) + 1, kFusedRunsFrom = 64ll << 20;   // JobRuns
 
-void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t max_span, int vw,
+void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t part, int vw,
                        bool gather, hipStream_t stream) {
     if (classes.empty()) return;
-    // The last part of a tile is what is left, so that every part but that one
-    // fills its lanes. Tiles above 64 KiB ran 1.1-1.25x faster in 8 KiB parts than
-    // in eight parts each; parts of 4 KiB ran 0.88-1.05x of these rates (MI355X,
-    // tiles of 4 to 256 KiB).
-    const int64_t part = page_part_bytes(max_span, classes[0].tiles);
-    const FastDiv parts(static_cast<uint32_t>((max_span + part - 1) / part));
-    const int part_units = static_cast<int>((part + vw - 1) / vw);
     if (gather) {
-        for_job_rows(classes, parts.d, part, [&](int j0, const JobRows& g, unsigned blocks) {
-#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, true, JobRows>), blocks, kThreads, 0, stream, d, j0, g, parts, part_units)
+        for_job_rows(classes, 1, part, [&](int j0, const JobRows& g, unsigned blocks) {
+#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, true, JobRows>), blocks, kThreads, 0, stream, d, j0, g)
             if (vw == 16) DARIC_CP(16); else if (vw == 4) DARIC_CP(4); else DARIC_CP(1);
 #undef DARIC_CP
             check_launch("gather_pages");
         });
         return;
     }
-    for_job_runs(classes, parts.d, part, kScatterRunsFrom, [&](int j0, const JobRuns& g, unsigned blocks) {
-#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, false, JobRuns>), blocks, kThreads, 0, stream, d, j0, g, parts, part_units)
+    for_job_runs(classes, 1, part, kScatterRunsFrom, [&](int j0, const JobRuns& g, unsigned blocks) {
+#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, false, JobRuns>), blocks, kThreads, 0, stream, d, j0, g)
         if (vw == 16) DARIC_CP(16); else if (vw == 4) DARIC_CP(4); else DARIC_CP(1);
 #undef DARIC_CP
         check_launch("scatter_pages");

@@ -7,7 +7,30 @@
 
 #include <cstdint>
 
+#ifdef __HIPCC__
+#define DARIC_HD __host__ __device__
+#else
+#define DARIC_HD
+#endif
+
 namespace daric {
+
+// Fast 32-bit division by a run-time constant d (n, d < 2^31):
+// q = (umulhi(n, m) + n) >> s with s = ceil(log2 d), m = floor(2^32 (2^s - d) / d) + 1.
+struct FastDiv {
+    uint32_t d = 1, m = 1, s = 0;
+    FastDiv() = default;
+    explicit FastDiv(uint32_t div) : d(div) {
+        s = 0;
+        while ((1ull << s) < div) ++s;
+        m = static_cast<uint32_t>(((1ull << 32) * ((1ull << s) - div)) / div + 1);
+    }
+    inline DARIC_HD uint32_t div(uint32_t n) const {
+        // (n * m) >> 32 lowers to v_mul_hi_u32 on the device.
+        const uint32_t hi = static_cast<uint32_t>((static_cast<uint64_t>(n) * m) >> 32);
+        return (hi + n) >> s;
+    }
+};
 
 // Hand-over of a call's descriptors (jobs, segments, chunks, layer pointer
 // tables) to its kernels. Descriptors of up to kInlineDescBytes travel inline
@@ -95,13 +118,14 @@ struct alignas(16) CopyJob {
     const int32_t* idx;
     int64_t prefix_stride;
     int64_t page_stride;
-    int64_t span;
+    int32_t span;
     int32_t n_sel;
     int32_t prefix;
     int32_t num_pages;        // page ids outside [1, num_pages) are skipped
     int32_t n_tokens;         // fused rotate: tokens of the job to rotate
     float delta;              // fused rotate: fp32(new_pos - old_pos)
-    int32_t pad0;
+    int32_t part_units;       // page copies: accesses of a part of a tile
+    FastDiv parts;            // page copies: parts a tile is cut into
 };
 static_assert(sizeof(CopyJob) == 80, "CopyJob layout");
 

@@ -11,30 +11,7 @@
 
 #include "jobs.h"
 
-#ifdef __HIPCC__
-#define DARIC_HD __host__ __device__
-#else
-#define DARIC_HD
-#endif
-
 namespace daric {
-
-// Fast 32-bit division by a run-time constant d (n, d < 2^31):
-// q = (umulhi(n, m) + n) >> s with s = ceil(log2 d), m = floor(2^32 (2^s - d) / d) + 1.
-struct FastDiv {
-    uint32_t d = 1, m = 1, s = 0;
-    FastDiv() = default;
-    explicit FastDiv(uint32_t div) : d(div) {
-        s = 0;
-        while ((1ull << s) < div) ++s;
-        m = static_cast<uint32_t>(((1ull << 32) * ((1ull << s) - div)) / div + 1);
-    }
-    inline DARIC_HD uint32_t div(uint32_t n) const {
-        // (n * m) >> 32 lowers to v_mul_hi_u32 on the device.
-        const uint32_t hi = static_cast<uint32_t>((static_cast<uint64_t>(n) * m) >> 32);
-        return (hi + n) >> s;
-    }
-};
 
 struct RowGeomDiv {
     RowGeom g;
@@ -254,22 +231,48 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
 }
 
 // Bytes of the parts that a page copy cuts its tiles into, the last part of a
-// tile what is left, for tiles of up to max_span bytes and at most `tiles` of
-// them in a job: one up to 11 KiB, two equal ones up to 16 KiB, then 8 KiB (two
+// tile what is left, for a job of `tiles` tiles of `span` bytes: one up to 11 KiB, two equal ones up to 16 KiB, then 8 KiB (two
 // accesses of 16 bytes per lane), and more where a job's parts would not fit in
 // one launch. A part as long as the tile ends the doubling: a job of up to
-// kMaxGridBlocks tiles then has a workgroup per tile.
+// kMaxGridBlocks tiles then has a workgroup per tile. Each job is cut by its own
+// span: by the call's largest, 60 layers of 8 KiB pages beside 4 of 128 KiB had
+// 16 workgroups to each of their pages, 15 of them idle (gather of 584 MiB 645 ->
+// 195 us).
 // Exact 8 KiB parts left pages of 8.5 to 15 KiB a small second part: gathers of
 // 300 MiB in pages of 8.5, 9, 10 and 12 KiB ran at 0.79, 0.81, 0.88 and 0.97 of
 // the rate of one part per page, scatters at 0.87, 0.91, 0.95 and 1.01, and by
 // this rule at 1.02, 0.99, 0.99 and 1.00, and 1.00, 0.98, 1.00 and 1.03. From
 // 16 KiB up exact parts are 0.99-1.05 of parts of 8 to 16 KiB, and equal parts
-// 0.97-1.03 of exact ones (MI355X).
-inline int64_t page_part_bytes(int64_t max_span, int64_t tiles) {
-    int64_t part = max_span <= 11 * 1024 ? std::max<int64_t>(max_span, 8192)
-                 : max_span <= 16 * 1024 ? ((max_span + 1) / 2 + 255) / 256 * 256 : 8192;
-    while (part < max_span && (max_span + part - 1) / part * tiles > kMaxGridBlocks) part *= 2;
+// 0.97-1.03 of exact ones; above 64 KiB they are 1.1-1.25 of eight parts each, and
+// parts of 4 KiB 0.88-1.05 of these rates (MI355X).
+inline int64_t page_part_bytes(int64_t span, int64_t tiles) {
+    int64_t part = span <= 11 * 1024 ? std::max<int64_t>(span, 8192)
+                 : span <= 16 * 1024 ? ((span + 1) / 2 + 255) / 256 * 256 : 8192;
+    while (part < span && (span + part - 1) / part * tiles > kMaxGridBlocks) part *= 2;
     return part;
+}
+
+// Cuts the jobs' tiles into parts for accesses of vw bytes and orders the jobs by
+// their parts. *part gets the longest part's bytes.
+inline JobClasses cut_pages(std::vector<CopyJob>& jobs, int vw, int64_t* part) {
+    *part = 0;
+    const CopyJob* like = nullptr;     // job whose tiles the last one had: no divisions again
+    for (CopyJob& j : jobs) {
+        const int64_t tiles = static_cast<int64_t>(j.prefix) * j.n_sel;
+        if (like != nullptr && like->span == j.span && like->n_sel == j.n_sel && like->prefix == j.prefix) {
+            j.part_units = like->part_units;
+            j.parts = like->parts;
+        } else {
+            const int64_t bytes = page_part_bytes(j.span, tiles);
+            j.part_units = static_cast<int32_t>((bytes + vw - 1) / vw);
+            j.parts = FastDiv(static_cast<uint32_t>(std::max<int64_t>(1, (j.span + bytes - 1) / bytes)));
+            if (tiles > 0) *part = std::max(*part, bytes);
+            like = &j;
+        }
+    }
+    return order_jobs(jobs, [](const CopyJob& j) {
+        return static_cast<int64_t>(j.prefix) * j.n_sel * j.parts.d;
+    });
 }
 
 // Where the blocks of each class begin, and what they divide by. A block compares
@@ -490,10 +493,9 @@ static_assert(sizeof(TokenJob) == 112, "TokenJob layout");
 void launch_token_copy(const DescArg& d, const JobClasses& classes, int64_t part_bytes, int vw,
                        bool lds, bool gather, hipStream_t stream);
 
-// Plain page copies of the CopyJobs in `d`, ordered by their tiles (order_jobs).
-// vw is the access width in bytes (16, 4 or 1); max_span is the largest page
-// span (bytes) of the jobs.
-void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t max_span, int vw,
+// Plain page copies of the CopyJobs in `d`, cut and ordered by cut_pages for
+// accesses of vw bytes (16, 4 or 1); part is its longest part.
+void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t part, int vw,
                        bool gather, hipStream_t stream);
 
 // Fused scatter + K re-rotation of the CopyJobs in `d`, ordered by their tiles

@@ -583,6 +583,18 @@ def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
             assert job_grid(hosttest, gather, [tiles, 3], parts, part, 64 << 20)[0] == 2
 
 
+def test_page_copies_cut_each_job_by_its_own_span(hosttest):
+    """Layers of different page sizes in one call: a page has the workgroups that
+    its own bytes need, whatever the other pages' size."""
+    spans = [131072, 8192, 4608, 9216, 12288, 73728, 16] * 3
+    tiles = [40 + i for i in range(len(spans))]
+    t, s = np.asarray(tiles, np.int64), np.asarray(spans, np.int64)
+    units = np.zeros_like(t)
+    hosttest.daric_hosttest_page_units(ctypes.c_void_p(t.ctypes.data), ctypes.c_void_p(s.ctypes.data),
+                                       ctypes.c_int64(t.size), ctypes.c_int(16), ctypes.c_void_p(units.ctypes.data))
+    assert (units // t).tolist() == [16, 1, 1, 1, 2, 9, 1] * 3
+
+
 @pytest.mark.parametrize("n", range(2, 20, 2))
 def test_store_unit_head_leaves_the_rest_alone(hosttest, n):
     """The in-place rotation of e4m3 rows writes a unit's rotated bytes only:
