@@ -464,13 +464,6 @@ int copy_tokens(daric_copier* c, const char* const* names, int64_t n_jobs, const
         const auto parts_of = [](const TokenJob& j) {
             return static_cast<int64_t>(j.n_kv) * j.n_sel * j.parts_per_page;
         };
-        // Row kernel parts: 8 KiB, two accesses per lane, up to a quarter more where
-        // that saves a part, and parts of a page equal in size. Against 16 KiB
-        // (MI355X): 1.00-1.13x on gathers, 0.95-1.13x on scatters; 4 KiB 0.7-1.05x.
-        // Against exact 8 KiB, which cut pages of 9 to 10 KiB in one full and one
-        // small part: 1.03-1.14x on those, 0.99-1.01x elsewhere (scatter of 11 layers
-        // of 9 KiB pages 21.0 -> 18.4 us).
-        constexpr int64_t kRowPart = 10240;
         const TokenJob* like = nullptr;     // job whose geometry the last one had: no divisions again
         for (TokenJob& j : jobs) {
             if (like != nullptr && like->H == j.H && like->row_bytes == j.row_bytes && like->PS == j.PS) {
@@ -481,15 +474,10 @@ int copy_tokens(daric_copier* c, const char* const* names, int64_t n_jobs, const
             } else {
                 const int64_t row_units = j.row_bytes / vw;
                 const int64_t head_units = static_cast<int64_t>(j.H) * row_units;
-                int64_t pt;
-                if (lds) pt = std::max<int64_t>(1, 512 / head_units);                 // 8 KiB of LDS
-                else pt = std::max<int64_t>(1, (vw == 16 ? kRowPart : 4096) / (static_cast<int64_t>(j.H) * j.row_bytes));
-                pt = std::min<int64_t>(pt, j.PS);
-                int64_t parts = (j.PS + pt - 1) / pt;
-                if (!lds) {
-                    pt = (j.PS + parts - 1) / parts;
-                    parts = (j.PS + pt - 1) / pt;
-                }
+                const int64_t tok_bytes = static_cast<int64_t>(j.H) * j.row_bytes;
+                const int64_t pt = lds ? std::min<int64_t>(j.PS, std::max<int64_t>(1, 512 / head_units))   // 8 KiB of LDS
+                                       : token_row_part(j.PS, tok_bytes, vw);
+                const int64_t parts = (j.PS + pt - 1) / pt;
                 DARIC_CHECK(pt * head_units <= kIntMax, "page part exceeds int range");
                 j.part_tokens = static_cast<int32_t>(pt);
                 j.parts_per_page = static_cast<int32_t>(parts);

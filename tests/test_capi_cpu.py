@@ -583,6 +583,17 @@ def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
             assert job_grid(hosttest, gather, [tiles, 3], parts, part, 64 << 20)[0] == 2
 
 
+# (tokens of a page, bytes of a token, access width, tokens of a part)
+@pytest.mark.parametrize("ps,tok,vw,want", [
+    (16, 576, 16, 16), (16, 768, 16, 16), (16, 896, 16, 16), (16, 912, 16, 8), (16, 1024, 16, 8), (16, 1792, 16, 8),
+    (16, 2048, 16, 4), (64, 1152, 16, 8), (65, 160, 16, 65), (3, 10368, 16, 1), (1, 70000, 16, 1), (16, 768, 1, 4),
+    (16, 5000, 1, 1), (5, 16, 16, 5),
+])
+def test_token_row_parts(hosttest, ps, tok, vw, want):
+    hosttest.daric_hosttest_token_row_part.restype = ctypes.c_int64
+    assert hosttest.daric_hosttest_token_row_part(ctypes.c_int64(ps), ctypes.c_int64(tok), ctypes.c_int(vw)) == want
+
+
 def test_page_copies_cut_each_job_by_its_own_span(hosttest):
     """Layers of different page sizes in one call: a page has the workgroups that
     its own bytes need, whatever the other pages' size."""

@@ -88,11 +88,13 @@ def test_token_copies_llama3_8b_hnd(dev, gather):
           sels=[list(range(1, 33)), [5, 0, 7, 39, 41]])
 
 
-# Row kernel parts: pages (one of K or V) of 9 KiB, exactly 10 KiB and one token
-# more, of tokens that do not divide into equal parts, and tokens past a part.
+# Row kernel parts: pages (one of K or V) of 9 and 10 KiB, of 14 and 28 KiB exactly
+# and more, of tokens that do not divide into equal parts, and tokens past a part.
 @pytest.mark.parametrize("gather", [True, False])
 @pytest.mark.parametrize("layout,ps,h,d", [("mla", 16, 1, 576), ("nhd", 64, 2, 80), ("nhd", 64, 1, 160),
-                                           ("pf", 65, 2, 80), ("nhd", 37, 4, 144), ("nhd", 3, 8, 1296)])
+                                           ("pf", 65, 2, 80), ("nhd", 37, 4, 144), ("nhd", 3, 8, 1296),
+                                           ("nhd", 16, 1, 896), ("nhd", 16, 2, 456), ("nhd", 14, 1, 2048),
+                                           ("pf", 15, 1, 1888), ("nhd", 29, 1, 992)])
 def test_token_row_parts(dev, layout, ps, h, d, gather):
     _case(dev, [layout, layout], torch.uint8, d=d, h=h, ps=ps, gather=gather, seed=9)
 
