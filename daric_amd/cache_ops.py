@@ -284,11 +284,13 @@ def _layer_array(layers: Sequence[torch.Tensor]):
 
 def _segments(segs):
     """(address of daric_rope_segment[n], n, keep-alive) of a list of 4-tuples
-    of ints (0.4 us for four of them; through numpy 1.8 us), or of what else
-    numpy takes as rows of four int64 values."""
-    if all(type(s) is tuple and len(s) == 4 for s in segs):
+    of ints, or of what else numpy takes as rows of four int64 values. Without a
+    Python-level loop: 4, 100 and 1000 tuples take 0.8, 7.0 and 63 us on the
+    host, through numpy 1.5, 10.8 and 95 (with a generator over the tuples 0.9,
+    11.8 and 111)."""
+    if set(map(type, segs)) == {tuple} and set(map(len, segs)) == {4}:
         try:
-            flat = array.array("q", chain.from_iterable(segs))
+            flat = array.array("q", list(chain.from_iterable(segs)))
             return flat.buffer_info()[0], len(segs), flat
         except TypeError:       # not ints: numpy converts or refuses them
             pass
