@@ -705,10 +705,28 @@ std::vector<uint8_t*> layer_ptrs(const daric_tensor* layers, int64_t n) {
     return v;
 }
 
-// Fewest rotated units of a page for which the page tiles of the rows kernel
-// beat the element kernel's runs across pages: 48 (one head, 16 tokens) ran 28 ->
-// 36 us, 320 (64 tokens) 41 -> 22 us on MI355X.
-constexpr int64_t kRowsPageUnits = 128;
+// Fewest rotated units per workgroup, on average over a call's segments, for which
+// the rows kernel's parts of pages beat the element kernel's runs across pages.
+// MI355X, whole pages: 48 (one head, 16 tokens) 28 -> 36 us, 320 (64 tokens) 41 ->
+// 22 us; short segments in 24 layers of 8 heads of 80: 25 (100 of 7 tokens, pages
+// of 256) 46 -> 62 us, 40 (1000 of one token, pages of 16) 51 -> 62 us, 280 (100 of
+// 7, pages of 16) 41 -> 18 us.
+constexpr int64_t kRowsUnits = 128;
+
+// Parts of pages that the segments touch, and their tokens in all. Segments that
+// the checks refuse count nothing.
+struct PartCount {
+    int64_t parts = 0, tokens = 0;
+    PartCount(const daric_rope_segment* segments, int64_t n, int64_t PS, int64_t per_page) {
+        for (int64_t i = 0; i < n; ++i) {
+            const daric_rope_segment& s = segments[i];
+            if (s.n_tokens <= 0 || s.delta == 0 || s.tok_start < 0 || s.tok_start > kIntMax || s.n_tokens > kIntMax)
+                continue;
+            parts += ((s.tok_start + s.n_tokens - 1) / PS - s.tok_start / PS + 1) * per_page;
+            tokens += s.n_tokens;
+        }
+    }
+};
 
 // A validated in-place rotation: the geometry, kernel path and descriptor
 // bytes (segments, then the layer pointer table) of one call.
@@ -792,9 +810,10 @@ InplacePlan plan_inplace(const daric_tensor* layers, int64_t n_layers, int page_
                    (units >> (lp + 1)) % upr == 0)
                 ++lp;
             g.log2_parts = lp;
-        } else if (page_rows && !vec && kind == kE4M3 && L.PS * L.H * walk >= kRowsPageUnits) {
-            path = kRotRows;
+        } else if (page_rows && !vec && kind == kE4M3) {
             const RowParts rp(L.PS * L.H, walk);
+            const PartCount count(segments, n_segments, L.PS, rp.parts);
+            if (count.parts <= kMaxTiles && count.tokens * L.H * walk >= kRowsUnits * count.parts) path = kRotRows;
             g.upr = static_cast<int32_t>(upr);
             g.tok_div = static_cast<int32_t>(tok_div);
             g.walk = static_cast<int32_t>(walk);

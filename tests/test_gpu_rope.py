@@ -221,6 +221,19 @@ def test_inplace_fp8_rows_kernel(dev, layout, ps, h, d, neox, rotary_dim):
     inplace_case(dev, layout, torch.uint8, neox, rotary_dim, nb=40, ps=ps, h=h, d=d, L=3, seed=43)
 
 
+@pytest.mark.parametrize("ps,segs", [
+    (256, [(0, 3 + 40 * i, 1 + i % 7, 5 - i) for i in range(12)]),      # far apart: a few tokens of each part
+    (16, [(0, 16 * i + i % 16, 1, 7 + i) for i in range(30)]),          # one token a page
+    (64, [(0, 0, 64, 9), (0, 70, 3, -9), (0, 128, 200, 1), (0, 500, 1, 2)]),
+])
+@pytest.mark.parametrize("neox", [True, False])
+def test_inplace_fp8_short_segments(dev, ps, segs, neox):
+    """Segments that fill little of the page parts they touch, beside whole
+    pages: element and rows kernels."""
+    inplace_case(dev, "nhd", torch.uint8, neox, 72, nb=40, ps=ps, h=4, d=80, L=2, seed=44,
+                 plan=lambda perm: (np.asarray(perm[:-(-600 // ps)], np.int32), segs))
+
+
 def test_inplace_fp8_rows_beside_a_writer_of_v(dev):
     """Packed e4m3 rows of 72 K values and 72 V values: the last K unit holds
     eight V values. V written on another stream while K is rotated stays as it
