@@ -1195,23 +1195,6 @@ Chunks build_chunks(const daric_chunk* chunks, int64_t n, int64_t PS, int64_t bt
     return c;
 }
 
-// Sets each chunk's first batch of `rows` index slots; returns all batches (none
-// where rows is 0: the element kernel has a grid of its own). top_k: the indices
-// are the top-k's own, whose slots past the chunk's tokens are empty. A caller's
-// may stand in any of a chunk's first min(k, kmax) slots.
-int64_t merge_batches(std::vector<SelChunk>& chunks, int64_t kmax, int rows, bool top_k) {
-    if (rows == 0) return 0;
-    int64_t n = 0;
-    for (SelChunk& c : chunks) {
-        DARIC_CHECK(n <= kIntMax, "too many selected rows in one call");
-        c.tile_begin = static_cast<int32_t>(n);
-        const int64_t slots = std::min<int64_t>(c.k, kmax);
-        n += ((top_k ? std::min<int64_t>(slots, c.n_tokens) : slots) + rows - 1) / rows;
-    }
-    DARIC_CHECK(n <= kIntMax, "too many selected rows in one call");
-    return n;
-}
-
 void check_rows_tensor(const daric_tensor* x, const daric_tensor& layer, int64_t n_layers,
                        int64_t H, int64_t D, const char* what, int64_t* T) {
     check_tensor_struct(x, what);
@@ -1370,7 +1353,8 @@ int daric_merge_rows(const daric_tensor* layers, int64_t n_layers, int page_firs
         // index slots): no launch, so empty k_new / v_new (whose data pointer
         // may be null) are never read.
         if (kmax == 0 || T == 0 || c.max_k == 0) return;
-        const int64_t batches = merge_batches(c.v, kmax, merge_rows_per_block(g, t.elem_size, quant), false);
+        const MergeBatches batches = merge_batches(c.v, kmax, merge_rows_per_block(g, t.elem_size, quant), false);
+        DARIC_CHECK(batches.n <= kIntMax, "too many selected rows in one call");
         DeviceGuard guard(t.device);
         const hipStream_t st = as_stream(stream);
         const size_t cb = c.v.size() * sizeof(SelChunk);
@@ -1477,8 +1461,9 @@ int daric_select_merge(const daric_tensor* layers, int64_t n_layers, int page_fi
         std::memcpy(blob.data(), c.v.data(), cb);
         const auto ptrs = layer_ptrs(layers, n_layers);
         std::memcpy(blob.data() + cb, ptrs.data(), n_layers * sizeof(uint8_t*));
-        int64_t batches = 0;
+        MergeBatches batches;
         if (merges) batches = merge_batches(c.v, kmax, merge_rows_per_block(g, t.elem_size, quant), true);
+        DARIC_CHECK(batches.n <= kIntMax, "too many selected rows in one call");
         if (both) std::memcpy(blob.data() + chunks2, c.v.data(), cb);
         DescHandOver ho(t.device, blob.data(), blob.size(), st);
         const float* ksc = quant ? static_cast<const float*>(k_scales->data) : nullptr;

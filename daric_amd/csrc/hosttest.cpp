@@ -150,4 +150,19 @@ int64_t daric_hosttest_page_part_bytes(int64_t max_span, int64_t tiles) {
     return daric::page_part_bytes(max_span, tiles);
 }
 
+// The batches that the row merge makes of chunks of n_tokens[i] tokens and k[i]
+// slots: begin[i] and, as return value, their number; *each as MergeBatches has it.
+int64_t daric_hosttest_merge_batches(const int32_t* n_tokens, const int32_t* k, int64_t n, int64_t kmax, int rows,
+                                     int top_k, int32_t* begin, int64_t* each) {
+    std::vector<daric::SelChunk> chunks(static_cast<size_t>(n));
+    for (size_t i = 0; i < chunks.size(); ++i) {
+        chunks[i].n_tokens = n_tokens[i];
+        chunks[i].k = k[i];
+    }
+    const daric::MergeBatches b = daric::merge_batches(chunks, kmax, rows, top_k != 0);
+    for (size_t i = 0; i < chunks.size(); ++i) begin[i] = chunks[i].tile_begin;
+    *each = b.each;
+    return b.n;
+}
+
 }

@@ -548,9 +548,31 @@ void launch_deviation(const DescArg& d, int layer_off, int n_layers, const KVGeo
                       const float* k_scales, float* keys, hipStream_t stream);
 void launch_topk(const float* keys, int n_layers, int64_t T, const DescArg& d,
                  int n_chunks, int max_tokens, int32_t* out_idx, int kmax, hipStream_t stream);
-// merge: the SelChunks at byte chunk_off have their first batch of
-// merge_rows_per_block index slots in tile_begin, n_batches in all (0 rows and
-// batches where the row kernel does not take the geometry). quant_from is -1
+// Sets each chunk's first batch of `rows` index slots in tile_begin: n batches in
+// all, `each` per chunk (0 where the chunks differ); none where rows is 0 (the
+// element kernel has a grid of its own). top_k: the indices are the top-k's own,
+// whose slots past the chunk's tokens are empty. A caller's may stand in any of a
+// chunk's first min(k, kmax) slots.
+struct MergeBatches {
+    int64_t n = 0, each = 0;
+};
+inline MergeBatches merge_batches(std::vector<SelChunk>& chunks, int64_t kmax, int rows, bool top_k) {
+    MergeBatches b;
+    if (rows == 0) return b;
+    for (size_t i = 0; i < chunks.size(); ++i) {
+        SelChunk& c = chunks[i];
+        c.tile_begin = static_cast<int32_t>(b.n);
+        const int64_t slots = std::min<int64_t>(c.k, kmax);
+        const int64_t own = ((top_k ? std::min<int64_t>(slots, c.n_tokens) : slots) + rows - 1) / rows;
+        b.each = i == 0 || b.each == own ? own : 0;
+        b.n += own;
+        if (b.n > 0x7fffffff) break;      // refused by the caller
+    }
+    return b;
+}
+// merge: the SelChunks at byte chunk_off have their batches of merge_rows_per_block
+// index slots (merge_batches; 0 rows and batches where the row kernel does not
+// take the geometry). quant_from is -1
 // (rows are copied as bytes) or the ElemKind of bf16 / fp16 rows quantised into
 // an e4m3 cache with the [n_layers, H] fp32 k_scales / v_scales.
 // merge_fits_rows: whether the row kernel takes the geometry (required for
@@ -561,7 +583,7 @@ int64_t merge_max_row_bytes();
 int merge_rows_per_block(const KVGeom& g, int elem_size, bool quant);
 void launch_merge(const DescArg& d, int chunk_off, int layer_off, int n_layers, const KVGeom& g, int elem_size,
                   const int32_t* block_table, const uint8_t* k_new, const uint8_t* v_new,
-                  int64_t T, int n_chunks, int64_t n_batches, const int32_t* sel_idx, int kmax, int quant_from,
+                  int64_t T, int n_chunks, const MergeBatches& batches, const int32_t* sel_idx, int kmax, int quant_from,
                   const float* k_scales, const float* v_scales, hipStream_t stream);
 // Fused selection, one workgroup per (layer, chunk): top-k on the chunk's
 // keys held in LDS and the merge of its selected rows, with (with_keys) or

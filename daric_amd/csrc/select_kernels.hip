@@ -561,12 +561,15 @@ __device__ __forceinline__ void merge_units(
 // recompute policy gives a prompt's last document most of its budget), and a
 // grid of the largest count times the chunks left most workgroups idle (MI355X,
 // counts of 2% to 90% of 8 chunks of 3000 tokens, 22 layers of 4 x 96: 80 -> 60 us).
+// Chunks of d_each.d batches each (0: uneven) are found by a division: the search's
+// chain of loads cost 0.5 us in a short launch and 8 us in one of 400 chunks (32
+// layers of 2 x 64, 10 rows each: 43.6 us, 36.0 by division).
 template <int MODE, bool DENSE>
 __global__ __launch_bounds__(kMergeThreads) void merge_rows_kernel(
     DescArg d, int chunk_off, int layer_off, KVGeom g, int ces, const int32_t* __restrict__ bt,
     const uint8_t* __restrict__ k_new, const uint8_t* __restrict__ v_new, int64_t T,
     int n_chunks, const int32_t* __restrict__ sel, int kmax, int tpb, int units,
-    FastDiv d_tok_units, FastDiv d_upr, const float* __restrict__ k_scales,
+    FastDiv d_tok_units, FastDiv d_upr, FastDiv d_each, const float* __restrict__ k_scales,
     const float* __restrict__ v_scales, LayerMinor lm) {
     __shared__ int64_t s_src[kMergeMaxTok];   // byte offset of the token's recomputed rows (-1: skip)
     __shared__ int64_t s_dst[kMergeMaxTok];   // byte offset of the token's K row in the layer
@@ -576,7 +579,8 @@ __global__ __launch_bounds__(kMergeThreads) void merge_rows_kernel(
     int l;
     int64_t item;
     lm.at(l, item);
-    const int ci = find_by_tile(chunks, n_chunks, static_cast<int>(item));
+    const int ci = d_each.d ? static_cast<int>(d_each.div(static_cast<uint32_t>(item)))
+                            : find_by_tile(chunks, n_chunks, static_cast<int>(item));
     const SelChunk c = desc_load(chunks + ci);
     const int bx = static_cast<int>(item) - c.tile_begin;
     const int tid = static_cast<int>(threadIdx.x);
@@ -735,7 +739,7 @@ int merge_rows_per_block(const KVGeom& g, int elem_size, bool quant) {
 
 void launch_merge(const DescArg& d, int chunk_off, int layer_off, int n_layers, const KVGeom& g, int elem_size,
                   const int32_t* block_table, const uint8_t* k_new, const uint8_t* v_new,
-                  int64_t T, int n_chunks, int64_t n_batches, const int32_t* sel_idx, int kmax, int quant_from,
+                  int64_t T, int n_chunks, const MergeBatches& batches, const int32_t* sel_idx, int kmax, int quant_from,
                   const float* k_scales, const float* v_scales, hipStream_t stream) {
     const bool quant = quant_from >= 0;
     if (merge_fits_rows(g, elem_size, quant)) {
@@ -746,11 +750,13 @@ void launch_merge(const DescArg& d, int chunk_off, int layer_off, int n_layers, 
         const int tok_units = (g.v_off >= 0 ? 2 : 1) * units;
         const int tpb = merge_rows_per_block(g, elem_size, quant);
         const FastDiv dtu(static_cast<uint32_t>(tok_units)), dupr(static_cast<uint32_t>(upr));
+        FastDiv deach(static_cast<uint32_t>(std::max<int64_t>(batches.each, 1)));
+        if (batches.each == 0) deach.d = 0;
         const bool dense = g.sh == g.D;
-        for_layer_minor(n_layers, n_batches, [&](const LayerMinor& lm, unsigned blocks) {
+        for_layer_minor(n_layers, batches.n, [&](const LayerMinor& lm, unsigned blocks) {
 #define DARIC_MR(M, DN) DARIC_LAUNCH((merge_rows_kernel<M, DN>), blocks, kMergeThreads, 0, stream, d, chunk_off, \
                                      layer_off, g, elem_size, block_table, k_new, v_new, T, n_chunks, sel_idx, kmax, \
-                                     tpb, units, dtu, dupr, k_scales, v_scales, lm)
+                                     tpb, units, dtu, dupr, deach, k_scales, v_scales, lm)
             if (!quant) { if (dense) DARIC_MR(kMergeCopy, true); else DARIC_MR(kMergeCopy, false); }
             else if (quant_from == kBF16) { if (dense) DARIC_MR(kMergeFromBF16, true); else DARIC_MR(kMergeFromBF16, false); }
             else { if (dense) DARIC_MR(kMergeFromF16, true); else DARIC_MR(kMergeFromF16, false); }

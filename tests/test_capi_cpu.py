@@ -627,6 +627,28 @@ def test_topk_slots_cover_the_chunk(hosttest, n, lanes):
     assert (slots - 1) * lanes < n <= slots * lanes < 1 << 32
 
 
+@pytest.mark.parametrize("top_k", [0, 1])
+@pytest.mark.parametrize("lens,ks,kmax", [
+    ([40] * 7, [24] * 7, 24), ([40] * 7, [24] * 6 + [8], 24), ([3, 20, 40], [60, 33, 17], 60), ([5, 5], [0, 0], 4),
+    ([9, 9, 9], [0, 9, 9], 9), ([30], [17], 16), ([8, 8, 8], [1, 8, 5], 8),
+])
+def test_merge_batches(hosttest, lens, ks, kmax, top_k):
+    """A batch's chunk by division (chunks of as many batches each) is the last
+    chunk that begins at or before it, which the kernel searches otherwise."""
+    hosttest.daric_hosttest_merge_batches.restype = ctypes.c_int64
+    n, k, begin = np.asarray(lens, np.int32), np.asarray(ks, np.int32), np.zeros(len(lens), np.int32)
+    each = ctypes.c_int64()
+    total = hosttest.daric_hosttest_merge_batches(
+        ctypes.c_void_p(n.ctypes.data), ctypes.c_void_p(k.ctypes.data), ctypes.c_int64(n.size), ctypes.c_int64(kmax),
+        ctypes.c_int(8), ctypes.c_int(top_k), ctypes.c_void_p(begin.ctypes.data), ctypes.byref(each))
+    own = [-(-min(x, y, kmax) // 8) if top_k else -(-min(y, kmax) // 8) for x, y in zip(lens, ks)]
+    assert total == sum(own) and begin.tolist() == [sum(own[:i]) for i in range(len(own))]
+    assert each.value == (own[0] if len(set(own)) == 1 else 0)
+    if each.value:
+        for b in range(total):
+            assert b // each.value == max(i for i in range(len(own)) if begin[i] <= b)
+
+
 def test_segment_forms():
     """Tuples of ints take the short way; every other form numpy's, with the same values and errors."""
     from daric_amd.cache_ops import _segments
