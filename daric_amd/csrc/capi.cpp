@@ -400,15 +400,6 @@ TokenLayout token_layout(const daric_tensor& t, bool page_first) {
     return r;
 }
 
-// Copies whose job descriptors fit in a CU's 16 KiB scalar cache read them from
-// the pinned slot itself: no upload kernel (4-5 us with its gap) before the copy.
-// Same process, MI355X, wall: scatter of 26 layers of one 86-token chunk 16.5 ->
-// 12.3 us, token scatter of 72 jobs onto 24 head-major layers 75.9 -> 71.1 us,
-// gather of 40 jobs 35.1 -> 31.5 us, 185 page jobs (14.5 KiB) 234.8 -> 231.9 us.
-// Larger lists are read over the host link again and again where neighbouring
-// blocks take different jobs: 328 token jobs (36 KiB) 211.6 -> 223.9 us.
-constexpr size_t kDirectDescBytes = 16 * 1024;
-
 int copy_tokens(daric_copier* c, const char* const* names, int64_t n_jobs, const int64_t* offsets,
                 int64_t n_offsets, const int64_t* byte_sizes, int64_t n_byte_sizes,
                 const daric_tensor* indices, const int64_t* indices_offsets,
@@ -493,7 +484,7 @@ int copy_tokens(daric_copier* c, const char* const* names, int64_t n_jobs, const
         DeviceGuard guard(device);
         const hipStream_t st = as_stream(stream);
         const size_t bytes = jobs.size() * sizeof(TokenJob);
-        DescHandOver ho(device, jobs.data(), bytes, st, bytes <= kDirectDescBytes);
+        DescHandOver ho(device, jobs.data(), bytes, st, bytes <= direct_desc_bytes(gather, part_bytes));
         launch_token_copy(ho.arg(), classes, part_bytes, vw, lds, gather, st);
     });
 }
@@ -513,7 +504,9 @@ int copy_pages(daric_copier* c, const char* const* names, int64_t n_jobs, const 
         DeviceGuard guard(r.device);
         const hipStream_t st = as_stream(stream);
         const size_t bytes = r.jobs.size() * sizeof(CopyJob);
-        DescHandOver ho(r.device, r.jobs.data(), bytes, st, bytes <= kDirectDescBytes);
+        int64_t span = 0;
+        for (const CopyJob& j : r.jobs) span = std::max<int64_t>(span, j.span);
+        DescHandOver ho(r.device, r.jobs.data(), bytes, st, bytes <= direct_desc_bytes(gather, std::min(span, part)));
         launch_copy_pages(ho.arg(), classes, part, r.vw, gather, st);
     });
 }
@@ -1033,11 +1026,10 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
                 continue;
             }
             // Job sets too large to travel inline are read by the fused
-            // kernels straight from the pinned slot (one 80-byte read per
-            // workgroup of at least 16 KiB): no upload kernel and no
-            // dependency gap before them, ~4 us less per call on MI355X. The
-            // copy kernels keep the upload: their 8 KiB workgroups are more,
-            // and reading over the host link cost the gather ~5 us.
+            // kernels straight from the pinned slot, whatever their size: no
+            // upload kernel and no dependency gap before them, ~4 us less per
+            // call on MI355X, also where copies fill the host link meanwhile
+            // (64 to 256 jobs, 80 to 320 of 4 KiB pages).
             DescHandOver ho(r.device, gr.jobs.data(), bytes, st, true);
             launch_scatter_rotate(ho.arg(), gr.classes, gr.g, gr.kind, rope->is_neox != 0, rope->inv_freq, st);
         }

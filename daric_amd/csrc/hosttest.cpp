@@ -165,4 +165,8 @@ int64_t daric_hosttest_merge_batches(const int32_t* n_tokens, const int32_t* k, 
     return b.n;
 }
 
+int64_t daric_hosttest_direct_desc_bytes(int gather, int64_t unit_bytes) {
+    return static_cast<int64_t>(daric::direct_desc_bytes(gather != 0, unit_bytes));
+}
+
 }

@@ -606,6 +606,18 @@ def test_page_copies_cut_each_job_by_its_own_span(hosttest):
     assert (units // t).tolist() == [16, 1, 1, 1, 2, 9, 1] * 3
 
 
+# (gather, workgroup's bytes, jobs of 80 bytes read in place, jobs uploaded)
+@pytest.mark.parametrize("gather,unit,direct,uploaded", [
+    (1, 8192, 51, 52), (1, 4096, 40, 96), (0, 8192, 204, 205), (0, 4096, 153, 160), (0, 2048, 72, 160),
+])
+def test_descriptors_read_in_place(hosttest, gather, unit, direct, uploaded):
+    """Job lists that the copies read over the host link: those whose reads cost
+    less than an upload beside copies that fill the link."""
+    hosttest.daric_hosttest_direct_desc_bytes.restype = ctypes.c_int64
+    most = hosttest.daric_hosttest_direct_desc_bytes(ctypes.c_int(gather), ctypes.c_int64(unit))
+    assert 80 * direct <= most < 80 * uploaded
+
+
 @pytest.mark.parametrize("n", range(2, 20, 2))
 def test_store_unit_head_leaves_the_rest_alone(hosttest, n):
     """The in-place rotation of e4m3 rows writes a unit's rotated bytes only:
