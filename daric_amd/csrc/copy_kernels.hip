@@ -377,8 +377,6 @@ __global__ __launch_bounds__(kThreads) void upload_kernel(const u32x4* __restric
     if (i < n16) dst[i] = src[i];
 }
 
-constexpr int64_t kScatterRunsFrom = (128ll << 20) + 1, kFusedRunsFrom = 64ll << 20;   // JobRuns
-
 void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t part, int vw,
                        bool gather, hipStream_t stream) {
     if (classes.empty()) return;
@@ -427,7 +425,8 @@ void launch_scatter_rotate(const DescArg& d, const JobClasses& classes, const Ro
         int lp = 0;
         while ((units >> (lp + 1)) * 16 >= 16384 && units % (2ll << lp) == 0 && (units >> (lp + 1)) % upr == 0)
             ++lp;
-        for_job_runs(classes, 1ll << lp, (units * 16) >> lp, kFusedRunsFrom,
+        const int64_t unit = (units * 16) >> lp;
+        for_job_runs(classes, 1ll << lp, unit, fused_runs_from(unit),
                      [&](int j0, const JobRuns& jr, unsigned blocks) {
 #define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_lane_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq, lp)
             if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
@@ -441,8 +440,8 @@ void launch_scatter_rotate(const DescArg& d, const JobClasses& classes, const Ro
     const RowParts rp(g.n_rows, upr);
     gd.parts = FastDiv(static_cast<uint32_t>(rp.parts));
     gd.part_rows = rp.part_rows;
-    for_job_runs(classes, rp.parts, static_cast<int64_t>(rp.part_rows) * upr * 16,
-                 kFusedRunsFrom, [&](int j0, const JobRuns& jr, unsigned blocks) {
+    const int64_t unit = static_cast<int64_t>(rp.part_rows) * upr * 16;
+    for_job_runs(classes, rp.parts, unit, fused_runs_from(unit), [&](int j0, const JobRuns& jr, unsigned blocks) {
 #define DARIC_SR(K, N, A) DARIC_LAUNCH((scatter_rotate_rows_kernel<K, N, A>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq)
 #define DARIC_SRA(K, N) do { if (g.aligned) DARIC_SR(K, N, true); else DARIC_SR(K, N, false); } while (0)
         if (kind == kBF16) { if (neox) DARIC_SRA(kBF16, true); else DARIC_SRA(kBF16, false); }

@@ -169,4 +169,6 @@ int64_t daric_hosttest_direct_desc_bytes(int gather, int64_t unit_bytes) {
     return static_cast<int64_t>(daric::direct_desc_bytes(gather != 0, unit_bytes));
 }
 
+int64_t daric_hosttest_fused_runs_from(int64_t unit_bytes) { return daric::fused_runs_from(unit_bytes); }
+
 }

@@ -345,11 +345,9 @@ static_assert(sizeof(JobGrid::Class) == 16, "JobGrid::Class layout");
 // 404 -> 381 and 345 -> 332 us; fused fp8 scatter of 1280 jobs 2135 -> 2016 us.
 // Runs of 64 KiB gained half as much and runs of 512 KiB nothing on the
 // fused scatter. Below `runs_from` bytes, where a call's traffic stays mostly in
-// the 256 MB Infinity Cache, runs gained nothing and cost up to 5%: fused scatter
-// 1.00-1.08x from 64 MiB and 0.96-1.02x below, plain scatter 1.00-1.05x above
-// 128 MiB and 0.96-1.00x up to it, token-major scatter 1.01-1.04x from 512 MiB
-// and 0.95-1.02x below 256 MiB (same process, 1 to 80 layers, even and uneven
-// chunks). Fewer than 16 runs per XCD leave some XCDs idle at the end, so such
+// the 256 MB Infinity Cache, runs gained nothing and cost up to 5% (kScatterRunsFrom,
+// fused_runs_from; token-major scatter 0.92-1.04x at 384 MiB, 0.93-1.05x at 512,
+// 0.96-1.05x at 768). Fewer than 16 runs per XCD leave some XCDs idle at the end, so such
 // calls take shorter runs. Runs of one unit are not shifted: units of 72 KiB ran
 // 2.5% slower so.
 struct JobRuns : JobGrid {
@@ -458,6 +456,21 @@ void for_job_runs(const JobClasses& classes, int64_t parts, int64_t unit_bytes, 
         }
         return blocks(g.log2_run);
     }, launch);
+}
+
+// Fewest bytes of a call from which its scatters run in runs (JobRuns). Plain order
+// against runs, MI355X, layers of 8 x 64 fp16, 8 x 96 and 8 x 128 bf16, 8 x 128
+// e4m3, one chunk and four: plain scatter 0.95-1.05x at 64 MiB, 0.97-1.02x at 128,
+// 1.01-1.07x at 160, 0.99-1.05x at 256, 1.00-1.07x from 384.
+constexpr int64_t kScatterRunsFrom = 144ll << 20;
+// Fused scatter with units of 8 KiB and more: 0.95-0.99x at 64 MiB, 0.95-1.02x at
+// 128, 0.97-1.03x at 192, 0.97-1.05x at 256, 0.94-1.05x at 384, 0.96-1.04x at 768
+// (8 x 96 alone behind, 8 x 128 1.01-1.04x). Smaller units never: those of 4 KiB
+// ran 0.75-0.91x from 64 to 256 MiB (96 MiB in four chunks of 80 layers 49 -> 64 us,
+// 56 in the plain order of earlier grids) and 0.90-0.99x at 768, of 2 KiB
+// 0.69-0.95x, since each reads its job over the host link.
+inline int64_t fused_runs_from(int64_t unit_bytes) {
+    return unit_bytes < 8192 ? INT64_MAX : 320ll << 20;
 }
 
 // JobRows launches.

@@ -606,6 +606,18 @@ def test_page_copies_cut_each_job_by_its_own_span(hosttest):
     assert (units // t).tolist() == [16, 1, 1, 1, 2, 9, 1] * 3
 
 
+@pytest.mark.parametrize("unit,mib,runs", [
+    (16384, 1024, True), (8192, 384, True), (8192, 256, False), (16384, 64, False), (4096, 1024, False), (2048, 512, False),
+])
+def test_fused_scatters_in_runs(hosttest, unit, mib, runs):
+    """Fused scatters take the jobs' runs per XCD where calls are large and
+    workgroups not small; the plain order elsewhere."""
+    hosttest.daric_hosttest_fused_runs_from.restype = ctypes.c_int64
+    n_from = hosttest.daric_hosttest_fused_runs_from(ctypes.c_int64(unit))
+    launches, log2_run, _idle = job_grid(hosttest, 0, [(mib << 20) // unit // 64] * 64, 1, unit, n_from)
+    assert launches == 1 and (log2_run > 0) == runs
+
+
 # (gather, workgroup's bytes, jobs of 80 bytes read in place, jobs uploaded)
 @pytest.mark.parametrize("gather,unit,direct,uploaded", [
     (1, 8192, 51, 52), (1, 4096, 40, 96), (0, 8192, 204, 205), (0, 4096, 153, 160), (0, 2048, 72, 160),
