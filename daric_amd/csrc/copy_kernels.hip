@@ -116,8 +116,11 @@ __global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job
 // K+V pages of 64 x 8 x 192 bf16 99 -> 69 us. Rotary halves inside a unit took a
 // scatter and a pass per layer before: 18 layers, 8 heads of 80 with 40 rotated,
 // 22000 tokens 686 -> 362 us in one launch instead of 19.
+// Eight wavefronts per SIMD: the compiler took 66 to 68 registers of its own accord,
+// seven wavefronts (fp16 pairs of 96 in K+V pages 30.1 -> 29.0 us, 80 layers of 1 x
+// 192 bf16 82.7 -> 75.5).
 template <int KIND, bool NEOX, bool ALIGNED>
-__global__ __launch_bounds__(kThreads) void scatter_rotate_rows_kernel(
+__global__ __launch_bounds__(kThreads, 8) void scatter_rotate_rows_kernel(
     DescArg d, int job0, JobRuns jr, RowGeomDiv gd, const float* __restrict__ inv_freq) {
     static_assert(kThreads == kRowThreads && kRowPartUnits == kRowUnits, "one part per workgroup");
     using RR = RowRotation<KIND, NEOX, ALIGNED>;
