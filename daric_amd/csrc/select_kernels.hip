@@ -700,18 +700,23 @@ void launch_deviation(const DescArg& d, int layer_off, int n_layers, const KVGeo
 // lanes, so beyond one per CU those of up to 8192 tokens take 512 lanes: 512
 // chunks of 3000 tokens 17.4 -> 14.5 us, 3200 of 2100 tokens 84.9 -> 47.6 (256
 // lanes over keys in LDS: 59.7), 3200 of 8000 168 -> 109; at 256 chunks of 8000
-// they would take 19.4 instead of 14.9 (MI355X).
+// they would take 19.4 instead of 14.9. Chunks read from memory again in each pass
+// need fewer registers and fit twice; from 1024 of them on 512 lanes each: 1280 of
+// 40000 tokens 475 -> 373 us, 3200 of 40000 1248 -> 940 (256 lanes and four passes:
+// 1136), 4096 of 33000 1296 -> 927 (1099), where 1024 of 100000 would take 1079
+// instead of 990 (MI355X).
 void launch_topk(const float* keys, int n_layers, int64_t T, const DescArg& d,
                  int n_chunks, int max_tokens, int32_t* out_idx, int kmax, hipStream_t stream) {
-    const bool many = static_cast<int64_t>(n_chunks) * n_layers > 256;
+    const int64_t groups = static_cast<int64_t>(n_chunks) * n_layers;
     for (int l0 = 0; l0 < n_layers; l0 += kMaxGridYZ) {
         const dim3 grid(static_cast<unsigned>(n_chunks), static_cast<unsigned>(std::min(kMaxGridYZ, n_layers - l0)));
 #define DARIC_TK(TH, KPT) DARIC_LAUNCH((topk_kernel<TH, KPT>), grid, TH, 0, stream, keys, T, d, n_chunks, out_idx, kmax, l0)
         if (max_tokens <= kTopkWave) DARIC_TK(64, kTopkWave / 64);
         else if (max_tokens <= kTopkGroup) DARIC_TK(256, kTopkGroup / 256);
-        else if (max_tokens <= 8192 && many) DARIC_TK(512, 16);
+        else if (max_tokens <= 8192 && groups > 256) DARIC_TK(512, 16);
         else if (max_tokens <= 8192) DARIC_TK(1024, 8);
         else if (max_tokens <= 32768) DARIC_TK(1024, 32);
+        else if (groups > 1024) DARIC_TK(512, 0);
         else DARIC_TK(1024, 0);
 #undef DARIC_TK
         check_launch("topk_per_chunk");

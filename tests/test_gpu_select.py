@@ -208,9 +208,10 @@ def test_topk_workgroup_edges(dev, n, kind):
     assert np.array_equal(got.cpu().numpy(), want)
 
 
-# More chunks than CUs, where those of up to 8192 tokens take fewer lanes; they
-# share rows.
-@pytest.mark.parametrize("n_chunks,longest", [(128, 4097), (129, 2049), (129, 4097), (129, 8192), (129, 8193)])
+# More chunks than CUs, where those of up to 8192 tokens take fewer lanes, and four
+# times as many, where those of more than 32768 do; they share rows.
+@pytest.mark.parametrize("n_chunks,longest", [(128, 4097), (129, 2049), (129, 4097), (129, 8192), (129, 8193),
+                                              (512, 32769), (513, 32769), (513, 40001)])
 def test_topk_of_many_long_chunks(dev, n_chunks, longest):
     rng = np.random.default_rng(longest)
     keys = np.stack([topk_keys(kind, rng, longest + n_chunks) for kind in ("spread", "few")])
