@@ -516,17 +516,21 @@ struct alignas(16) TokenJob {
 static_assert(sizeof(TokenJob) == 112, "TokenJob layout");
 
 // Tokens of a part of a page (one of K or V) of PS tokens of tok_bytes each, for
-// the row kernel with accesses of vw bytes: 8 KiB, two accesses per lane, up to a
-// quarter more where that saves a part, and parts of a page equal in size; pages
-// of up to 28 KiB in one part or two, of up to 14 KiB. Against 16 KiB (MI355X):
-// 1.00-1.13x on gathers, 0.95-1.13x on scatters; 4 KiB 0.7-1.05x. Gathers of 400
-// MiB in pages of 11, 12, 13, 14 and 28 KiB, against 16 KiB: 1.05, 1.04, 1.04,
-// 1.03 and 1.02x, where parts of up to 10 KiB left them two parts or four and 0.88,
-// 0.91, 0.91, 0.97 and 0.96x; 24 KiB 1.15x for 1.10x, 16 KiB 1.07x in two parts
-// and 1.02x in one, 32 KiB 1.07x in four and 1.02x in two.
+// the row kernel with accesses of vw bytes: 8 KiB, two accesses per lane, where whole
+// tokens make them up, else up to a quarter more where that saves a part, and parts
+// of a page equal in size; pages of up to 28 KiB in one part or two, of up to 14
+// KiB. Against 16 KiB (MI355X): 1.00-1.13x on gathers, 0.95-1.13x on scatters; 4 KiB
+// 0.7-1.05x. Gathers of 400 MiB in pages of 11, 12, 13, 14 and 28 KiB, against 16
+// KiB: 1.05, 1.04, 1.04, 1.03 and 1.02x, where parts of up to 10 KiB left them two
+// parts or four and 0.88, 0.91, 0.91, 0.97 and 0.96x; 24 KiB 1.15x for 1.10x, 16 KiB
+// 1.07x in two parts and 1.02x in one, 32 KiB 1.07x in four and 1.02x in two. Pages
+// of 64, 96, 128 and 512 KiB of 512- and 2048-byte tokens, gathers and scatters of
+// 300 MiB: 1.02-1.03, 1.06, 1.01 and 1.06x, 1.06, 1.06, 1.07 and 1.02x, in parts of
+// 10 KiB 0.98-1.00, 1.04, 1.00 and 1.05x, 1.03, 1.04, 1.03 and 1.02x; tokens of
+// 576 to 3072 bytes ran up to 1.13x faster in parts of up to 10 KiB than of 8.
 inline int64_t token_row_part(int64_t PS, int64_t tok_bytes, int vw) {
-    constexpr int64_t kPart = 10 * 1024, kMost = 14 * 1024;
-    const int64_t bytes = vw != 16 ? 4096 : PS * tok_bytes <= 2 * kMost ? kMost : kPart;
+    constexpr int64_t kPart = 10 * 1024, kEven = 8 * 1024, kMost = 14 * 1024;
+    const int64_t bytes = vw != 16 ? 4096 : PS * tok_bytes <= 2 * kMost ? kMost : kEven % tok_bytes == 0 ? kEven : kPart;
     const int64_t most = std::min<int64_t>(PS, std::max<int64_t>(1, bytes / tok_bytes));
     const int64_t parts = (PS + most - 1) / most;
     return (PS + parts - 1) / parts;

@@ -586,7 +586,7 @@ def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
 # (tokens of a page, bytes of a token, access width, tokens of a part)
 @pytest.mark.parametrize("ps,tok,vw,want", [
     (16, 576, 16, 16), (16, 768, 16, 16), (16, 896, 16, 16), (16, 912, 16, 8), (16, 1024, 16, 8), (16, 1792, 16, 8),
-    (16, 2048, 16, 4), (64, 1152, 16, 8), (65, 160, 16, 65), (3, 10368, 16, 1), (1, 70000, 16, 1), (16, 768, 1, 4),
+    (16, 2048, 16, 4), (256, 2048, 16, 4), (37, 2048, 16, 4), (128, 512, 16, 16), (64, 1152, 16, 8), (65, 160, 16, 65), (3, 10368, 16, 1), (1, 70000, 16, 1), (16, 768, 1, 4),
     (16, 5000, 1, 1), (5, 16, 16, 5),
 ])
 def test_token_row_parts(hosttest, ps, tok, vw, want):
