@@ -457,7 +457,9 @@ int copy_tokens(daric_copier* c, const char* const* names, int64_t n_jobs, const
         };
         const TokenJob* like = nullptr;     // job whose geometry the last one had: no divisions again
         for (TokenJob& j : jobs) {
-            if (like != nullptr && like->H == j.H && like->row_bytes == j.row_bytes && like->PS == j.PS) {
+            const int64_t pages = static_cast<int64_t>(j.n_kv) * j.n_sel;
+            if (like != nullptr && like->H == j.H && like->row_bytes == j.row_bytes && like->PS == j.PS &&
+                pages * like->parts_per_page <= kMaxTiles) {
                 j.part_tokens = like->part_tokens;
                 j.parts_per_page = like->parts_per_page;
                 j.d_upr = like->d_upr;
@@ -467,7 +469,7 @@ int copy_tokens(daric_copier* c, const char* const* names, int64_t n_jobs, const
                 const int64_t head_units = static_cast<int64_t>(j.H) * row_units;
                 const int64_t tok_bytes = static_cast<int64_t>(j.H) * j.row_bytes;
                 const int64_t pt = lds ? std::min<int64_t>(j.PS, std::max<int64_t>(1, 512 / head_units))   // 8 KiB of LDS
-                                       : token_row_part(j.PS, tok_bytes, vw);
+                                       : token_row_part(j.PS, tok_bytes, vw, pages);
                 const int64_t parts = (j.PS + pt - 1) / pt;
                 DARIC_CHECK(pt * head_units <= kIntMax, "page part exceeds int range");
                 j.part_tokens = static_cast<int32_t>(pt);

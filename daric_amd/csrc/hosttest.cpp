@@ -124,8 +124,8 @@ void daric_hosttest_store_unit_head(uint8_t* dst, const uint32_t* words, int n) 
     daric::store_unit_head(dst, words, n);
 }
 
-int64_t daric_hosttest_token_row_part(int64_t page_tokens, int64_t tok_bytes, int vw) {
-    return daric::token_row_part(page_tokens, tok_bytes, vw);
+int64_t daric_hosttest_token_row_part(int64_t page_tokens, int64_t tok_bytes, int vw, int64_t pages) {
+    return daric::token_row_part(page_tokens, tok_bytes, vw, pages);
 }
 
 int daric_hosttest_topk_slots(int n, int lanes) { return daric::topk_slots(n, lanes); }

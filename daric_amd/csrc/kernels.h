@@ -528,11 +528,13 @@ static_assert(sizeof(TokenJob) == 112, "TokenJob layout");
 // 300 MiB: 1.02-1.03, 1.06, 1.01 and 1.06x, 1.06, 1.06, 1.07 and 1.02x, in parts of
 // 10 KiB 0.98-1.00, 1.04, 1.00 and 1.05x, 1.03, 1.04, 1.03 and 1.02x; tokens of
 // 576 to 3072 bytes ran up to 1.13x faster in parts of up to 10 KiB than of 8.
-inline int64_t token_row_part(int64_t PS, int64_t tok_bytes, int vw) {
-    constexpr int64_t kPart = 10 * 1024, kEven = 8 * 1024, kMost = 14 * 1024;
+// A job of `pages` pages whose parts would not fit one launch takes parts of 16 KiB.
+inline int64_t token_row_part(int64_t PS, int64_t tok_bytes, int vw, int64_t pages) {
+    constexpr int64_t kPart = 10 * 1024, kEven = 8 * 1024, kMost = 14 * 1024, kLongest = 16 * 1024;
     const int64_t bytes = vw != 16 ? 4096 : PS * tok_bytes <= 2 * kMost ? kMost : kEven % tok_bytes == 0 ? kEven : kPart;
     const int64_t most = std::min<int64_t>(PS, std::max<int64_t>(1, bytes / tok_bytes));
     const int64_t parts = (PS + most - 1) / most;
+    if (vw == 16 && parts * pages > kMaxGridBlocks) return std::min<int64_t>(PS, std::max<int64_t>(1, kLongest / tok_bytes));
     return (PS + parts - 1) / parts;
 }
 

@@ -591,7 +591,20 @@ def test_page_parts_end_and_fit_a_launch(hosttest, span, tiles):
 ])
 def test_token_row_parts(hosttest, ps, tok, vw, want):
     hosttest.daric_hosttest_token_row_part.restype = ctypes.c_int64
-    assert hosttest.daric_hosttest_token_row_part(ctypes.c_int64(ps), ctypes.c_int64(tok), ctypes.c_int(vw)) == want
+    assert hosttest.daric_hosttest_token_row_part(ctypes.c_int64(ps), ctypes.c_int64(tok), ctypes.c_int(vw),
+                                                  ctypes.c_int64(8)) == want
+
+
+@pytest.mark.parametrize("ps,tok", [(16, 2048), (64, 1152), (16, 912), (256, 2048), (3, 10368), (65, 160)])
+def test_token_rows_take_jobs_of_2_24_parts(hosttest, ps, tok):
+    """A job of as many pages as fit one launch in parts of 16 KiB is accepted:
+    parts of a smaller target give way to those."""
+    hosttest.daric_hosttest_token_row_part.restype = ctypes.c_int64
+    longest = min(ps, max(1, 16384 // tok))
+    pages = ((1 << 24) - 1) // -(-ps // longest)
+    part = hosttest.daric_hosttest_token_row_part(ctypes.c_int64(ps), ctypes.c_int64(tok), ctypes.c_int(16),
+                                                  ctypes.c_int64(pages))
+    assert -(-ps // part) * pages < 1 << 24
 
 
 def test_page_copies_cut_each_job_by_its_own_span(hosttest):
