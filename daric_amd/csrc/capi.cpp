@@ -990,7 +990,10 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
             scatter_then_rotate(r, indices, indices_offsets, deltas, num_tokens, rope, stream);
             return;
         }
-        for (Group& gr : groups) gr.classes = order_jobs(gr.jobs, tiles_of);
+        for (Group& gr : groups) {
+            split_long_jobs(gr.jobs, FusedCut(gr.g, gr.kind == kE4M3 ? 16 : 8).parts, gr.g.PS);
+            gr.classes = order_jobs(gr.jobs, tiles_of);
+        }
         // Allocation-free variant: job sets that do not travel inline are
         // staged in the static scratch array, one region per launch group.
         size_t staged = 0;

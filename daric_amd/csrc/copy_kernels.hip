@@ -414,22 +414,12 @@ void launch_scatter_rotate(const DescArg& d, const JobClasses& classes, const Ro
     gd.g = g;
     gd.tok_div = FastDiv(static_cast<uint32_t>(g.tok_div));
     gd.ps = FastDiv(static_cast<uint32_t>(g.PS));
-    const int upr = g.W / (kind == kE4M3 ? 16 : 8);
-    gd.upr = FastDiv(static_cast<uint32_t>(upr));
-    const int64_t units = static_cast<int64_t>(g.n_rows) * upr;   // 16-byte units per page span
-    // The lane-exchange kernel needs whole rows inside a wavefront and pair
-    // halves of whole units; the rows kernel takes the other rows.
-    if (g.aligned && 64 % upr == 0) {
-        // Pages cut into parts of at least 16 KiB, whole rows each. Two 16 KiB
-        // halves of the 32 KiB bf16 pages measured ~1% faster than whole pages
-        // at config 2, kernel and whole call alike (347.2 against 350.2 us per
-        // kernel, 347.5 against 350.7 us per call; bit-identical output);
-        // 8 KiB parts were 4% slower.
-        int lp = 0;
-        while ((units >> (lp + 1)) * 16 >= 16384 && units % (2ll << lp) == 0 && (units >> (lp + 1)) % upr == 0)
-            ++lp;
-        const int64_t unit = (units * 16) >> lp;
-        for_job_runs(classes, 1ll << lp, unit, fused_runs_from(unit),
+    const int unit_elems = kind == kE4M3 ? 16 : 8;
+    gd.upr = FastDiv(static_cast<uint32_t>(g.W / unit_elems));
+    const FusedCut cut(g, unit_elems);
+    const int lp = cut.log2_parts;
+    if (cut.lane) {
+        for_job_runs(classes, cut.parts, cut.unit_bytes, fused_runs_from(cut.unit_bytes),
                      [&](int j0, const JobRuns& jr, unsigned blocks) {
 #define DARIC_SR(K, N) DARIC_LAUNCH((scatter_rotate_lane_kernel<K, N>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq, lp)
             if (kind == kBF16) { if (neox) DARIC_SR(kBF16, true); else DARIC_SR(kBF16, false); }
@@ -440,11 +430,10 @@ void launch_scatter_rotate(const DescArg& d, const JobClasses& classes, const Ro
         });
         return;
     }
-    const RowParts rp(g.n_rows, upr);
-    gd.parts = FastDiv(static_cast<uint32_t>(rp.parts));
-    gd.part_rows = rp.part_rows;
-    const int64_t unit = static_cast<int64_t>(rp.part_rows) * upr * 16;
-    for_job_runs(classes, rp.parts, unit, fused_runs_from(unit), [&](int j0, const JobRuns& jr, unsigned blocks) {
+    gd.parts = FastDiv(static_cast<uint32_t>(cut.parts));
+    gd.part_rows = static_cast<int32_t>(cut.part_rows);
+    for_job_runs(classes, cut.parts, cut.unit_bytes, fused_runs_from(cut.unit_bytes),
+                 [&](int j0, const JobRuns& jr, unsigned blocks) {
 #define DARIC_SR(K, N, A) DARIC_LAUNCH((scatter_rotate_rows_kernel<K, N, A>), blocks, kThreads, 0, stream, d, j0, jr, gd, inv_freq)
 #define DARIC_SRA(K, N) do { if (g.aligned) DARIC_SR(K, N, true); else DARIC_SR(K, N, false); } while (0)
         if (kind == kBF16) { if (neox) DARIC_SRA(kBF16, true); else DARIC_SRA(kBF16, false); }

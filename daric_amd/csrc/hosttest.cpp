@@ -171,4 +171,43 @@ int64_t daric_hosttest_direct_desc_bytes(int gather, int64_t unit_bytes) {
 
 int64_t daric_hosttest_fused_runs_from(int64_t unit_bytes) { return daric::fused_runs_from(unit_bytes); }
 
+// Splits one job (split_long_jobs) and lists, for every tile of the pieces in
+// order, the page span it takes: place in the layer before the page id, place in
+// staging, place in the id list and tokens it rotates (-1: copied). Returns the
+// tiles, or -1 where a piece has more units than a launch holds.
+int64_t daric_hosttest_split_job(int prefix, int n_sel, int64_t prefix_stride, int span, int n_tokens, int64_t parts,
+                                 int64_t page_tokens, int64_t* out, int64_t cap) {
+    uint8_t base[1];
+    const int32_t ids[1] = {0};
+    daric::CopyJob j{};
+    j.layer = base;
+    j.stage = base;
+    j.idx = ids;
+    j.prefix = prefix;
+    j.n_sel = n_sel;
+    j.prefix_stride = prefix_stride;
+    j.span = span;
+    j.n_tokens = n_tokens;
+    j.delta = 3.0f;
+    std::vector<daric::CopyJob> jobs(3, j);
+    jobs[0].n_sel = jobs[2].n_sel = 1;
+    jobs[0].prefix = jobs[2].prefix = 1;
+    daric::split_long_jobs(jobs, parts, page_tokens);
+    if (jobs.front().n_sel != 1 || jobs.back().n_sel != 1) return -2;
+    int64_t n = 0;
+    for (size_t i = 1; i + 1 < jobs.size(); ++i) {
+        const daric::CopyJob& q = jobs[i];
+        if (static_cast<int64_t>(q.prefix) * q.n_sel * parts > daric::kMaxGridBlocks) return -1;
+        for (int64_t t = 0; t < static_cast<int64_t>(q.prefix) * q.n_sel && n < cap; ++t, ++n) {
+            const int64_t p = t / q.n_sel, s = t % q.n_sel;
+            out[4 * n] = reinterpret_cast<intptr_t>(q.layer) - reinterpret_cast<intptr_t>(base) + p * q.prefix_stride;
+            out[4 * n + 1] = reinterpret_cast<intptr_t>(q.stage) - reinterpret_cast<intptr_t>(base) + t * q.span;
+            out[4 * n + 2] = (reinterpret_cast<intptr_t>(q.idx) - reinterpret_cast<intptr_t>(ids)) / 4 + s;
+            const int64_t left = q.n_tokens - s * page_tokens;
+            out[4 * n + 3] = p == 0 && q.delta != 0.0f && left > 0 ? (left < page_tokens ? left : page_tokens) : -1;
+        }
+    }
+    return n;
+}
+
 }

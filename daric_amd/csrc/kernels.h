@@ -252,6 +252,70 @@ inline int64_t page_part_bytes(int64_t span, int64_t tiles) {
     return part;
 }
 
+// Parts of a page span in the fused scatter, whose jobs share a row geometry; lane:
+// the lane-exchange kernel (whole rows inside a wavefront, pair halves of whole
+// units), log2_parts of its pages. The rows kernel takes the other rows. unit_elems:
+// values in 16 bytes.
+struct FusedCut {
+    bool lane;
+    int log2_parts = 0;
+    int64_t parts, unit_bytes, part_rows = 0;
+    FusedCut(const RowGeom& g, int unit_elems) {
+        const int upr = g.W / unit_elems;
+        const int64_t units = static_cast<int64_t>(g.n_rows) * upr;   // 16-byte units per page span
+        lane = g.aligned && 64 % upr == 0;
+        if (lane) {
+            // Pages cut into parts of at least 16 KiB, whole rows each. Two 16 KiB
+            // halves of the 32 KiB bf16 pages measured ~1% faster than whole pages
+            // at config 2, kernel and whole call alike (347.2 against 350.2 us per
+            // kernel, 347.5 against 350.7 us per call; bit-identical output);
+            // 8 KiB parts were 4% slower.
+            while ((units >> (log2_parts + 1)) * 16 >= 16384 && units % (2ll << log2_parts) == 0 &&
+                   (units >> (log2_parts + 1)) % upr == 0)
+                ++log2_parts;
+            parts = 1ll << log2_parts;
+            unit_bytes = (units * 16) >> log2_parts;
+        } else {
+            const RowParts rp(g.n_rows, upr);
+            parts = rp.parts;
+            part_rows = rp.part_rows;
+            unit_bytes = part_rows * upr * 16;
+        }
+    }
+};
+
+// Jobs of the fused scatter whose parts would not fit one launch (2^24 - 1 pages of
+// two parts and more) go as several: of consecutive pages, of K and of V apart. V's
+// are copied, which a delta of 0 asks for; PS: tokens of a page.
+inline void split_long_jobs(std::vector<CopyJob>& jobs, int64_t parts, int64_t PS) {
+    const int64_t most = std::max<int64_t>(1, kMaxGridBlocks / parts);
+    std::vector<CopyJob> out;
+    for (size_t i = 0; i < jobs.size(); ++i) {
+        const CopyJob& j = jobs[i];
+        const bool fits = static_cast<int64_t>(j.prefix) * j.n_sel <= most;
+        if (fits && out.empty()) continue;
+        if (out.empty()) out.assign(jobs.begin(), jobs.begin() + static_cast<std::ptrdiff_t>(i));
+        if (fits) {
+            out.push_back(j);
+            continue;
+        }
+        for (int64_t p = 0; p < j.prefix; ++p) {
+            for (int64_t s = 0; s < j.n_sel; s += most) {
+                CopyJob piece = j;
+                piece.layer += p * j.prefix_stride;
+                piece.stage += (p * j.n_sel + s) * j.span;
+                piece.idx += s;
+                piece.prefix = 1;
+                piece.n_sel = static_cast<int32_t>(std::min<int64_t>(most, j.n_sel - s));
+                piece.n_tokens = static_cast<int32_t>(std::max<int64_t>(0, j.n_tokens - s * PS));
+                if (p > 0) piece.delta = 0.0f;
+                out.push_back(piece);
+            }
+        }
+    }
+    if (!out.empty()) jobs.swap(out);
+}
+
 // Cuts the jobs' tiles into parts for accesses of vw bytes and orders the jobs by
 // their parts. *part gets the longest part's bytes.
 inline JobClasses cut_pages(std::vector<CopyJob>& jobs, int vw, int64_t* part) {

@@ -631,6 +631,29 @@ def test_fused_scatters_in_runs(hosttest, unit, mib, runs):
     assert launches == 1 and (log2_run > 0) == runs
 
 
+@pytest.mark.parametrize("prefix,n_sel,tokens,parts", [
+    (2, 10, 150, (1 << 24) // 4), (2, 10, 160, (1 << 24) // 19), (1, 10, 33, (1 << 24) // 3), (2, 1, 5, 1 << 23),
+    (2, 7, 0, 1 << 22), (2, 10, 150, 2), (1, 1, 9, (1 << 24) - 1),
+])
+def test_long_jobs_of_the_fused_scatter_split(hosttest, prefix, n_sel, tokens, parts):
+    """A job whose parts exceed a launch goes as several that take the same page
+    spans, rotate the same tokens of K and copy V."""
+    hosttest.daric_hosttest_split_job.restype = ctypes.c_int64
+    cap, span, stride, ps = 64, 48, 100_000, 16
+
+    def spans(parts):
+        out = np.zeros((cap, 4), np.int64)
+        n = hosttest.daric_hosttest_split_job(
+            ctypes.c_int(prefix), ctypes.c_int(n_sel), ctypes.c_int64(stride), ctypes.c_int(span), ctypes.c_int(tokens),
+            ctypes.c_int64(parts), ctypes.c_int64(ps), ctypes.c_void_p(out.ctypes.data), ctypes.c_int64(cap))
+        return n, out[:max(n, 0)].tolist()
+    n, got = spans(parts)
+    want = [[p * stride, (p * n_sel + s) * span, s,
+             min(ps, tokens - s * ps) if p == 0 and tokens > s * ps else -1]
+            for p in range(prefix) for s in range(n_sel)]
+    assert n == prefix * n_sel and got == want == spans(1)[1]
+
+
 # (gather, workgroup's bytes, jobs of 80 bytes read in place, jobs uploaded)
 @pytest.mark.parametrize("gather,unit,direct,uploaded", [
     (1, 8192, 51, 52), (1, 4096, 40, 96), (0, 8192, 204, 205), (0, 4096, 153, 160), (0, 2048, 72, 160),
