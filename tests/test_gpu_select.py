@@ -396,13 +396,14 @@ def test_allocated_keys_cover_rows(dev, moved, one_call):
     assert np.array_equal(keys.cpu().numpy().view(np.uint32), np.asarray(want, np.float32).view(np.uint32))
 
 
-def test_topk_chunk_longer_than_lds_budget(dev):
-    """A 20000-token chunk (past the 8192 tokens whose keys the kernel stages
-    in LDS) and a short one in the same call: the long chunk's keys are read
-    from global memory in every pass; indices bit-exact, ties to the lower
-    index (the keys repeat every 97 tokens)."""
+@pytest.mark.parametrize("n_long", [20000, 50000])
+def test_topk_chunk_longer_than_lds_budget(dev, n_long):
+    """A chunk of 20000 tokens, whose keys a workgroup of 1024 lanes holds in
+    registers, or of 50000, whose keys are read from memory in every pass,
+    beside a short one; indices bit-exact, ties to the lower index (the keys
+    repeat every 97 tokens)."""
     rng = np.random.default_rng(11)
-    n_long, n_short = 20000, 300
+    n_short = 300
     base = rng.standard_normal(97).astype(np.float32) ** 2
     keys = np.concatenate([np.tile(base, n_long // 97 + 1)[:n_long],
                            rng.standard_normal(n_short).astype(np.float32) ** 2])[None, :].repeat(2, 0)
@@ -528,9 +529,9 @@ def test_select_merge_fp8_cache(dev, row_dtype, one_pass):
 
 
 def test_select_merge_long_chunk_takes_three_launches(dev):
-    """A 9000-token chunk (past the 8192 keys the fused kernel holds in LDS)
-    beside a short one: the call runs deviation, top-k and merge in turn, with
-    the same results."""
+    """A 9000-token chunk (past the 2048 keys whose top-k the fused kernel
+    takes) beside a short one: the call runs deviation, top-k and merge in
+    turn, with the same results."""
     layers, pf, bt, chunks, k_new, v_new = setup_case(dev, "nhd", nb=600, h=2, d=64, L=1,
                                                       chunk_tokens=(9000, 120), seed=9)
     cpu = [t for t, _ in layers]
@@ -543,6 +544,52 @@ def test_select_merge_long_chunk_takes_three_launches(dev):
     assert np.array_equal(keys_g.cpu().numpy().view(np.uint32), keys_o.view(np.uint32))
     assert np.array_equal(sel_g.cpu().numpy(), sel_o)
     assert same_bytes(gpu[0], cpu[0])
+
+
+@pytest.mark.parametrize("mode", ["default", "keys_ready", "one_pass"])
+@pytest.mark.parametrize("n", [2047, 2048, 2049])
+def test_select_merge_at_the_fused_limit(dev, n, mode):
+    """Chunks of 2048 tokens are the longest of the fused forms: one below, at
+    and one past them, beside short chunks."""
+    layers, pf, bt, chunks, k_new, v_new = setup_case(dev, "nhd", nb=300, h=1, d=64, L=2, chunk_tokens=(n, 40, 500),
+                                                      seed=n)
+    cpu = [t for t, _ in layers]
+    gpu = [to_dev(t, dev) for t in cpu]
+    btd = torch.from_numpy(bt).to(dev)
+    kmax = max(c[3] for c in chunks)
+    keys_o, sel_o = _oracle_selection(cpu, pf, bt, k_new, v_new, chunks, kmax)
+    keys = cache_ops.kv_deviation(gpu, pf, btd, k_new.to(dev), chunks) if mode == "keys_ready" else None
+    keys_g, sel_g = cache_ops.select_merge(gpu, pf, btd, k_new.to(dev), v_new.to(dev), chunks, keys=keys,
+                                           keys_ready=mode == "keys_ready", one_pass=mode == "one_pass")
+    torch.cuda.synchronize()
+    assert np.array_equal(keys_g.cpu().numpy().view(np.uint32), keys_o.view(np.uint32))
+    assert np.array_equal(sel_g.cpu().numpy(), sel_o)
+    for t, td in zip(cpu, gpu):
+        assert same_bytes(td, t)
+
+
+@pytest.mark.parametrize("n_chunks,even", [(8, False), (60, False), (60, True), (100, False), (100, True)])
+def test_select_merge_batch_tables(dev, n_chunks, even):
+    """One chunk of 2100 tokens keeps the call from the fused form. The merge's
+    batches of 8 chunks travel with the call's, of 60 in arguments of their own,
+    of 100 in the ring; uneven counts, some 0, or two of every chunk."""
+    rng = np.random.default_rng(n_chunks)
+    lens = [2100] + [int(n) for n in rng.integers(8, 50, n_chunks - 1)]
+    layers, pf, bt, chunks, k_new, v_new = setup_case(dev, "nhd", nb=700, h=2, d=128, L=2, chunk_tokens=tuple(lens),
+                                                      seed=n_chunks)
+    ks = [2] * n_chunks if even else [int(rng.integers(0, min(n, 600) + 1)) * (i % 5 != 3) for i, n in enumerate(lens)]
+    chunks = [c[:3] + (k,) for c, k in zip(chunks, ks)]
+    cpu = [t for t, _ in layers]
+    gpu = [to_dev(t, dev) for t in cpu]
+    kmax = max(ks)
+    keys_o, sel_o = _oracle_selection(cpu, pf, bt, k_new, v_new, chunks, kmax)
+    keys_g, sel_g = cache_ops.select_merge(gpu, pf, torch.from_numpy(bt).to(dev), k_new.to(dev), v_new.to(dev),
+                                           chunks)
+    torch.cuda.synchronize()
+    assert np.array_equal(keys_g.cpu().numpy().view(np.uint32), keys_o.view(np.uint32))
+    assert np.array_equal(sel_g.cpu().numpy(), sel_o)
+    for t, td in zip(cpu, gpu):
+        assert same_bytes(td, t)
 
 
 @pytest.mark.parametrize("one_pass", [False, True])
