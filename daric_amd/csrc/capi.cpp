@@ -1483,7 +1483,8 @@ int daric_select_merge(const daric_tensor* layers, int64_t n_layers, int page_fi
             return;
         }
         // the same work as three launches (chunks longer than the fused
-        // kernel's LDS holds, or rows it does not take)
+        // kernel's registers hold, more selected rows than it handles well, or
+        // rows it does not take)
         if (!keys_ready && c.tiles > 0)
             launch_deviation(ho.arg(), static_cast<int>(cb), static_cast<int>(n_layers), g, ck, btp, kn, nk, T,
                              static_cast<int>(n_chunks), static_cast<int>(c.tiles), quant ? ksc : nullptr, kd, st);

@@ -8,11 +8,11 @@
 // stores are nontemporal: every byte is touched once.
 //
 // Block order (measured on MI355X at the Llama-3-8B shape): both directions
-// cut each tile into parts of 8 KiB. The scatter direction and the fused
-// scatter + rotation deal runs of 128 KiB of each job to the XCDs (JobRuns);
-// the gather direction runs job by job, tile by tile (JobRows), which sustained
-// ~6.3 TB/s (256 jobs of 64 pages) and 5.8-6.0 TB/s (32 of 4096), against
-// 5.5-5.6 TB/s for whole-tile workgroups and job-minor orders.
+// cut each tile into parts of 8 KiB (page_part_bytes). In large calls the scatter
+// direction and the fused scatter + rotation deal runs of 128 KiB of each job to
+// the XCDs (JobRuns); the gather direction runs job by job, tile by tile (JobRows),
+// which sustained ~6.3 TB/s (256 jobs of 64 pages) and 5.8-6.0 TB/s (32 of 4096),
+// against 5.5-5.6 TB/s for whole-tile workgroups and job-minor orders.
 //
 // Pages whose block id is 0 (vLLM's null block) are skipped, as the
 // reference's kernels skip them (csrc/cache_ops/kernels.cu:26,39,69,79,104,117);

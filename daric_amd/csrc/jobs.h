@@ -84,7 +84,6 @@ __device__ __forceinline__ T desc_load(DescPtr<T> p) {
 }
 // Has the listed kernel arguments (up to 8 words or pointers) in registers before
 // what follows, so that their loads share one round trip.
-#define DARIC_ARGS_TOGETHER2(a, b) asm volatile("" ::"s"(a), "s"(b))
 #define DARIC_ARGS_TOGETHER4(a, b, c, d) asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d))
 #define DARIC_ARGS_TOGETHER6(a, b, c, d, e, f) asm volatile("" ::"s"(a), "s"(b), "s"(c), "s"(d), "s"(e), "s"(f))
 // Reads one value of a list that every lane of the workgroup reads at the same

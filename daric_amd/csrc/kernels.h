@@ -231,9 +231,9 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
 }
 
 // Bytes of the parts that a page copy cuts its tiles into, the last part of a
-// tile what is left, for a job of `tiles` tiles of `span` bytes: one up to 11 KiB, two equal ones up to 16 KiB, then 8 KiB (two
-// accesses of 16 bytes per lane), and more where a job's parts would not fit in
-// one launch. A part as long as the tile ends the doubling: a job of up to
+// tile what is left, for a job of `tiles` tiles of `span` bytes: one up to 11 KiB,
+// two equal ones up to 16 KiB, then 8 KiB (two accesses of 16 bytes per lane), and
+// more where a job's parts would not fit in one launch. A part as long as the tile ends the doubling: a job of up to
 // kMaxGridBlocks tiles then has a workgroup per tile. Each job is cut by its own
 // span: by the call's largest, 60 layers of 8 KiB pages beside 4 of 128 KiB had
 // 16 workgroups to each of their pages, 15 of them idle (gather of 584 MiB 645 ->
