@@ -527,14 +527,15 @@ void for_job_runs(const JobClasses& classes, int64_t parts, int64_t unit_bytes, 
 // e4m3, one chunk and four: plain scatter 0.95-1.05x at 64 MiB, 0.97-1.02x at 128,
 // 1.01-1.07x at 160, 0.99-1.05x at 256, 1.00-1.07x from 384.
 constexpr int64_t kScatterRunsFrom = 144ll << 20;
-// Fused scatter with units of 8 KiB and more: 0.95-0.99x at 64 MiB, 0.95-1.02x at
-// 128, 0.97-1.03x at 192, 0.97-1.05x at 256, 0.94-1.05x at 384, 0.96-1.04x at 768
-// (8 x 96 alone behind, 8 x 128 1.01-1.04x). Smaller units never: those of 4 KiB
+// Fused scatter with units of 8 KiB and more, and 2 x 128 bf16, 8 x 192 and MLA rows
+// beside those: 0.95-0.99x at 64 MiB, 0.95-1.02x at 128, 0.96-1.03x at 160 (mean
+// 0.99), 0.97-1.03x at 192 (1.00), 0.99-1.06x at 224 (1.01), 0.98-1.04x at 256
+// (1.01), 0.99-1.06x at 320 (1.01), 0.98-1.05x at 352 (1.01). Smaller units never: those of 4 KiB
 // ran 0.75-0.91x from 64 to 256 MiB (96 MiB in four chunks of 80 layers 49 -> 64 us,
 // 56 in the plain order of earlier grids) and 0.90-0.99x at 768, of 2 KiB
 // 0.69-0.95x, since each reads its job over the host link.
 inline int64_t fused_runs_from(int64_t unit_bytes) {
-    return unit_bytes < 8192 ? INT64_MAX : 320ll << 20;
+    return unit_bytes < 8192 ? INT64_MAX : 208ll << 20;
 }
 
 // JobRows launches.

@@ -802,11 +802,13 @@ size_t select_merge_lds(int64_t max_tokens, int64_t kmax, bool one_pass) {
 constexpr size_t kSelectMergeMaxLds = 40 * 1024;   // beside the 8 KiB of the top-k
 // A fused workgroup merges its chunk's selected rows alone, in rounds of
 // kMergeThreads x kMergeUnits 16-byte units. Up to this many rounds per chunk
-// the fused top-k + merge beat topk_kernel + merge_rows_kernel on MI355X
-// (config 3: 77 rows of 4 KiB, 10 rounds, 0.635 ms against 0.039 + 0.611 ms,
-// both layer-minor); beyond it the merge kernel's spread over (chunk, row
-// batch) wins (config 5: 205 quantised rows, 26 rounds, 0.39 ms against
-// 0.36 ms).
+// the fused top-k + merge is as fast as topk_kernel + merge_rows_kernel or faster;
+// beyond it the merge kernel's spread over (chunk, row batch) wins. MI355X, whole
+// selections, fused against three launches: 96 chunks of 512 tokens in 32 layers of
+// 8 x 128 bf16 1318 and 1320 us at 10 rounds, 1412 and 1414 at 12, 1961 and 1942 at
+// 26; 6 of 1500 220.3 and 219.0 at 10, 240 and 234 at 16; 64 of 1000 in 80 layers of
+// 1 x 128 495 and 509 at 1, 1173 and 1192 at 11; 16 of 512 in 80 e4m3 layers 382 and
+// 388 at 3, 517 and 504 at 12, 571 and 549 at 16.
 constexpr int64_t kFusedMaxRounds = 12;
 
 bool select_merge_fits(const KVGeom& g, int elem_size, bool quant, int64_t max_tokens, int64_t kmax,

@@ -620,7 +620,7 @@ def test_page_copies_cut_each_job_by_its_own_span(hosttest):
 
 
 @pytest.mark.parametrize("unit,mib,runs", [
-    (16384, 1024, True), (8192, 384, True), (8192, 256, False), (16384, 64, False), (4096, 1024, False), (2048, 512, False),
+    (16384, 1024, True), (8192, 224, True), (8192, 192, False), (16384, 64, False), (4096, 1024, False), (2048, 512, False),
 ])
 def test_fused_scatters_in_runs(hosttest, unit, mib, runs):
     """Fused scatters take the jobs' runs per XCD where calls are large and
