@@ -506,9 +506,7 @@ int copy_pages(daric_copier* c, const char* const* names, int64_t n_jobs, const 
         DeviceGuard guard(r.device);
         const hipStream_t st = as_stream(stream);
         const size_t bytes = r.jobs.size() * sizeof(CopyJob);
-        int64_t span = 0;
-        for (const CopyJob& j : r.jobs) span = std::max<int64_t>(span, j.span);
-        DescHandOver ho(r.device, r.jobs.data(), bytes, st, bytes <= direct_desc_bytes(gather, std::min(span, part)));
+        DescHandOver ho(r.device, r.jobs.data(), bytes, st, bytes <= direct_desc_bytes(gather, part));
         launch_copy_pages(ho.arg(), classes, part, r.vw, gather, st);
     });
 }

@@ -43,23 +43,24 @@ __device__ __forceinline__ T ld_nt(const T* p) { return __builtin_nontemporal_lo
 template <typename T>
 __device__ __forceinline__ void st_nt(T* p, T v) { __builtin_nontemporal_store(v, p); }
 
-// Copies n_units units of VW bytes from src to dst (n_units < 2^31).
-template <int VW>
+// Copies n_units units of VW bytes from src to dst (n_units < 2^31) by the LANES
+// lanes of a workgroup.
+template <int VW, int LANES = kThreads>
 __device__ __forceinline__ void copy_units(const uint8_t* __restrict__ src,
                                            uint8_t* __restrict__ dst, int n_units) {
     using T = typename VecOf<VW>::T;
     const T* s = reinterpret_cast<const T*>(src);
     T* d = reinterpret_cast<T*>(dst);
-    for (int base = 0; base < n_units; base += kThreads * kUnroll) {
+    for (int base = 0; base < n_units; base += LANES * kUnroll) {
         T v[kUnroll];
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            const int i = base + u * kThreads + static_cast<int>(threadIdx.x);
+            const int i = base + u * LANES + static_cast<int>(threadIdx.x);
             if (i < n_units) v[u] = ld_nt(s + i);
         }
 #pragma unroll
         for (int u = 0; u < kUnroll; ++u) {
-            const int i = base + u * kThreads + static_cast<int>(threadIdx.x);
+            const int i = base + u * LANES + static_cast<int>(threadIdx.x);
             if (i < n_units) st_nt(d + i, v[u]);
         }
     }
@@ -83,9 +84,9 @@ __device__ __forceinline__ bool resolve_tile(const CopyJob& j, int t, int& p, in
 }
 
 // A unit is a part of a tile: part_units accesses of VW bytes, the last part of a
-// tile what is left.
-template <int VW, bool GATHER, class Grid>
-__global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job0, Grid grid) {
+// tile what is left. LANES: copy_lanes of the longest unit.
+template <int VW, bool GATHER, class Grid, int LANES>
+__global__ __launch_bounds__(LANES) void copy_pages_kernel(DescArg d, int job0, Grid grid) {
     DARIC_ARGS_TOGETHER4(d.ptr, job0, grid.begin[1], grid.cls[0].div.d);
     int jb, unit;
     grid.at_block(blockIdx.x, jb, unit);
@@ -99,9 +100,9 @@ __global__ __launch_bounds__(kThreads) void copy_pages_kernel(DescArg d, int job
     if (cnt <= 0) return;
     const int64_t b0 = static_cast<int64_t>(u0) * VW;
     if (GATHER)
-        copy_units<VW>(cache + b0, stage + b0, cnt);
+        copy_units<VW, LANES>(cache + b0, stage + b0, cnt);
     else
-        copy_units<VW>(stage + b0, cache + b0, cnt);
+        copy_units<VW, LANES>(stage + b0, cache + b0, cnt);
 }
 
 // Fused scatter + rotation for any row width (rotate_rows.h). A workgroup takes
@@ -383,21 +384,29 @@ __global__ __launch_bounds__(kThreads) void upload_kernel(const u32x4* __restric
 void launch_copy_pages(const DescArg& d, const JobClasses& classes, int64_t part, int vw,
                        bool gather, hipStream_t stream) {
     if (classes.empty()) return;
+    const int lanes = copy_lanes(part, vw);
+#define DARIC_CP(VW, G, GRID, T) DARIC_LAUNCH((copy_pages_kernel<VW, G, GRID, T>), blocks, T, 0, stream, d, j0, g)
+#define DARIC_CPV(G, GRID)                                                                               \
+    do {                                                                                                 \
+        if (vw == 16 && lanes == 64) DARIC_CP(16, G, GRID, 64);                                          \
+        else if (vw == 16 && lanes == 128) DARIC_CP(16, G, GRID, 128);                                   \
+        else if (vw == 16) DARIC_CP(16, G, GRID, 256);                                                   \
+        else if (vw == 4) DARIC_CP(4, G, GRID, 256);                                                     \
+        else DARIC_CP(1, G, GRID, 256);                                                                  \
+    } while (0)
     if (gather) {
         for_job_rows(classes, 1, part, [&](int j0, const JobRows& g, unsigned blocks) {
-#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, true, JobRows>), blocks, kThreads, 0, stream, d, j0, g)
-            if (vw == 16) DARIC_CP(16); else if (vw == 4) DARIC_CP(4); else DARIC_CP(1);
-#undef DARIC_CP
+            DARIC_CPV(true, JobRows);
             check_launch("gather_pages");
         });
         return;
     }
     for_job_runs(classes, 1, part, kScatterRunsFrom, [&](int j0, const JobRuns& g, unsigned blocks) {
-#define DARIC_CP(VW) DARIC_LAUNCH((copy_pages_kernel<VW, false, JobRuns>), blocks, kThreads, 0, stream, d, j0, g)
-        if (vw == 16) DARIC_CP(16); else if (vw == 4) DARIC_CP(4); else DARIC_CP(1);
-#undef DARIC_CP
+        DARIC_CPV(false, JobRuns);
         check_launch("scatter_pages");
     });
+#undef DARIC_CPV
+#undef DARIC_CP
 }
 
 void launch_upload(const void* src, void* dst, size_t n16, hipStream_t stream) {

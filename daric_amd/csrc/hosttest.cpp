@@ -132,7 +132,8 @@ int daric_hosttest_topk_slots(int n, int lanes) { return daric::topk_slots(n, la
 
 // Units (parts of tiles) that a page copy of one call has for jobs of tiles[i]
 // tiles of span[i] bytes: units[i], in the order of the arguments.
-void daric_hosttest_page_units(const int64_t* tiles, const int64_t* span, int64_t n, int vw, int64_t* units) {
+// Returns the longest unit's bytes.
+int64_t daric_hosttest_page_units(const int64_t* tiles, const int64_t* span, int64_t n, int vw, int64_t* units) {
     std::vector<daric::CopyJob> jobs(static_cast<size_t>(n));
     for (int64_t i = 0; i < n; ++i) {
         daric::CopyJob& j = jobs[static_cast<size_t>(i)];
@@ -144,7 +145,10 @@ void daric_hosttest_page_units(const int64_t* tiles, const int64_t* span, int64_
     int64_t part;
     daric::cut_pages(jobs, vw, &part);
     for (const daric::CopyJob& j : jobs) units[j.n_tokens] = static_cast<int64_t>(j.n_sel) * j.parts.d;
+    return part;
 }
+
+int daric_hosttest_copy_lanes(int64_t unit_bytes, int vw) { return daric::copy_lanes(unit_bytes, vw); }
 
 int64_t daric_hosttest_page_part_bytes(int64_t max_span, int64_t tiles) {
     return daric::page_part_bytes(max_span, tiles);

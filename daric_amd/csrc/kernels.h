@@ -317,7 +317,8 @@ inline void split_long_jobs(std::vector<CopyJob>& jobs, int64_t parts, int64_t P
 }
 
 // Cuts the jobs' tiles into parts for accesses of vw bytes and orders the jobs by
-// their parts. *part gets the longest part's bytes.
+// their parts. *part gets the longest part's bytes, of pages shorter than a part the
+// page's.
 inline JobClasses cut_pages(std::vector<CopyJob>& jobs, int vw, int64_t* part) {
     *part = 0;
     const CopyJob* like = nullptr;     // job whose tiles the last one had: no divisions again
@@ -330,13 +331,25 @@ inline JobClasses cut_pages(std::vector<CopyJob>& jobs, int vw, int64_t* part) {
             const int64_t bytes = page_part_bytes(j.span, tiles);
             j.part_units = static_cast<int32_t>((bytes + vw - 1) / vw);
             j.parts = FastDiv(static_cast<uint32_t>(std::max<int64_t>(1, (j.span + bytes - 1) / bytes)));
-            if (tiles > 0) *part = std::max(*part, bytes);
+            if (tiles > 0) *part = std::max(*part, std::min<int64_t>(bytes, j.span));
             like = &j;
         }
     }
     return order_jobs(jobs, [](const CopyJob& j) {
         return static_cast<int64_t>(j.prefix) * j.n_sel * j.parts.d;
     });
+}
+
+// Lanes of a copy's workgroups of up to unit_bytes: 256, or as many as have two
+// accesses of 16 bytes each where units are small. Such workgroups are bound by
+// their start, a chain of loads from the grid's class over the job and the page id
+// to the data, times those a CU holds, 8 of 256 lanes: 640 MiB in pages of 2 KiB (80
+// layers of 1 x 64 bf16) were gathered in 418 us by 256 lanes each, in 222 by 128 and
+// in 216 by 64, scattered in 405, 253 and 246, token by token in 529, 269 and 221; in
+// pages of 4 KiB (1 x 128) in 222, 216 and 229, scattered in 252, 244 and 248, token
+// by token in 273, 221 and 227 (MI355X).
+inline int copy_lanes(int64_t unit_bytes, int vw) {
+    return vw != 16 || unit_bytes > 4096 ? 256 : unit_bytes > 2048 ? 128 : 64;
 }
 
 // Most bytes of job descriptors that a copy's kernels read from the pinned slot

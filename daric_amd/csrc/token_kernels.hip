@@ -84,8 +84,9 @@ __device__ __forceinline__ bool resolve_part(const TokenJob& j, int q, uint8_t*&
     return true;
 }
 
-template <int VW, bool GATHER, class Grid>
-__global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job0, Grid grid) {
+// LANES: copy_lanes of the longest part.
+template <int VW, bool GATHER, class Grid, int LANES>
+__global__ __launch_bounds__(LANES) void token_rows_kernel(DescArg d, int job0, Grid grid) {
     using T = typename Unit<VW>::T;
     DARIC_ARGS_TOGETHER4(d.ptr, job0, grid.begin[1], grid.cls[0].div.d);
     int jb, q;
@@ -97,12 +98,12 @@ __global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job
     const int upr = static_cast<int>(j.d_upr.d);
     const int units = n_tok * j.H * upr;
     T* __restrict__ st = reinterpret_cast<T*>(stage);
-    for (int base = 0; base < units; base += kThreads * kRowUnroll) {
+    for (int base = 0; base < units; base += LANES * kRowUnroll) {
         T v[kRowUnroll];
         T* cp[kRowUnroll];
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
-            const int i = base + u * kThreads + static_cast<int>(threadIdx.x);
+            const int i = base + u * LANES + static_cast<int>(threadIdx.x);
             cp[u] = nullptr;
             if (i >= units) continue;
             const uint32_t row = j.d_upr.div(static_cast<uint32_t>(i));   // token-major: tok * H + h
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(kThreads) void token_rows_kernel(DescArg d, int job
         }
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
-            const int i = base + u * kThreads + static_cast<int>(threadIdx.x);
+            const int i = base + u * LANES + static_cast<int>(threadIdx.x);
             if (cp[u] == nullptr) continue;
             if (GATHER) st_nt(st + i, v[u]);
             else st_nt(cp[u], v[u]);
@@ -203,11 +204,15 @@ __global__ __launch_bounds__(kThreads) void token_lds_kernel(DescArg d, int job0
 
 void launch_token_copy(const DescArg& d, const JobClasses& classes, int64_t part_bytes, int vw,
                        bool lds, bool gather, hipStream_t stream) {
+    const int lanes = copy_lanes(part_bytes, vw);
+#define DARIC_TR(VW, G, GRID, T) DARIC_LAUNCH((token_rows_kernel<VW, G, GRID, T>), blocks, T, 0, stream, d, j0, g)
 #define DARIC_TOK(G, GRID)                                                                              \
     do {                                                                                               \
         if (lds) DARIC_LAUNCH((token_lds_kernel<G, GRID>), blocks, kThreads, 0, stream, d, j0, g);       \
-        else if (vw == 16) DARIC_LAUNCH((token_rows_kernel<16, G, GRID>), blocks, kThreads, 0, stream, d, j0, g); \
-        else DARIC_LAUNCH((token_rows_kernel<1, G, GRID>), blocks, kThreads, 0, stream, d, j0, g);       \
+        else if (vw == 16 && lanes == 64) DARIC_TR(16, G, GRID, 64);                                     \
+        else if (vw == 16 && lanes == 128) DARIC_TR(16, G, GRID, 128);                                   \
+        else if (vw == 16) DARIC_TR(16, G, GRID, 256);                                                   \
+        else DARIC_TR(1, G, GRID, 256);                                                                  \
         check_launch(G ? "gather_tokens" : "scatter_tokens");                                         \
     } while (0)
     if (gather)
@@ -216,6 +221,7 @@ void launch_token_copy(const DescArg& d, const JobClasses& classes, int64_t part
         for_job_runs(classes, 1, part_bytes, kRunsFrom,
                      [&](int j0, const JobRuns& g, unsigned blocks) { DARIC_TOK(false, JobRuns); });
 #undef DARIC_TOK
+#undef DARIC_TR
 }
 
 }  // namespace daric

@@ -619,6 +619,24 @@ def test_page_copies_cut_each_job_by_its_own_span(hosttest):
     assert (units // t).tolist() == [16, 1, 1, 1, 2, 9, 1] * 3
 
 
+@pytest.mark.parametrize("spans,longest,lanes", [
+    ([16], 16, 64), ([2048, 512], 2048, 64), ([2064], 2064, 128), ([4096, 2048], 4096, 128), ([4112], 4112, 256),
+    ([2048, 9216], 9216, 256), ([131072], 8192, 256), ([12288, 16], 6144, 256),
+])
+def test_lanes_of_small_pages(hosttest, spans, longest, lanes):
+    """The longest unit is the page where that is shorter than a part, and
+    chooses the lanes: two accesses of 16 bytes each."""
+    hosttest.daric_hosttest_page_units.restype = ctypes.c_int64
+    t, s = np.full(len(spans), 7, np.int64), np.asarray(spans, np.int64)
+    units = np.zeros_like(t)
+    part = hosttest.daric_hosttest_page_units(
+        ctypes.c_void_p(t.ctypes.data), ctypes.c_void_p(s.ctypes.data), ctypes.c_int64(t.size), ctypes.c_int(16),
+        ctypes.c_void_p(units.ctypes.data))
+    assert part == longest
+    assert hosttest.daric_hosttest_copy_lanes(ctypes.c_int64(part), ctypes.c_int(16)) == lanes
+    assert hosttest.daric_hosttest_copy_lanes(ctypes.c_int64(part), ctypes.c_int(1)) == 256
+
+
 @pytest.mark.parametrize("unit,mib,runs", [
     (16384, 1024, True), (8192, 224, True), (8192, 192, False), (16384, 64, False), (4096, 1024, False), (2048, 512, False),
 ])

@@ -153,6 +153,41 @@ def test_as_many_pages_as_a_job_may_have(dev, n_sel):
         c.gather_pages(["l"], [0], [16 << 24], more, [0, 1 << 24])
 
 
+@pytest.mark.parametrize("spans", [(16,), (1008,), (2048,), (2064,), (4096, 2048), (4112,), (8192, 16, 2048), (2052,),
+                                   (2050, 30)])
+def test_small_pages(dev, spans):
+    """Pages at the edges of 64, 128 and 256 lanes, of one size and several in a
+    call, and ones for 4- and 1-byte accesses: gathered and scattered back."""
+    nb, n_sel = 50, 33
+    g = torch.Generator().manual_seed(sum(spans))
+    layers = [torch.randint(0, 256, (nb, 1, s), dtype=torch.uint8, generator=g).to(dev) for s in spans]
+    ids = [torch.randperm(nb - 1, generator=g)[:n_sel] + 1 for _ in spans]
+    offs, at = [], 0
+    for s in spans:
+        offs.append(at)
+        at += s * n_sel
+    store = torch.full((at + 16,), 0x5A, dtype=torch.uint8, device=dev)
+    c = cache_ops.CacheCopier()
+    names = [f"l{i}" for i in range(len(spans))]
+    for name, t in zip(names, layers):
+        c.register_layer(name, t, True)
+    c.register_store(store)
+    jobs = (names, offs, [s * n_sel for s in spans], torch.cat(ids).to(torch.int32).to(dev),
+            [n_sel * i for i in range(len(spans) + 1)])
+    c.gather_pages(*jobs)
+    want = [t.clone() for t in layers]
+    for s, o, i, t in zip(spans, offs, ids, layers):
+        assert torch.equal(store[o:o + s * n_sel].view(n_sel, s), t[i.to(dev), 0])
+        t.zero_()
+    assert (store[at:] == 0x5A).all()
+    c.scatter_pages(*jobs)
+    for i, t, w in zip(ids, layers, want):
+        rest = torch.ones(nb, dtype=torch.bool)
+        rest[i] = False
+        w[rest.to(dev)] = 0
+        assert torch.equal(t, w)
+
+
 def test_errors_surface_as_runtime_error(dev):
     gc = cache_ops.CacheCopier()
     t = torch.zeros(2, 4, 16, 2, 8, dtype=torch.bfloat16, device=dev)

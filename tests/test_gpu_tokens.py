@@ -95,7 +95,9 @@ def test_token_copies_llama3_8b_hnd(dev, gather):
                                            ("pf", 65, 2, 80), ("nhd", 37, 4, 144), ("nhd", 3, 8, 1296),
                                            ("nhd", 16, 1, 896), ("nhd", 16, 2, 456), ("nhd", 14, 1, 2048),
                                            ("pf", 15, 1, 1888), ("nhd", 29, 1, 992), ("nhd", 37, 2, 1024),
-                                           ("pf", 130, 4, 128)])
+                                           ("pf", 130, 4, 128), ("nhd", 16, 1, 128), ("nhd", 16, 2, 64),
+                                           ("mla", 9, 1, 240), ("pf", 16, 1, 256), ("nhd", 3, 1, 16),
+                                           ("nhd", 17, 1, 256), ("nhd", 257, 1, 16)])
 def test_token_row_parts(dev, layout, ps, h, d, gather):
     _case(dev, [layout, layout], torch.uint8, d=d, h=h, ps=ps, gather=gather, seed=9)
 
