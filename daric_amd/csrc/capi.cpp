@@ -937,6 +937,7 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
             RowGeom g;
             std::vector<CopyJob> jobs;
             JobClasses classes;
+            bool even = true;     // every job has the first one's tiles
         };
         std::vector<Group> groups;
         for (int64_t i = 0; i < n_jobs; ++i) {
@@ -975,11 +976,12 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
             for (auto& gr : groups)
                 if (gr.kind == kind && std::memcmp(&gr.g, &L->geom, sizeof(RowGeom)) == 0) { grp = &gr; break; }
             if (grp == nullptr) {
-                groups.push_back(Group{kind, L->geom, {}, {}});
+                groups.push_back(Group{kind, L->geom, {}, {}, true});
                 grp = &groups.back();
                 grp->jobs.reserve(n_jobs);
             }
             grp->jobs.push_back(j);
+            grp->even = grp->even && tiles_of(j) == tiles_of(grp->jobs.front());
         }
         if (noalloc)
             DARIC_CHECK(fused && aligned, "scatter_pages_rerotate_noalloc needs a layout the fused kernel takes "
@@ -989,8 +991,11 @@ int scatter_rerotate(daric_copier* c, const char* const* names, int64_t n_jobs, 
             return;
         }
         for (Group& gr : groups) {
-            split_long_jobs(gr.jobs, FusedCut(gr.g, gr.kind == kE4M3 ? 16 : 8).parts, gr.g.PS);
-            gr.classes = order_jobs(gr.jobs, tiles_of);
+            const int64_t parts = FusedCut(gr.g, gr.kind == kE4M3 ? 16 : 8).parts;
+            const bool fit = r.max_tiles * parts <= kMaxGridBlocks;
+            if (!fit) split_long_jobs(gr.jobs, parts, gr.g.PS);
+            gr.classes = fit && gr.even ? JobClasses::even(static_cast<int64_t>(gr.jobs.size()), tiles_of(gr.jobs[0]))
+                                        : order_jobs(gr.jobs, tiles_of);
         }
         // Allocation-free variant: job sets that do not travel inline are
         // staged in the static scratch array, one region per launch group.

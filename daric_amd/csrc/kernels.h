@@ -118,6 +118,12 @@ struct JobClasses {
         for (int k = 0; k < n; ++k) s += c[k].jobs;
         return s;
     }
+    // One class of `jobs` jobs (none of jobs without tiles).
+    static JobClasses even(int64_t jobs, int64_t tiles) {
+        JobClasses r;
+        if (tiles > 0 && jobs > 0) r.c[r.n++] = {jobs, tiles};
+        return r;
+    }
 };
 
 // Joins neighbours of a descending list of lengths until at most kJobClasses
@@ -162,12 +168,7 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
         even = even && t == longest;
         longest = std::max(longest, t);
     }
-    if (longest == 0) return out;
-    if (even) {
-        out.n = 1;
-        out.c[0] = {static_cast<int64_t>(n), longest};
-        return out;
-    }
+    if (even) return JobClasses::even(static_cast<int64_t>(n), longest);
     std::vector<uint32_t> to(n);      // a job's length, then its place
     // lengths in at most 63 steps of the longest (exact up to 63 tiles, or where
     // no more than 64 lengths occur), rounded up
@@ -190,11 +191,7 @@ JobClasses order_jobs(std::vector<Job>& jobs, Count&& count) {
         ++d[last].jobs;
         to[i] = static_cast<uint32_t>(last);
     }
-    if (nd == 1) {
-        out.n = 1;
-        out.c[0] = {static_cast<int64_t>(n), longest};
-        return out;
-    }
+    if (nd == 1) return JobClasses::even(static_cast<int64_t>(n), longest);
     int rank[kLengths], joined[kLengths];
     JobClass s[kLengths];
     int ns = 0;
@@ -322,6 +319,7 @@ inline void split_long_jobs(std::vector<CopyJob>& jobs, int64_t parts, int64_t P
 inline JobClasses cut_pages(std::vector<CopyJob>& jobs, int vw, int64_t* part) {
     *part = 0;
     const CopyJob* like = nullptr;     // job whose tiles the last one had: no divisions again
+    bool even = true;                  // no second pass over the jobs of the usual call
     for (CopyJob& j : jobs) {
         const int64_t tiles = static_cast<int64_t>(j.prefix) * j.n_sel;
         if (like != nullptr && like->span == j.span && like->n_sel == j.n_sel && like->prefix == j.prefix) {
@@ -332,9 +330,12 @@ inline JobClasses cut_pages(std::vector<CopyJob>& jobs, int vw, int64_t* part) {
             j.part_units = static_cast<int32_t>((bytes + vw - 1) / vw);
             j.parts = FastDiv(static_cast<uint32_t>(std::max<int64_t>(1, (j.span + bytes - 1) / bytes)));
             if (tiles > 0) *part = std::max(*part, std::min<int64_t>(bytes, j.span));
+            even = like == nullptr;
             like = &j;
         }
     }
+    if (even && like != nullptr)
+        return JobClasses::even(static_cast<int64_t>(jobs.size()), static_cast<int64_t>(like->prefix) * like->n_sel * like->parts.d);
     return order_jobs(jobs, [](const CopyJob& j) {
         return static_cast<int64_t>(j.prefix) * j.n_sel * j.parts.d;
     });
