@@ -362,7 +362,7 @@ inline int copy_lanes(int64_t unit_bytes, int vw) {
 // way to the host). MI355X, uploaded against read in place, idle and beside
 // host-to-device copies: gathers of 40 jobs (3.1 KiB) 44.2 and 45.6 -> 41.5 and 45.7
 // us, 40 (4.4) 45.4 and 47.3 -> 44.0 and 50.0, 96 (10.5) 73.0 and 75.1 -> 75.1 and
-// 85.2, 160 of 4 KiB pages (12.5) 57.1 and 59.8 -> 65.8 and 81.6; scatters of 48
+// 85.2, 160 of 4 KiB pages (12.5; 256 lanes) 57.1 and 59.8 -> 65.8 and 81.6; scatters of 48
 // (5.3) 28.4 and 29.7 -> 23.2 and 24.8, 128 (14) 104.9 and 108.9 -> 100.2 and 103.9,
 // 160 of 4 KiB pages 64.2 and 66.4 -> 65.6 and 74.2.
 inline size_t direct_desc_bytes(bool gather, int64_t unit_bytes) {
